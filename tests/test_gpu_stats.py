@@ -123,3 +123,33 @@ def test_invalid_arguments(handle, mfx):
     small = torch.empty((8, 4), device=DEV)
     with pytest.raises(mfx.MfxError):
         handle.covariance(data, mean, cen, small[:, :3], 10.0)
+
+
+@pytest.mark.parametrize("n,m,pad", [(1, 1, 0), (63, 64, 0), (65, 63, 0), (257, 68, 4), (300, 130, 3), (8300, 36, 0),
+                                     (20001, 500, 0), (64, 1025, 0)])
+def test_statistics_at_strip_and_slab_edges(handle, n, m, pad):
+    """Mean, deviation and centred data at the edges of the 64-column strips
+    and row slabs, vector and scalar loads.  Bounds: a compensated float sum
+    is within 2 ulp of max|x| per element of the mean; squares and the root
+    add a few ulp (2^-23) relative to the deviation; a centred value carries
+    the mean's error plus one rounding of |x - mean| <= 2.5."""
+    base = torch.empty((n, m + pad), device=DEV)
+    handle.fill_uniform(base, 31, n % 7)
+    data = base[:, :m]
+    data += 0.25
+    print(f"statistics n={n} m={m} pad={pad}", flush=True)
+    mean, sd = torch.empty(m, device=DEV), torch.empty(m, device=DEV)
+    cen, sym = torch.empty((n, m), device=DEV), torch.empty((m, m), device=DEV)
+    x = data.double()
+    mu = x.mean(0)
+    handle.covariance(data, mean, cen, sym, float(n), prec="fp32")
+    assert (mean.double() - mu).abs().max().item() <= 4 * 2**-24 * 1.25
+    assert (cen.double() - (x - mu)).abs().max().item() <= 2.5 * 2**-24 + 4 * 2**-24 * 1.25
+    handle.correlation(data, mean, sd, cen, sym, float(n), 0.005, prec="fp32")
+    dev = ((x - mu) ** 2).mean(0).sqrt()
+    dev = torch.where(dev <= 0.005, torch.ones_like(dev), dev)
+    assert ((sd.double() - dev).abs() / dev).max().item() <= 8 * 2**-23
+    want = (x - mu) / np.sqrt(float(n)) / dev
+    scale = (2.5 / np.sqrt(float(n)) / dev.min()).item()
+    assert (cen.double() - want).abs().max().item() <= 12 * 2**-23 * scale
+    assert torch.all(torch.diagonal(sym) == 1.0).item()
