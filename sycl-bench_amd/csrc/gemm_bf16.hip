@@ -1,13 +1,14 @@
 // Split-BF16 and single-BF16 dense contractions on v_mfma_f32_32x32x16_bf16
 // (building blocks in tile_bf16.h).
 //
-// Two kernels per call:
+// Two or three kernels per call:
 //  1. pack: converts each operand once into fragment order (hi and lo), with
 //     zero padding, so the contraction loop has no bounds checks and every
-//     load is a contiguous 16-byte chunk;
-//  2. contract: BM x BN tiles, BK = 32 (two MFMA k-steps) per stage,
-//     double-buffered LDS in the same fragment order (ds_read_b128 of
-//     consecutive 16-byte chunks: conflict-free), fused alpha/beta epilogue.
+//     load is a contiguous 16-byte chunk; both operands in one launch;
+//  2. contract: BM x BN tiles, LDS stages in the same fragment order
+//     (ds_read_b128 of consecutive 16-byte chunks: conflict-free), fused
+//     alpha/beta epilogue; tiles that do not fill a round of the CUs in k
+//     slices (SplitPlan), summed by a third kernel.
 // The same packed layout serves an operand in either role (A rows, or B
 // columns), which is what lets syrk use one packed copy of A for both.
 #include "tile_bf16.h"
@@ -15,11 +16,15 @@
 namespace mfx {
 namespace {
 
-struct PackParams {
+struct PackOperand {
   PackSrc s;
   int blocks;  // padded rows / 32
   int kbs;     // padded K / 16
   u32x4* dst;
+};
+struct PackParams {
+  PackOperand a, b;
+  int grid_a;  // workgroups of a; the rest are b's
 };
 
 // One lane-chunk per thread; a non-k-major source goes through the wave's
@@ -27,9 +32,11 @@ struct PackParams {
 // the (blk, kb) pairs walked kb-major so that neighbouring waves read
 // neighbouring segments of the same source rows.
 template <int NHL>
-__global__ __launch_bounds__(256) void pack_bf16x_kernel(const PackParams p) {
+__global__ __launch_bounds__(256) void pack_bf16x_kernel(const PackParams pp) {
   __shared__ float tiles[4][STAGED_TILE_FLOATS];
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const bool first = (int)blockIdx.x < pp.grid_a;
+  const PackOperand& p = first ? pp.a : pp.b;
+  const int64_t gid = (int64_t)(first ? blockIdx.x : blockIdx.x - pp.grid_a) * 256 + threadIdx.x;
   const int64_t total = (int64_t)p.blocks * p.kbs * 64;
   const bool active = gid < total;
   const int lane = (int)(gid & 63);
@@ -47,23 +54,33 @@ __global__ __launch_bounds__(256) void pack_bf16x_kernel(const PackParams p) {
 struct BfParams {
   BfTileArgs t;
   int tiles_m, tiles_n, group;
-  int mode;  // TILES_FULL / LOWER / UPPER
-  int tail_first = -1, tail_ratio = 1, big_tiles = 0;  // triangle_tile's re-tiled last round
+  int mode;        // TILES_FULL / LOWER / UPPER
+  SplitPlan plan;  // workgroups [0, head) take whole tiles, the rest slices
+  int tiles;       // tiles of the schedule
+  float* partial;
 };
 
 template <int BM, int BN, int WM, int WN, int NHL>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16x_kernel(const BfParams p) {
-  __shared__ u32x4 lds[BfCfg<BM, BN, WM, WN, NHL>::SMEM_CHUNKS];
+  using Cfg = BfCfg<BM, BN, WM, WN, NHL>;
+  __shared__ u32x4 lds[Cfg::SMEM_CHUNKS];
   int tm, tn;
-  const int pid = xcd_remap(blockIdx.x, gridDim.x);
-  if(p.mode == TILES_FULL) {
-    grouped_tile(pid, p.tiles_m, p.tiles_n, p.group, tm, tn);
-  } else {
-    int ti, tj;
-    if(!triangle_tile(pid, p.tiles_m, p.group, p.tail_first, p.tail_ratio, p.big_tiles, ti, tj)) return;
-    if(p.mode == TILES_LOWER) { tm = ti; tn = tj; } else { tm = tj; tn = ti; }
+  const int steps = p.t.kbs / Cfg::KB * p.t.nprod;
+  if((int)blockIdx.x < p.plan.head) {
+    tile_of(p.mode, xcd_remap(blockIdx.x, p.plan.head), p.tiles_m, p.tiles_n, p.group, tm, tn);
+    bf16_tile<BM, BN, WM, WN, NHL>(p.t, tm, tn, 0, steps, p.t.ep, tm * BM, tn * BN, lds);
+    return;
   }
-  bf16_tile<BM, BN, WM, WN, NHL>(p.t, tm, tn, lds);
+  // slice-major: an XCD's consecutive workgroups read the same k range of
+  // neighbouring tiles, which share operand panels in its L2
+  const int rest = p.tiles - p.plan.head, splits = p.plan.splits;
+  const int id = xcd_remap(blockIdx.x - p.plan.head, rest * splits);
+  const int slice = id / rest, tile = id - slice * rest;
+  tile_of(p.mode, p.plan.head + tile, p.tiles_m, p.tiles_n, p.group, tm, tn);
+  const int s0 = (int)((int64_t)steps * slice / splits), s1 = (int)((int64_t)steps * (slice + 1) / splits);
+  float* slot = p.partial + ((int64_t)tile * splits + slice) * (BM * BN);
+  const Epilogue ep{slot, BN, 1.0f, 0.0f, BM, BN, TILES_FULL, 0};
+  bf16_tile<BM, BN, WM, WN, NHL>(p.t, tm, tn, s0, s1, ep, 0, 0, lds);
 }
 
 struct BfConfig {
@@ -106,33 +123,66 @@ mfx_status launch_bf_config(Handle* h, const BfParams& p, bool split, int config
 
 struct PackPlan {
   int64_t rows_pad_a, rows_pad_b, kbs;
-  size_t bytes_a, bytes_b;
+  size_t bytes_a, bytes_b;  // rounded to 256
+  int64_t tiles;
+  SplitPlan split;
+  size_t bytes_partial;
 };
 
-PackPlan plan(const DenseOp& op, bool split, int config) {
+PackPlan plan(const DenseOp& op, bool split, int config, int cus, int forced_splits) {
   const BfConfig& c = kBfConfigs[config];
   PackPlan pl;
   const int nhl = split ? 2 : 1;
   // rows padded to 32 only (bf16_tile reads the last block again past them)
   pl.rows_pad_a = round_up(op.M, 32);
   pl.rows_pad_b = round_up(op.N, 32);
-  (void)c;
-  pl.kbs = round_up(op.K, 16 * kb_per_stage_of(nhl)) / 16;
-  pl.bytes_a = (size_t)pl.rows_pad_a * pl.kbs * 16 * nhl * 2;
-  pl.bytes_b = (size_t)pl.rows_pad_b * pl.kbs * 16 * nhl * 2;
+  const int stage = kb_per_stage_of(nhl);
+  pl.kbs = round_up(op.K, 16 * stage) / 16;
+  pl.bytes_a = (size_t)round_up(pl.rows_pad_a * pl.kbs * 16 * nhl * 2, 256);
+  pl.bytes_b = (size_t)round_up(pl.rows_pad_b * pl.kbs * 16 * nhl * 2, 256);
+  const int64_t tm = ceil_div(op.M, c.bm), tn = ceil_div(op.N, c.bn);
+  pl.tiles = op.tiles == TILES_FULL ? tm * tn : tm * (tm + 1) / 2;
+  pl.split = SplitPlan{(int)pl.tiles, 1};
+  pl.bytes_partial = 0;
+  const int64_t steps = pl.kbs / stage * op.nprod;
+  // Partial tiles stay within kMaxPartialBytes and, where the packed operands
+  // fit the no-allocation entry point's array, within that array too, so both
+  // entry points split alike.
+  const int64_t packed = (int64_t)(pl.bytes_a + pl.bytes_b), array = (int64_t)MFX_NOALLOC_SCRATCH_BYTES;
+  const int64_t max_partial = packed <= array ? std::min(kMaxPartialBytes, array - packed) : kMaxPartialBytes;
+  if(forced_splits >= 2) {
+    int64_t s = std::min<int64_t>(forced_splits, steps);
+    while(s > 1 && pl.tiles * s * c.bm * c.bn * 4 > max_partial) --s;
+    if(s > 1) pl.split = SplitPlan{0, (int)s};
+  } else if(forced_splits < 0) {
+    plan_splits(split ? MFX_PREC_SPLIT_BF16 : MFX_PREC_BF16, config, pl.tiles, steps * stage * 16, cus, max_partial,
+        &pl.split);
+  }
+  if(pl.split.splits > 1)
+    pl.bytes_partial = (size_t)(pl.tiles - pl.split.head) * pl.split.splits * c.bm * c.bn * sizeof(float);
   return pl;
 }
 
-mfx_status pack(Handle* h, const float* src, int64_t ld, int rows, int K, bool kmajor, int64_t rows_pad, int64_t kbs,
-    int nhl, u32x4* dst, hipStream_t s) {
+PackOperand pack_operand(const float* src, int64_t ld, int rows, int K, bool kmajor, int64_t rows_pad, int64_t kbs,
+    u32x4* dst) {
+  PackOperand o;
+  o.s = make_pack_src(src, ld, rows, K, kmajor);
+  o.blocks = (int)(rows_pad / 32);
+  o.kbs = (int)kbs;
+  o.dst = dst;
+  return o;
+}
+
+// Packs one operand, or both in one launch (b == nullptr: a alone).
+mfx_status pack(Handle* h, const PackOperand& a, const PackOperand* b, int nhl, hipStream_t s) {
   PackParams pp;
-  pp.s = make_pack_src(src, ld, rows, K, kmajor);
-  pp.blocks = (int)(rows_pad / 32);
-  pp.kbs = (int)kbs;
-  pp.dst = dst;
-  const int64_t total = rows_pad / 32 * kbs * 64;
-  if(total == 0) return MFX_SUCCESS;
-  const int grid = (int)ceil_div(total, 256);
+  pp.a = a;
+  pp.b = b ? *b : a;
+  const int64_t grid_a = ceil_div((int64_t)a.blocks * a.kbs * 64, 256);
+  const int64_t grid_b = b ? ceil_div((int64_t)b->blocks * b->kbs * 64, 256) : 0;
+  if(grid_a + grid_b == 0) return MFX_SUCCESS;
+  pp.grid_a = (int)grid_a;
+  const unsigned grid = (unsigned)(grid_a + grid_b);
   if(nhl == 2)
     return timed_launch(h, "pack_split_bf16", s, [&] { pack_bf16x_kernel<2><<<grid, 256, 0, s>>>(pp); });
   return timed_launch(h, "pack_bf16", s, [&] { pack_bf16x_kernel<1><<<grid, 256, 0, s>>>(pp); });
@@ -162,42 +212,42 @@ bool bf_config_info(int c, bool split, int* bm, int* bn, int* bk, int* waves) {
   return true;
 }
 
-size_t dense_bf16x_workspace(const DenseOp& op, bool split, int config) {
+size_t dense_bf16x_workspace(const DenseOp& op, bool split, int config, int cus, int forced_splits) {
   if(config < 0 || config >= kBfConfigCount) return 0;
-  PackPlan pl = plan(op, split, config);
+  const PackPlan pl = plan(op, split, config, cus, forced_splits);
   // syrk (single operand used in both roles) still reserves two slots; the
   // second is simply unused.
-  return round_up(pl.bytes_a, 256) + round_up(pl.bytes_b, 256);
+  return pl.bytes_a + pl.bytes_b + pl.bytes_partial;
 }
 
 mfx_status launch_dense_bf16x(Handle* h, const DenseOp& op, bool split, int config, hipStream_t s) {
   if(config < 0 || config >= kBfConfigCount) return invalid("BF16 tile configuration out of range");
   if(op.M == 0 || op.N == 0) return MFX_SUCCESS;
   void* ws = nullptr;
-  MFX_CHECK(workspace(h, dense_bf16x_workspace(op, split, config), &ws));
+  MFX_CHECK(workspace(h, dense_bf16x_workspace(op, split, config, cus_of(h), h->forced_splits), &ws));
   return launch_dense_bf16x_ws(h, op, split, config, ws, s);
 }
 
 // The pack kernels write every chunk of both padded panels (zeros past the
-// matrix), so `ws` needs no clearing and may hold anything on entry.
+// matrix) and the slices every partial tile, so `ws` needs no clearing and
+// may hold anything on entry.
 mfx_status launch_dense_bf16x_ws(Handle* h, const DenseOp& op, bool split, int config, void* ws, hipStream_t s) {
   if(config < 0 || config >= kBfConfigCount) return invalid("BF16 tile configuration out of range");
   const BfConfig& c = kBfConfigs[config];
   if(op.M == 0 || op.N == 0) return MFX_SUCCESS;
   const int nhl = split ? 2 : 1;
-  PackPlan pl = plan(op, split, config);
+  const PackPlan pl = plan(op, split, config, cus_of(h), h->forced_splits);
   const bool same = op.A == op.B && op.lda == op.ldb && op.a_kmajor == op.b_kmajor && op.M == op.N &&
                     pl.rows_pad_a == pl.rows_pad_b;
   if(op.nprod == 2 && pl.rows_pad_a != pl.rows_pad_b) return invalid("two-product form needs equal operand shapes");
-  u32x4* pa = static_cast<u32x4*>(ws);
-  u32x4* pb = reinterpret_cast<u32x4*>(static_cast<char*>(ws) + round_up(pl.bytes_a, 256));
+  if(op.tiles != TILES_FULL && (op.M != op.N || c.bm != c.bn)) return invalid("triangular schedule needs square tiles");
+  char* w = static_cast<char*>(ws);
+  u32x4* pa = reinterpret_cast<u32x4*>(w);
+  u32x4* pb = same ? pa : reinterpret_cast<u32x4*>(w + pl.bytes_a);
   // The B-role operand is indexed (n, k): B[n*ldb + k] if b_kmajor else B[k*ldb + n].
-  MFX_CHECK(pack(h, op.A, op.lda, op.M, op.K, op.a_kmajor, pl.rows_pad_a, pl.kbs, nhl, pa, s));
-  if(same) {
-    pb = pa;
-  } else {
-    MFX_CHECK(pack(h, op.B, op.ldb, op.N, op.K, op.b_kmajor, pl.rows_pad_b, pl.kbs, nhl, pb, s));
-  }
+  const PackOperand oa = pack_operand(op.A, op.lda, op.M, op.K, op.a_kmajor, pl.rows_pad_a, pl.kbs, pa);
+  const PackOperand ob = pack_operand(op.B, op.ldb, op.N, op.K, op.b_kmajor, pl.rows_pad_b, pl.kbs, pb);
+  MFX_CHECK(pack(h, oa, same ? nullptr : &ob, nhl, s));
   BfParams p;
   p.t.PA = pa;
   p.t.PB = pb;
@@ -210,29 +260,15 @@ mfx_status launch_dense_bf16x_ws(Handle* h, const DenseOp& op, bool split, int c
   p.tiles_n = (int)ceil_div(op.N, c.bn);
   p.group = 8;
   p.mode = op.tiles;
-  int grid;
-  if(op.tiles == TILES_FULL) {
-    grid = p.tiles_m * p.tiles_n;
-  } else {
-    if(p.tiles_m != p.tiles_n || c.bm != c.bn) return invalid("triangular schedule needs square tiles");
-    grid = p.tiles_m * (p.tiles_m + 1) / 2;
-  }
-  if(grid == 0) return MFX_SUCCESS;
-  if(op.tiles != TILES_FULL) {
-    const TriTail tail =
-        tri_tail(split ? MFX_PREC_SPLIT_BF16 : MFX_PREC_BF16, config, p.tiles_m, h->cu_count > 0 ? h->cu_count : 256);
-    if(tail.small >= 0) {
-      // the full rounds on this tile, the last round's big tiles re-tiled
-      MFX_CHECK(launch_bf_config(h, p, split, config, tail.head, s));
-      BfParams q = p;
-      q.tiles_m = q.tiles_n = (int)ceil_div(op.M, kBfConfigs[tail.small].bm);
-      q.tail_first = tail.head;
-      q.tail_ratio = tail.ratio;
-      q.big_tiles = p.tiles_m;
-      return launch_bf_config(h, q, split, tail.small, (grid - tail.head) * tail.ratio * tail.ratio, s);
-    }
-  }
-  return launch_bf_config(h, p, split, config, grid, s);
+  p.plan = pl.split;
+  p.tiles = (int)pl.tiles;
+  p.partial = reinterpret_cast<float*>(w + pl.bytes_a + pl.bytes_b);
+  const int grid = p.plan.head + (p.tiles - p.plan.head) * p.plan.splits;
+  MFX_CHECK(launch_bf_config(h, p, split, config, grid, s));
+  if(p.plan.splits == 1) return MFX_SUCCESS;
+  const SplitReduceArgs r{p.partial, c.bm, c.bn, p.plan.splits, p.plan.head, p.tiles, p.mode, p.tiles_m, p.tiles_n,
+      p.group, op.ep};
+  return launch_splitk_reduce(h, r, s);
 }
 
 // Element-wise split used by mfx_split_bf16 (a test and tooling utility).

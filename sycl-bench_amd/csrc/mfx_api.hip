@@ -209,18 +209,39 @@ int least_time_config(Handle* h, mfx_precision p, bool square_only, Tiles&& tile
   return best < 0 ? 0 : best;
 }
 
+// The configuration whose estimated launch, split-K included, is shortest
+// (plan_splits; split / single BF16).  `tiles(bm, bn)` as above.
+template <class Tiles>
+int least_cost_config(Handle* h, mfx_precision p, int64_t k, bool square_only, Tiles&& tiles) {
+  int best = 0;
+  double best_t = -1.0;
+  for(int c = 0; c < config_count(p); ++c) {
+    int bm, bn, bk, w;
+    if(!config_info(p, c, &bm, &bn, &bk, &w) || (square_only && bm != bn)) continue;
+    const double t = plan_splits(p, c, tiles(bm, bn), k, cus_of(h), kMaxPartialBytes, nullptr);
+    if(best_t < 0.0 || t < best_t) {
+      best = c;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
+bool has_cost_model(mfx_precision p) { return p == MFX_PREC_SPLIT_BF16 || p == MFX_PREC_BF16; }
+
 // FP32 configuration with sixteen waves on a 64x64 tile (four k-groups).
 constexpr int kF32KGroupConfig = 7;
 
 int heuristic_config(Handle* h, mfx_precision p, int64_t m, int64_t n, int64_t k) {
-  (void)k;
+  auto grid = [&](int bm, int bn) { return ceil_div(m, bm) * ceil_div(n, bn); };
+  if(has_cost_model(p)) return least_cost_config(h, p, k, false, grid);
   // FP32 grids of at most one 64x64 tile per CU: the k-grouped tile (one
   // sixteen-wave workgroup per CU hides load latency that four-wave tiles
   // leave exposed at this size; split-K then fills the CUs if tiles are
   // few).  Measured on MI355X: 1024^3 in 27-30 us against 32-36 us.
   const int cus = h->cu_count > 0 ? h->cu_count : 256;
   if(p == MFX_PREC_FP32 && ceil_div(m, 64) * ceil_div(n, 64) <= cus) return kF32KGroupConfig;
-  return least_time_config(h, p, false, [&](int bm, int bn) { return ceil_div(m, bm) * ceil_div(n, bn); });
+  return least_time_config(h, p, false, grid);
 }
 
 int choose_config(Handle* h, mfx_precision p, int64_t m, int64_t n, int64_t k) {
@@ -344,6 +365,8 @@ int choose_square_config(Handle* h, mfx_precision p, int64_t n, int64_t k) {
   }
   int bm, bn, bk, w;
   if(c >= 0) return config_info(p, c, &bm, &bn, &bk, &w) && bm == bn ? c : 0;
+  if(has_cost_model(p))
+    return least_cost_config(h, p, k, true, [&](int b, int) { return ceil_div(n, b) * (ceil_div(n, b) + 1) / 2; });
   return least_time_triangle(h, p, n);
 }
 
@@ -505,15 +528,11 @@ size_t mfx_gemm_workspace_size(mfx_precision prec, int64_t m, int64_t n, int64_t
   op.K = (int)k;
   op.nprod = 1;
   size_t best = 0;
-  // FP32 needs workspace only for split-K partial tiles, whose count depends
-  // on the CUs of the current device.
-  int cus = 0;
-  if(prec == MFX_PREC_FP32) {
-    int dev = 0;
-    if(hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-      cus = 256;
-  }
+  // split-K partial tiles depend on the CUs of the current device
+  int cus = 0, dev = 0;
+  if(hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
   // The largest need over all configurations, so any tuned choice fits.
   for(int c = 0; c < config_count(prec); ++c) {
     size_t b = 0;
@@ -524,7 +543,7 @@ size_t mfx_gemm_workspace_size(mfx_precision prec, int64_t m, int64_t n, int64_t
       const int splits = f32_splits(c, tiles, k, cus);
       if(splits > 1) b = f32_splitk_workspace(c, tiles, splits);
     } else if(prec == MFX_PREC_SPLIT_BF16 || prec == MFX_PREC_BF16)
-      b = dense_bf16x_workspace(op, prec == MFX_PREC_SPLIT_BF16, c);
+      b = dense_bf16x_workspace(op, prec == MFX_PREC_SPLIT_BF16, c, cus, -1);
     else if(prec == MFX_PREC_FP8_BLOCK || prec == MFX_PREC_FP8_BLOCK2)
       b = dense_fp8_workspace(op, prec == MFX_PREC_FP8_BLOCK2, c);
     best = std::max(best, b);

@@ -67,8 +67,10 @@ struct Handle {
   size_t staging_bytes = 0;
   hipEvent_t staging_ready = nullptr;
   int* error_flag = nullptr;
-  int forced_splits = -1;  // FP32 split-K: -1 automatic, 1 never, >= 2 that many slices
+  int forced_splits = -1;  // split-K: -1 automatic, 1 never, >= 2 that many slices
 };
+
+inline int cus_of(const Handle* h) { return h->cu_count > 0 ? h->cu_count : 256; }
 
 // Looks up the device's fixed no-allocation scratch array (mfx_create calls
 // it with the device current).
@@ -211,11 +213,11 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblocks) {
 }
 
 // Grouped ordering: GROUP consecutive tile rows are walked column by column.
-__device__ __forceinline__ void grouped_tile(int pid, int tiles_m, int tiles_n, int group, int& tm, int& tn) {
+__host__ __device__ __forceinline__ void grouped_tile(int pid, int tiles_m, int tiles_n, int group, int& tm, int& tn) {
   const int in_group = group * tiles_n;
   const int gid = pid / in_group;
   const int first_m = gid * group;
-  const int gsize = min(tiles_m - first_m, group);
+  const int gsize = tiles_m - first_m < group ? tiles_m - first_m : group;
   const int r = pid - gid * in_group;
   tm = first_m + r % gsize;
   tn = r / gsize;
@@ -275,6 +277,26 @@ __host__ __device__ inline bool triangle_tile(int p, int T, int group, int tail_
 
 // Scheduling modes shared by the FP32 and BF16 kernel families.
 enum TileMode : int { TILES_FULL = 0, TILES_LOWER = 1, TILES_UPPER = 2 };
+
+// Tile `id` of a full grid, or of a triangle (tiles_m == tiles_n).
+__host__ __device__ inline void tile_of(int mode, int id, int tiles_m, int tiles_n, int group, int& tm, int& tn) {
+  if(mode == TILES_FULL) {
+    grouped_tile(id, tiles_m, tiles_n, group, tm, tn);
+  } else {
+    int ti, tj;
+    grouped_lower_tile(id, tiles_m, group, ti, tj);
+    tm = mode == TILES_LOWER ? ti : tj;
+    tn = mode == TILES_LOWER ? tj : ti;
+  }
+}
+
+// Split-K of a tiled launch: tiles [0, head) run whole; each tile from `head`
+// on runs as `splits` slices of its k stages, which write partial tiles
+// (tile - head) * splits + slice of bm x bn floats, summed in slice order by
+// splitk_reduce (splitk.hip).  splits == 1: no tile is split (head = tiles).
+struct SplitPlan {
+  int head = 0, splits = 1;
+};
 
 // Epilogue parameters common to all families.
 struct Epilogue {
@@ -398,8 +420,22 @@ mfx_status launch_f32_splitk(Handle* h, const DenseOp& op, int config, int split
 mfx_status launch_dense_bf16x(Handle* h, const DenseOp& op, bool split, int config, hipStream_t s);
 // The same on a caller-provided workspace of dense_bf16x_workspace() bytes.
 mfx_status launch_dense_bf16x_ws(Handle* h, const DenseOp& op, bool split, int config, void* ws, hipStream_t s);
+
+// Sums the partial tiles of a split launch and applies op's epilogue.
+struct SplitReduceArgs {
+  const float* partial;
+  int bm, bn, splits;
+  int head, tiles;  // split tiles are [head, tiles)
+  int mode, tiles_m, tiles_n, group;
+  Epilogue ep;
+};
+mfx_status launch_splitk_reduce(Handle* h, const SplitReduceArgs& a, hipStream_t s);
+constexpr int64_t kMaxPartialBytes = (int64_t)32 << 20;
+// Estimated microseconds of a dense launch on `config` (tile_cost's model)
+// and the split plan behind it; partial tiles take at most max_partial bytes.
+double plan_splits(mfx_precision p, int config, int64_t tiles, int64_t k, int cus, int64_t max_partial, SplitPlan* plan);
 mfx_status launch_dense_fp8(Handle* h, const DenseOp& op, bool two_term, int config, hipStream_t s);
-size_t dense_bf16x_workspace(const DenseOp& op, bool split, int config);
+size_t dense_bf16x_workspace(const DenseOp& op, bool split, int config, int cus, int forced_splits);
 size_t dense_fp8_workspace(const DenseOp& op, bool two_term, int config);
 
 int config_count(mfx_precision p);

@@ -13,8 +13,9 @@
 //
 // Every call on one device shares that device's array: calls that overlap
 // on one device (two streams, or two host threads) race.  The pack kernels
-// overwrite every byte of both packed panels before the contraction reads
-// them, so nothing has to be cleared between calls.
+// overwrite every byte of both packed panels, and the slices of a split call
+// every partial tile, before they are read, so nothing has to be cleared
+// between calls.
 #include <mutex>
 
 #include "mfx_internal.h"
@@ -96,7 +97,7 @@ mfx_status mfx_gemm_noalloc(mfx_handle handle, mfx_precision prec, mfx_op transA
     else st = launch_dense_f32_ws(h, op, cfg, ws, MFX_NOALLOC_SCRATCH_BYTES, s);
   } else {
     const bool split = prec == MFX_PREC_SPLIT_BF16;
-    const size_t need = dense_bf16x_workspace(op, split, cfg);
+    const size_t need = dense_bf16x_workspace(op, split, cfg, cus_of(h), h->forced_splits);
     void* ws = scratch_of(h->device);
     if(need > MFX_NOALLOC_SCRATCH_BYTES) {
       st = unsupported("mfx_gemm_noalloc: the packed operands need " + std::to_string(need) +

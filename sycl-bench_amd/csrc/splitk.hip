@@ -1,0 +1,157 @@
+// Split-K plans and the reduction behind them, shared by the kernel families.
+//
+// A schedule whose tiles do not fill whole rounds of the CUs runs the tiles
+// of its last, partial round (all of them, when there are fewer tiles than
+// CUs) as k slices in separate workgroups.  Each slice writes its partial
+// tile to the workspace; splitk_reduce, in a launch of its own, sums the
+// partials of every output element in slice order (the same result on every
+// run) and applies alpha / beta.  The kernel boundary orders the two, so no
+// workgroup waits for another: a form that summed in the last-arriving
+// workgroup had every workgroup write back its XCD's whole L2 and took twice
+// the time of the unsplit kernel.
+#include <algorithm>
+
+#include "mfx_internal.h"
+
+namespace mfx {
+namespace {
+
+// One 32 x 32 sub-block of a split tile per workgroup, four consecutive
+// columns per thread: 16-byte loads of the partials (four slices in flight),
+// 16-byte accesses to C where its alignment allows.  A mirrored block is
+// transposed through LDS, so its stores are row segments too.  HBM-bound:
+// splits * bm * bn * 4 bytes per tile, which the slices have just written.
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitReduceArgs p) {
+  const int sub_n = p.bn / 32, subs = p.bm / 32 * sub_n;
+  const int t = blockIdx.x / subs, sub = blockIdx.x - t * subs;
+  int tm, tn;
+  tile_of(p.mode, p.head + t, p.tiles_m, p.tiles_n, p.group, tm, tn);
+  const int lr0 = sub / sub_n * 32, lc0 = sub % sub_n * 32;  // within the tile
+  const int r0 = tm * p.bm + lr0, c0 = tn * p.bn + lc0;
+  const Epilogue& ep = p.ep;
+  if(r0 >= ep.M || c0 >= ep.N) return;
+  if(ep.uplo == TILES_LOWER && r0 + 31 < c0) return;
+  if(ep.uplo == TILES_UPPER && c0 + 31 < r0) return;
+  const int lr = threadIdx.x >> 3, lc = (threadIdx.x & 7) * 4;
+  const int64_t area4 = (int64_t)p.bm * p.bn / 4;
+  const floatx4* src = reinterpret_cast<const floatx4*>(p.partial) + (int64_t)t * p.splits * area4 +
+                       ((lr0 + lr) * p.bn + lc0 + lc) / 4;
+  floatx4 v = src[0];
+  int s = 1;
+  for(; s + 4 <= p.splits; s += 4) {
+    floatx4 w[4];
+#pragma unroll
+    for(int u = 0; u < 4; ++u) w[u] = src[(s + u) * area4];
+#pragma unroll
+    for(int u = 0; u < 4; ++u) v += w[u];
+  }
+  for(; s < p.splits; ++s) v += src[s * area4];
+
+  const int row = r0 + lr, col = c0 + lc;
+  const bool vec = (reinterpret_cast<uintptr_t>(ep.C) & 15u) == 0 && ep.ldc % 4 == 0;
+  const bool inside = r0 + 32 <= ep.M && c0 + 32 <= ep.N;
+  if(ep.uplo == TILES_FULL && inside && vec) {
+    floatx4* c = reinterpret_cast<floatx4*>(ep.C + (int64_t)row * ep.ldc + col);
+    *c = ep.beta != 0.0f ? ep.alpha * v + ep.beta * *c : ep.alpha * v;
+    return;
+  }
+  auto wanted = [&](int r, int c) {
+    return r < ep.M && c < ep.N && (ep.uplo == TILES_FULL || (ep.uplo == TILES_LOWER ? r >= c : r <= c));
+  };
+#pragma unroll
+  for(int e = 0; e < 4; ++e)
+    if(wanted(row, col + e)) {
+      float* c = ep.C + (int64_t)row * ep.ldc + col + e;
+      *c = ep.beta != 0.0f ? ep.alpha * v[e] + ep.beta * *c : ep.alpha * v[e];
+    }
+  if(ep.uplo == TILES_FULL || !ep.mirror) return;
+  // element (row, col) of the triangle also gives (col, row), from its own C
+  __shared__ float tr[32][33];
+#pragma unroll
+  for(int e = 0; e < 4; ++e) tr[lr][lc + e] = v[e];
+  __syncthreads();
+#pragma unroll
+  for(int e = 0; e < 4; ++e) {
+    const int r = r0 + lc + e, cc = c0 + lr;  // source element; its mirror is (cc, r)
+    if(r != cc && wanted(r, cc)) {
+      float* c = ep.C + (int64_t)cc * ep.ldc + r;
+      const float x = ep.alpha * tr[lc + e][lr];
+      *c = ep.beta != 0.0f ? x + ep.beta * *c : x;
+    }
+  }
+}
+
+// Time of one tile, microseconds: `fixed` for its launch, first loads and
+// epilogue, and nanoseconds per k with few CUs busy (latency and LDS bound)
+// and with all of them busy (power, L2 and fabric shared by every CU).
+// Measured on MI355X with one tile per CU at K = 1024 and 4096.
+struct TileCost {
+  double fixed, idle, full;
+};
+constexpr TileCost kSplitCost[] = {
+    {6.0, 44.0, 64.0},  // 256x256, four waves
+    {5.8, 12.4, 18.0},  // 128x128, four waves
+    {4.0, 6.7, 6.8},    // 64x64
+    {7.0, 22.5, 33.0},  // 256x128, four waves
+    {6.0, 43.6, 65.0},  // 256x256, eight waves
+    {6.5, 22.6, 34.0},  // 256x128, eight waves
+    {4.9, 13.3, 19.0},  // 128x128, eight waves
+};
+constexpr TileCost kBf16Cost[] = {
+    {7.5, 16.0, 24.5}, {4.5, 6.2, 8.2}, {3.4, 3.87, 3.9}, {5.5, 9.7, 14.0},
+    {6.0, 15.4, 24.5}, {5.3, 9.5, 13.8}, {4.0, 6.1, 8.3},
+};
+
+// Reading the partials back and the launch that does it.
+constexpr double kReduceFixedUs = 4.0, kReduceBytesPerUs = 3.0e6;
+
+bool tile_cost(mfx_precision p, int c, TileCost* out) {
+  if(c < 0 || c >= 7) return false;
+  if(p == MFX_PREC_SPLIT_BF16) *out = kSplitCost[c];
+  else if(p == MFX_PREC_BF16) *out = kBf16Cost[c];
+  else return false;
+  return true;
+}
+
+}  // namespace
+
+mfx_status launch_splitk_reduce(Handle* h, const SplitReduceArgs& a, hipStream_t s) {
+  const int64_t grid = (int64_t)(a.tiles - a.head) * (a.bm / 32) * (a.bn / 32);
+  if(grid == 0) return MFX_SUCCESS;
+  return timed_launch(h, "splitk_reduce", s, [&] { splitk_reduce_kernel<<<(unsigned)grid, 256, 0, s>>>(a); });
+}
+
+// Whole rounds of tiles run unsplit.  The rest -- the tiles that do not fill a
+// round -- run whole or in up to 64 slices of at least two stages, whichever
+// this model makes shorter: a round costs fixed + k * (ns per k at the share of
+// CUs it keeps busy), a split adds the reduction.
+double plan_splits(mfx_precision p, int config, int64_t tiles, int64_t k, int cus, int64_t max_partial,
+    SplitPlan* plan) {
+  TileCost tc;
+  int bm, bn, bk, w;
+  if(plan) *plan = SplitPlan{(int)tiles, 1};
+  if(!tile_cost(p, config, &tc) || !config_info(p, config, &bm, &bn, &bk, &w) || tiles <= 0) return 0.0;
+  auto per_k = [&](double busy) {  // us per k
+    const double x = std::max(0.0, (std::min(1.0, busy) - 0.5) / 0.5);
+    return 1e-3 * (tc.idle + (tc.full - tc.idle) * x);
+  };
+  const int64_t rounds = tiles / cus, rest = tiles - rounds * cus, steps = ceil_div(k, bk);
+  const double head = (double)rounds * (tc.fixed + (double)k * per_k(1.0));
+  if(rest == 0) return head;
+  double best = head + tc.fixed + (double)k * per_k((double)rest / cus);
+  const double tile_bytes = 4.0 * bm * bn;
+  for(int64_t s = 2; s <= 64 && 2 * s <= steps; ++s) {
+    const double bytes = (double)(rest * s) * tile_bytes;
+    if(bytes > (double)max_partial) break;
+    const int64_t slice_rounds = ceil_div(rest * s, cus);
+    const double t = head + (double)slice_rounds * (tc.fixed + (double)(ceil_div(steps, s) * bk) * per_k((double)(rest * s) / cus)) +
+                     kReduceFixedUs + bytes / kReduceBytesPerUs;
+    if(t < best * 0.97) {  // a split has to be clearly ahead
+      best = t;
+      if(plan) *plan = SplitPlan{(int)(rounds * cus), (int)s};
+    }
+  }
+  return best;
+}
+
+}  // namespace mfx

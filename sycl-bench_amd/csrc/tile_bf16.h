@@ -212,16 +212,25 @@ __device__ __forceinline__ void pack_chunk(const PackSrc& s, int blk, int kb, in
   store_chunk<NHL>(dst, blk, kb, lane, kbs, v);
 }
 
+// Geometry of bf16_tile.  A stage is kb_per_stage k blocks (half that for the
+// four-wave 256x256 single-BF16 tile, which gains 2 % from four shorter
+// stages), and as many stages as fit the 160 KiB of LDS, at most four, are
+// buffered: the small tiles, whose stages hold little MFMA work, need that
+// many in flight to cover the global-to-LDS latency.
 template <int BM, int BN, int WM, int WN, int NHL>
 struct BfCfg {
   static constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN, NT = NW * 64;
   static constexpr int FM = WM / 32, FN = WN / 32;
-  static constexpr int KB = kb_per_stage<NHL>();
+  static constexpr int KB = NHL == 1 && WM == 128 && WN == 128 ? 2 : kb_per_stage<NHL>();
   static constexpr int CH_A = BM / 32 * KB * NHL * 64;  // 16-byte chunks per stage
   static constexpr int CH_B = BN / 32 * KB * NHL * 64;
   static constexpr int PER_A = CH_A / NT, PER_B = CH_B / NT;
-  static constexpr int SMEM_CHUNKS = 2 * (CH_A + CH_B);
+  static constexpr int FIT = 160 * 1024 / (16 * (CH_A + CH_B));
+  static constexpr int NB = FIT < 4 ? FIT : 4;
+  static constexpr int SMEM_CHUNKS = NB * (CH_A + CH_B);
   static_assert(CH_A % NT == 0 && CH_B % NT == 0, "stage must split evenly");
+  static_assert(KB % 2 == 0 && NB >= 2, "fragment sets alternate over an even number of k blocks");
+  static_assert((NB - 1) * (PER_A + PER_B) < 64, "in-flight DMA count fits vmcnt");
 };
 
 // Packed operands of one contraction.
@@ -232,50 +241,17 @@ struct BfTileArgs {
   int nblk_a;       // 32-row blocks held by PA / PB (rows padded to 32 only)
   int nblk_b;
   int nprod;        // 2: second product uses (PB, PA)
-  Epilogue ep;
+  Epilogue ep;      // of the whole problem
 };
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 u) { return __builtin_bit_cast(bf16x8, u); }
 
-// MFMAs of one 16-wide k block `kb` of an LDS stage: acc[i][j] +=
-// A-fragments x B-fragments; sa / sb are the stage's A / B chunks.
-template <int FM, int FN, int NHL>
-__device__ __forceinline__ void bf16_kb_mma(floatx16 (&acc)[FM][FN], const u32x4* sa, const u32x4* sb, int wm, int wn,
-    int lane, int kb) {
-  bf16x8 ah[FM], al[FM], bh[FN], bl[FN];
-#pragma unroll
-  for(int i = 0; i < FM; ++i) {
-    const int blk = wm * FM + i;
-    ah[i] = as_bf16x8(sa[(blk * kb_per_stage<NHL>() + kb) * NHL * 64 + lane]);
-    if(NHL == 2) al[i] = as_bf16x8(sa[((blk * kb_per_stage<NHL>() + kb) * NHL + 1) * 64 + lane]);
-  }
-#pragma unroll
-  for(int j = 0; j < FN; ++j) {
-    const int blk = wn * FN + j;
-    bh[j] = as_bf16x8(sb[(blk * kb_per_stage<NHL>() + kb) * NHL * 64 + lane]);
-    if(NHL == 2) bl[j] = as_bf16x8(sb[((blk * kb_per_stage<NHL>() + kb) * NHL + 1) * 64 + lane]);
-  }
-  // Product-major order: consecutive MFMAs write different accumulators, so
-  // none waits on the previous one's result.  The small cross terms go in
-  // first so they are added while the accumulator is smallest.
-  if(NHL == 2) {
-#pragma unroll
-    for(int i = 0; i < FM; ++i)
-#pragma unroll
-      for(int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-    for(int i = 0; i < FM; ++i)
-#pragma unroll
-      for(int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-  }
-#pragma unroll
-  for(int i = 0; i < FM; ++i)
-#pragma unroll
-    for(int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-}
-
-// bf16_kb_mma for a stage of KBS k blocks (chunk (blk, kb, hl, lane) of a
-// stage at ((blk * KBS + kb) * NHL + hl) * 64 + lane).
+// MFMAs of one 16-wide k block `kb` of an LDS stage of KBS k blocks (chunk
+// (blk, kb, hl, lane) at ((blk * KBS + kb) * NHL + hl) * 64 + lane):
+// acc[i][j] += A-fragments x B-fragments; sa / sb are the stage's A / B
+// chunks.  Product-major order: consecutive MFMAs write different
+// accumulators, so none waits on the previous one's result.  The small cross
+// terms go in first so they are added while the accumulator is smallest.
 template <int FM, int FN, int NHL, int KBS>
 __device__ __forceinline__ void bf16_kb_mma_n(floatx16 (&acc)[FM][FN], const u32x4* sa, const u32x4* sb, int wm, int wn,
     int lane, int kb) {
@@ -308,14 +284,6 @@ __device__ __forceinline__ void bf16_kb_mma_n(floatx16 (&acc)[FM][FN], const u32
     for(int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
 }
 
-// MFMAs of a whole LDS stage (kb_per_stage k blocks).
-template <int FM, int FN, int NHL>
-__device__ __forceinline__ void bf16_stage_mma(floatx16 (&acc)[FM][FN], const u32x4* sa, const u32x4* sb, int wm,
-    int wn, int lane) {
-#pragma unroll
-  for(int kb = 0; kb < kb_per_stage<NHL>(); ++kb) bf16_kb_mma<FM, FN, NHL>(acc, sa, sb, wm, wn, lane, kb);
-}
-
 template <int FM, int FN>
 __device__ __forceinline__ void zero_acc(floatx16 (&acc)[FM][FN]) {
 #pragma unroll
@@ -326,91 +294,6 @@ __device__ __forceinline__ void zero_acc(floatx16 (&acc)[FM][FN]) {
       for(int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
 }
 
-// Computes tile (tm, tn) from packed operands and writes it through t.ep.
-// `lds` holds BfCfg::SMEM_CHUNKS chunks; the caller separates two calls that
-// reuse it with a barrier.
-template <int BM, int BN, int WM, int WN, int NHL>
-__device__ __forceinline__ void bf16_tile(const BfTileArgs& t, int tm, int tn, u32x4* lds) {
-  using Cfg = BfCfg<BM, BN, WM, WN, NHL>;
-  constexpr int NT = Cfg::NT, FM = Cfg::FM, FN = Cfg::FN;
-  constexpr int SA = Cfg::CH_A, SB = Cfg::CH_B;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int wm = wid / Cfg::NWN, wn = wid % Cfg::NWN;
-
-  floatx16 acc[FM][FN];
-  zero_acc(acc);
-
-  // Chunk c of a stage: block c / RUN of the tile, then the contiguous
-  // (kb, hl, lane) run of that block for this stage.
-  constexpr int RUN = Cfg::KB * NHL * 64;
-  const int KT = t.kbs / Cfg::KB;
-  const int steps = KT * t.nprod;
-  const int64_t blk_stride = (int64_t)t.kbs * NHL * 64;
-  // Packed operands hold only the 32-row blocks that meet the matrix: a tile
-  // block past the last one reads the last block again.  Those rows feed only
-  // output rows / columns past M / N, which the epilogue never stores, so any
-  // finite data will do.
-  // Global -> LDS without registers (global_load_lds_dwordx4): for one wave
-  // and one i, the 64 lanes' chunks c = wave*64 + i*NT + lane are 64
-  // consecutive chunks both in the packed operand (RUN is a multiple of 64)
-  // and in the LDS stage, so each instruction moves one contiguous 1 KiB.
-  // The LDS base of a wave is uniform: readfirstlane lets the compiler keep it
-  // (and so M0) in scalar registers.  Per-thread chunk offsets within the
-  // tile's A and B panels are computed once (32-bit: at most BM/32 blocks of
-  // one panel); a stage only moves the wave-uniform panel base along k.
-  const int wave_base = __builtin_amdgcn_readfirstlane(tid - lane);
-  int off_a[2][Cfg::PER_A], off_b[2][Cfg::PER_B];
-#pragma unroll
-  for(int p = 0; p < 2; ++p) {
-    const int last_a = (p ? t.nblk_b : t.nblk_a) - 1, last_b = (p ? t.nblk_a : t.nblk_b) - 1;
-#pragma unroll
-    for(int i = 0; i < Cfg::PER_A; ++i) {
-      const int c = tid + i * NT;
-      const int blk = c / RUN, run = c - blk * RUN;
-      off_a[p][i] = (min(tm * (BM / 32) + blk, last_a) - tm * (BM / 32)) * (int)blk_stride + run;
-    }
-#pragma unroll
-    for(int i = 0; i < Cfg::PER_B; ++i) {
-      const int c = tid + i * NT;
-      const int blk = c / RUN, run = c - blk * RUN;
-      off_b[p][i] = (min(tn * (BN / 32) + blk, last_b) - tn * (BN / 32)) * (int)blk_stride + run;
-    }
-  }
-  auto issue = [&](int s, int buf) __attribute__((always_inline)) {
-    const int prod = s / KT, kt = s - prod * KT;
-    const u32x4* A = (prod ? t.PB : t.PA) + ((int64_t)tm * (BM / 32) * blk_stride + (int64_t)kt * RUN);
-    const u32x4* B = (prod ? t.PA : t.PB) + ((int64_t)tn * (BN / 32) * blk_stride + (int64_t)kt * RUN);
-    u32x4* sa = lds + buf * (SA + SB);
-    u32x4* sb = sa + SA;
-#pragma unroll
-    for(int i = 0; i < Cfg::PER_A; ++i) lds_dma16(A + (prod ? off_a[1][i] : off_a[0][i]), sa + wave_base + i * NT);
-#pragma unroll
-    for(int i = 0; i < Cfg::PER_B; ++i) lds_dma16(B + (prod ? off_b[1][i] : off_b[0][i]), sb + wave_base + i * NT);
-  };
-  auto compute = [&](int cur) __attribute__((always_inline)) {
-    const u32x4* sa = lds + cur * (SA + SB);
-    bf16_stage_mma<FM, FN, NHL>(acc, sa, sa + SA, wm, wn, lane);
-  };
-
-  // Stage s+1 streams into the other buffer while stage s is contracted; the
-  // buffer it overwrites was last read before the previous barrier.
-  if(steps > 0) issue(0, 0);
-  lds_dma_wait();
-  __syncthreads();
-  for(int s = 0; s + 1 < steps; ++s) {
-    issue(s + 1, (s + 1) & 1);
-    compute(s & 1);
-    lds_dma_wait();
-    __syncthreads();
-  }
-  if(steps > 0) compute((steps - 1) & 1);
-
-  static_for<FM * FN>([&](auto ij) __attribute__((always_inline)) {
-    constexpr int i = decltype(ij)::value / FN, j = decltype(ij)::value % FN;
-    store_block32(t.ep, acc[i][j], tm * BM + wm * WM + i * 32, tn * BN + wn * WN + j * 32, lane);
-  });
-}
-
 // Waits until at most n of this wave's vector memory operations are
 // outstanding (s_waitcnt vmcnt(n), n <= 63; expcnt and lgkmcnt left alone).
 template <int n>
@@ -419,8 +302,183 @@ __device__ __forceinline__ void vm_wait() {
   __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
-// bf16_tile with a deeper pipeline: NB LDS buffers of KB k blocks each, NB-1
-// stages in flight.  A tile whose panels come from HBM rather than L2 (one
+// Waits for this wave's outstanding LDS operations only.
+__device__ __forceinline__ void lds_wait() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
+
+// s_barrier alone, with memory accesses kept on their side of it: the caller
+// has waited for what the other waves may read or overwrite.  (__syncthreads
+// would also wait for the global-to-LDS copies still in flight.)
+__device__ __forceinline__ void bare_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Contracts stages [s0, s1) of tile (tm, tn) from packed operands and writes
+// alpha * sum + beta * C through `ep` at row er, column ec.  The whole tile is
+// stages 0 .. kbs / KB * nprod (the second product's follow the first's).
+// `lds` holds BfCfg::SMEM_CHUNKS chunks; the caller separates two calls that
+// reuse it with a barrier.
+//
+// A wave keeps two sets of fragment registers: while the MFMAs of one k block
+// run, the LDS reads of the next are issued between them, across the stage
+// boundary too.  At a boundary every wave has read the old stage into
+// registers and still has one k block of MFMAs to issue, so the barrier and
+// the LDS latency are covered, and the stage NB further on is copied into the
+// buffer just freed, its DMA instructions spread over the same MFMAs.
+// sched_barrier keeps that order (the compiler otherwise gathers a k block's
+// reads in front of its MFMAs and waits for all of them: the MFMA pipe was
+// busy 66 % of the time in split BF16 and 49 % in single BF16).  Each DMA
+// instruction's source is uniform over the wave but for the lane's 16 bytes,
+// so its address is kept in scalar registers.  The order of the MFMAs of one
+// accumulator is k block by k block, lo*hi, hi*lo, hi*hi within one.
+// Measured on MI355X, kernel alone, against one stage in flight and fragments
+// read when needed: N = 8192 split BF16 2.48 -> 2.12 ms (1331 -> 1555
+// TFLOP/s), single BF16 0.947 -> 0.796 ms; 1024 x 1024 x 4096 split BF16 on
+// 64x64 tiles 75.7 -> 31.6 us.
+template <int BM, int BN, int WM, int WN, int NHL>
+__device__ __forceinline__ void bf16_tile(const BfTileArgs& t, int tm, int tn, int s0, int s1, const Epilogue& ep,
+    int er, int ec, u32x4* lds) {
+  using Cfg = BfCfg<BM, BN, WM, WN, NHL>;
+  constexpr int NT = Cfg::NT, FM = Cfg::FM, FN = Cfg::FN, KB = Cfg::KB, NB = Cfg::NB;
+  constexpr int SA = Cfg::CH_A, STAGE = Cfg::CH_A + Cfg::CH_B;
+  constexpr int PER = Cfg::PER_A + Cfg::PER_B;  // DMA instructions per stage and wave
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wid / Cfg::NWN, wn = wid % Cfg::NWN;
+
+  floatx16 acc[FM][FN];
+  zero_acc(acc);
+
+  // DMA instruction i of a wave moves 64 consecutive chunks c = wave * 64 +
+  // i * NT of a stage: block c / RUN of the tile, then the contiguous (kb,
+  // hl, lane) run of that block.  Packed operands hold only the 32-row blocks
+  // that meet the matrix: a tile block past the last one reads the last block
+  // again.  Those rows feed only output rows / columns past M / N, which the
+  // epilogue never stores, so any data will do.
+  constexpr int RUN = KB * NHL * 64;
+  const int KT = t.kbs / KB;
+  const int64_t blk_stride = (int64_t)t.kbs * NHL * 64;
+  const int wave_base = wid * 64;
+  int64_t off[PER];
+#pragma unroll
+  for(int i = 0; i < PER; ++i) {
+    const bool is_a = i < Cfg::PER_A;
+    const int c = wave_base + (is_a ? i : i - Cfg::PER_A) * NT, blk = c / RUN, run = c - blk * RUN;
+    off[i] = (is_a ? (int64_t)min(tm * (BM / 32) + blk, t.nblk_a - 1) : (int64_t)min(tn * (BN / 32) + blk, t.nblk_b - 1)) *
+                 blk_stride +
+             run;
+  }
+  // the next stage to issue, its k position in both operands and its buffer;
+  // past the last stage the last one is read again (into a buffer that no one
+  // reads any more), so the loop has no branch around its loads
+  int next = s0;
+  const bool swapped = s0 >= KT;  // product 1 reads (PB, PA)
+  const u32x4* cur_a = (swapped ? t.PB : t.PA) + (int64_t)(swapped ? s0 - KT : s0) * RUN;
+  const u32x4* cur_b = (swapped ? t.PA : t.PB) + (int64_t)(swapped ? s0 - KT : s0) * RUN;
+  u32x4* dst = lds;
+  auto issue_one = [&](int i) __attribute__((always_inline)) {
+    const bool is_a = i < Cfg::PER_A;
+    const char* src = reinterpret_cast<const char*>((is_a ? cur_a : cur_b) + off[i]);
+    lds_dma16(reinterpret_cast<const u32x4*>(src + (uint32_t)lane * 16),
+        dst + (is_a ? i * NT : SA + (i - Cfg::PER_A) * NT) + wave_base);
+  };
+  auto advance = [&]() __attribute__((always_inline)) {
+    ++next;
+    dst = dst + STAGE == lds + NB * STAGE ? lds : dst + STAGE;
+    const u32x4* na = next == KT ? t.PB : cur_a + RUN;
+    const u32x4* nb = next == KT ? t.PA : cur_b + RUN;
+    cur_a = next < s1 ? na : cur_a;
+    cur_b = next < s1 ? nb : cur_b;
+  };
+
+  u32x4 ah[2][FM], al[2][FM], bh[2][FN], bl[2][FN];
+  constexpr int NR = (FM + FN) * NHL;               // LDS reads per k block
+  constexpr int NM = (NHL == 2 ? 3 : 1) * FM * FN;  // MFMAs per k block
+  // Read r of k block kb of the stage at `st` into fragment set q, in the
+  // order the products need them.
+  auto read_one = [&](const u32x4* st, int kb, auto qq, auto rr) __attribute__((always_inline)) {
+    constexpr int q = decltype(qq)::value, r = decltype(rr)::value;
+    auto a_at = [&](int i, int hl) { return st[(((wm * FM + i) * KB + kb) * NHL + hl) * 64 + lane]; };
+    auto b_at = [&](int j, int hl) { return st[SA + (((wn * FN + j) * KB + kb) * NHL + hl) * 64 + lane]; };
+    if constexpr(r < FN) bh[q][r] = b_at(r, 0);
+    else if constexpr(NHL == 1) ah[q][r - FN] = a_at(r - FN, 0);
+    else if constexpr(r < FN + FM) al[q][r - FN] = a_at(r - FN, 1);
+    else if constexpr(r < 2 * FN + FM) bl[q][r - FN - FM] = b_at(r - FN - FM, 1);
+    else ah[q][r - 2 * FN - FM] = a_at(r - 2 * FN - FM, 0);
+  };
+  // The MFMAs of fragment set q, with the reads of the next k block (kb of
+  // the stage at `st`) into the other set over the first three quarters of
+  // them, and the next stage's DMA over all of them.
+  auto contract = [&](auto qq, const u32x4* st, int kb, auto reads, auto dma) __attribute__((always_inline)) {
+    constexpr int q = decltype(qq)::value;
+    static_for<NM>([&](auto mm) __attribute__((always_inline)) {
+      constexpr int m = decltype(mm)::value;
+      constexpr int MR = NM * 3 / 4 > 0 ? NM * 3 / 4 : 1;
+      constexpr int r0 = m < MR ? m * NR / MR : NR, r1 = m < MR ? (m + 1) * NR / MR : NR;
+      if constexpr(decltype(reads)::value)
+        static_for<r1 - r0>([&](auto x) __attribute__((always_inline)) {
+          read_one(st, kb, std::integral_constant<int, 1 - q>{}, std::integral_constant<int, r0 + decltype(x)::value>{});
+        });
+      constexpr int d0 = m * PER / NM, d1 = (m + 1) * PER / NM;
+      if constexpr(decltype(dma)::value)
+        static_for<d1 - d0>([&](auto x) __attribute__((always_inline)) { issue_one(d0 + decltype(x)::value); });
+      constexpr int prod = NHL == 2 ? m / (FM * FN) : 2, i = m % (FM * FN) / FN, j = m % FN;
+      const u32x4 fa = prod == 0 ? al[q][i] : ah[q][i], fb = prod == 1 ? bl[q][j] : bh[q][j];
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(fa), as_bf16x8(fb), acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  using Q0 = std::integral_constant<int, 0>;
+  using Q1 = std::integral_constant<int, 1>;
+  using Yes = std::true_type;
+  using No = std::false_type;
+  // all k blocks of a stage but the last, whose fragments end up in set 1
+  auto body = [&](const u32x4* st) __attribute__((always_inline)) {
+#pragma unroll
+    for(int kb = 0; kb + 2 < KB; kb += 2) {
+      contract(Q0{}, st, kb + 1, Yes{}, No{});
+      contract(Q1{}, st, kb + 2, Yes{}, No{});
+    }
+    contract(Q0{}, st, KB - 1, Yes{}, No{});
+  };
+
+  if(s1 > s0) {
+#pragma unroll
+    for(int b = 0; b < NB; ++b) {
+#pragma unroll
+      for(int i = 0; i < PER; ++i) issue_one(i);
+      advance();
+    }
+    vm_wait<(NB - 1) * PER>();  // stage s0
+    bare_barrier();
+    static_for<NR>([&](auto rr) __attribute__((always_inline)) { read_one(lds, 0, Q0{}, rr); });
+    const u32x4* st = lds;
+    for(int s = s0; s + 1 < s1; ++s) {
+      body(st);
+      // stage s + 1 has landed (the NB - 2 issued after it may still be in
+      // flight) and this wave has read all of stage s
+      vm_wait<(NB - 2) * PER>();
+      lds_wait();
+      bare_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      st = st + STAGE == lds + NB * STAGE ? lds : st + STAGE;
+      contract(Q1{}, st, 0, Yes{}, Yes{});
+      advance();
+    }
+    body(st);
+    contract(Q1{}, st, 0, No{}, No{});
+  }
+  lds_dma_wait();  // no copy into LDS is left behind
+
+  static_for<FM * FN>([&](auto ij) __attribute__((always_inline)) {
+    constexpr int i = decltype(ij)::value / FN, j = decltype(ij)::value % FN;
+    store_block32(ep, acc[i][j], er + wm * WM + i * 32, ec + wn * WN + j * 32, lane);
+  });
+}
+
+// The grouped kernels' tile on packed operands: NB LDS buffers of KB k
+// blocks each, NB-1 stages in flight.  A tile whose panels come from HBM rather than L2 (one
 // tile per problem, as in a batch of small problems) is bound by the bytes
 // it keeps in flight: two 64 KiB stages (one in flight) stream at about
 // 3.7 TB/s over the chip, so four 32 KiB stages (three in flight) in the
