@@ -352,7 +352,7 @@ mfx_status mfx_config_info(mfx_precision prec, int32_t config, int32_t* bm, int3
     int32_t* bk, int32_t* waves);
 /* Forces `config` (or -1 for the tuned / heuristic choice) for later calls of `prec`. */
 mfx_status mfx_force_config(mfx_handle handle, mfx_precision prec, int32_t config);
-/* Split-K override for later FP32, SPLIT_BF16 and BF16 calls: -1 automatic
+/* Split-K override for later gemm / syrk / syr2k calls: -1 automatic
  * (the default: k slices when the tile grid leaves the CUs short of work),
  * 1 never, >= 2 that many k slices (fewer when K or the 32 MiB partial-tile
  * bound does not allow them; FP32 splits single products on tiles up to

@@ -210,7 +210,7 @@ int least_time_config(Handle* h, mfx_precision p, bool square_only, Tiles&& tile
 }
 
 // The configuration whose estimated launch, split-K included, is shortest
-// (plan_splits; split / single BF16).  `tiles(bm, bn)` as above.
+// (plan_splits; every precision but FP32).  `tiles(bm, bn)` as above.
 template <class Tiles>
 int least_cost_config(Handle* h, mfx_precision p, int64_t k, bool square_only, Tiles&& tiles) {
   int best = 0;
@@ -227,7 +227,7 @@ int least_cost_config(Handle* h, mfx_precision p, int64_t k, bool square_only, T
   return best;
 }
 
-bool has_cost_model(mfx_precision p) { return p == MFX_PREC_SPLIT_BF16 || p == MFX_PREC_BF16; }
+bool has_cost_model(mfx_precision p) { return p != MFX_PREC_FP32; }
 
 // FP32 configuration with sixteen waves on a 64x64 tile (four k-groups).
 constexpr int kF32KGroupConfig = 7;
@@ -545,7 +545,7 @@ size_t mfx_gemm_workspace_size(mfx_precision prec, int64_t m, int64_t n, int64_t
     } else if(prec == MFX_PREC_SPLIT_BF16 || prec == MFX_PREC_BF16)
       b = dense_bf16x_workspace(op, prec == MFX_PREC_SPLIT_BF16, c, cus, -1);
     else if(prec == MFX_PREC_FP8_BLOCK || prec == MFX_PREC_FP8_BLOCK2)
-      b = dense_fp8_workspace(op, prec == MFX_PREC_FP8_BLOCK2, c);
+      b = dense_fp8_workspace(op, prec == MFX_PREC_FP8_BLOCK2, c, cus);
     best = std::max(best, b);
   }
   return best;

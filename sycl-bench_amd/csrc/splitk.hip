@@ -101,16 +101,26 @@ constexpr TileCost kBf16Cost[] = {
     {7.5, 16.0, 24.5}, {4.5, 6.2, 8.2}, {3.4, 3.87, 3.9}, {5.5, 9.7, 14.0},
     {6.0, 15.4, 24.5}, {5.3, 9.5, 13.8}, {4.0, 6.1, 8.3},
 };
+constexpr TileCost kFp8Cost[] = {
+    {16.0, 7.7, 10.8},  // 256x256, four waves
+    {6.5, 2.8, 3.5},    // 128x128
+    {10.0, 7.8, 10.9},  // 256x256, eight waves
+    {3.0, 1.6, 1.9},    // 64x64
+};
+constexpr TileCost kFp8TwoCost[] = {{14.0, 22.5, 30.6}, {6.0, 7.7, 9.7}, {9.0, 22.7, 32.0}, {3.0, 3.9, 4.3}};
 
 // Reading the partials back and the launch that does it.
 constexpr double kReduceFixedUs = 4.0, kReduceBytesPerUs = 3.0e6;
 
 bool tile_cost(mfx_precision p, int c, TileCost* out) {
-  if(c < 0 || c >= 7) return false;
-  if(p == MFX_PREC_SPLIT_BF16) *out = kSplitCost[c];
-  else if(p == MFX_PREC_BF16) *out = kBf16Cost[c];
-  else return false;
-  return true;
+  if(c < 0 || c >= config_count(p)) return false;
+  switch(p) {
+    case MFX_PREC_SPLIT_BF16: *out = kSplitCost[c]; return true;
+    case MFX_PREC_BF16: *out = kBf16Cost[c]; return true;
+    case MFX_PREC_FP8_BLOCK: *out = kFp8Cost[c]; return true;
+    case MFX_PREC_FP8_BLOCK2: *out = kFp8TwoCost[c]; return true;
+    default: return false;
+  }
 }
 
 }  // namespace

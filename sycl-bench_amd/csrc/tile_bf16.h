@@ -15,7 +15,7 @@
 // the tile size and k to the 32-wide stage with zeros.
 #pragma once
 
-#include "mfx_internal.h"
+#include "lds_pipe.h"
 
 namespace mfx {
 
@@ -292,26 +292,6 @@ __device__ __forceinline__ void zero_acc(floatx16 (&acc)[FM][FN]) {
     for(int j = 0; j < FN; ++j)
 #pragma unroll
       for(int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
-}
-
-// Waits until at most n of this wave's vector memory operations are
-// outstanding (s_waitcnt vmcnt(n), n <= 63; expcnt and lgkmcnt left alone).
-template <int n>
-__device__ __forceinline__ void vm_wait() {
-  static_assert(n >= 0 && n < 64, "vmcnt holds 6 bits");
-  __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-// Waits for this wave's outstanding LDS operations only.
-__device__ __forceinline__ void lds_wait() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
-
-// s_barrier alone, with memory accesses kept on their side of it: the caller
-// has waited for what the other waves may read or overwrite.  (__syncthreads
-// would also wait for the global-to-LDS copies still in flight.)
-__device__ __forceinline__ void bare_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 // Contracts stages [s0, s1) of tile (tm, tn) from packed operands and writes

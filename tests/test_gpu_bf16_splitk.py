@@ -1,4 +1,4 @@
-"""Split-K of the packed split / single BF16 path (GPU, through the C ABI):
+"""Split-K of the packed BF16 and FP8 paths (GPU, through the C ABI):
 whole tiles and k slices in one launch, the slices' partial tiles summed in
 slice order by splitk_reduce, on full and triangular schedules.
 
@@ -118,3 +118,30 @@ def test_whole_rounds_and_a_split_rest(handle, prec):
         handle.force_config(prec, -1)
     assert "splitk_reduce" in rec, rec
     assert rel(C, 1.5 * A.double() @ B.double() + 0.5 * C0.double()) < TOL[prec]
+
+
+@pytest.mark.parametrize("prec", ["fp8-block", "fp8-block2"])
+@pytest.mark.parametrize("config", [0, 1, 2, 3])
+@pytest.mark.parametrize("m,n,k,ta,tb,splits", [(64, 64, 128, False, False, 2), (200, 130, 700, True, False, 3),
+                                                (300, 270, 1000, False, True, 64)])
+def test_fp8_slices(handle, prec, config, m, n, k, ta, tb, splits):
+    """Slices of block-scaled FP8 tiles against the whole tiles' result: the
+    same codes and scales, so they differ by the instruction's summation error
+    only (about 2^-15 relative per 64-wide dot, as for the product itself)."""
+    print(f"fp8 split {prec} config {config} {m}x{n}x{k} ta={ta} tb={tb} S={splits}", flush=True)
+    A = seeded(handle, k if ta else m, m if ta else k, 0)
+    B = seeded(handle, n if tb else k, k if tb else n, 1)
+    C0 = seeded(handle, m, n, 2)
+    outs = {}
+    handle.force_config(prec, config)
+    try:
+        for s in (1, splits):
+            handle.force_splits(s)
+            C = C0.clone()
+            rec = recorded(handle, lambda: handle.gemm(A, B, C, alpha=1.5, beta=0.5, prec=prec, transA=ta, transB=tb))
+            assert ("splitk_reduce" in rec) == (s > 1 and k > 128), rec
+            outs[s] = C
+    finally:
+        handle.force_config(prec, -1)
+        handle.force_splits(-1)
+    assert rel(outs[splits], outs[1].double()) < 1e-4
