@@ -35,33 +35,39 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------
 // Quantisation
 // ---------------------------------------------------------------------------
-struct QuantParams {
+struct QuantOperand {
   const float* src;
   int64_t ld;
   int rows, K;
   int kmajor;       // element (r, k) at src[r*ld + k], else src[k*ld + r]
-  int vec;          // kmajor with 16-byte aligned rows: 128-bit loads
-  int kb128s;       // padded K / 128
-  int two_term;
+  int vec;          // 16-byte aligned rows: 128-bit loads along the contiguous dimension
+  int row_blocks, k_blocks;  // blocks of the padded operand
   u32x4* q1;        // packed, fragment order
   u32x4* q2;
-  int* e1;          // [rows_pad/128][kb128s]
+  int* e1;          // [row_blocks][k_blocks]
   int* e2;
-  // plain row-major output (mfx_quantize_fp8_block), used when q1 == nullptr
+  // plain row-major output (mfx_quantize_fp8_block)
   uint8_t* plain;
   int64_t plain_ld;
-  int block;        // 128 for the contraction; 32/64/128 for the utility
+};
+struct QuantParams {
+  QuantOperand a, b;
+  int grid_a;  // workgroups of a; the rest are b's
 };
 
+// Largest v of the workgroup's NT threads.
+template <int NT>
 __device__ __forceinline__ float block_max(float v, float* sh) {
   for(int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  const int w = threadIdx.x >> 6;
-  __syncthreads();
-  if((threadIdx.x & 63) == 0) sh[w] = v;
-  __syncthreads();
-  float m = sh[0];
-  for(int i = 1; i < (int)(blockDim.x >> 6); ++i) m = fmaxf(m, sh[i]);
-  return m;
+  if constexpr(NT > 64) {
+    __syncthreads();
+    if((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = sh[0];
+#pragma unroll
+    for(int i = 1; i < NT / 64; ++i) v = fmaxf(v, sh[i]);
+  }
+  return v;
 }
 
 // e4m3 codes of four floats, packed little-endian into one word, by the
@@ -80,118 +86,129 @@ __device__ __forceinline__ float e4m3_byte(uint32_t w) {
   return __builtin_amdgcn_cvt_f32_fp8((int)w, J);
 }
 
-// One workgroup per (row block, k block) of `block` x `block` elements;
-// thread t handles chunks of 16 consecutive k of one row.  k-contiguous
-// sources put consecutive threads along k (64-byte vector loads per
-// thread); row-contiguous ones put them along the rows (coalesced across
-// lanes).
 // Row pitch (bytes) of the LDS code tile: 128 codes + 16, so 16-byte reads
 // of one column by consecutive rows spread over the banks.
 constexpr int QPITCH = 144;
 
-__global__ __launch_bounds__(256) void quantize_fp8_kernel(const QuantParams p) {
-  __shared__ float sh[4];
-  __shared__ __align__(16) unsigned char qtile[2][128 * QPITCH];
-  // Neighbouring workgroups take neighbouring blocks along the source's
-  // contiguous dimension (k if k-major, rows if not), so they read
-  // neighbouring segments of the same memory rows.
-  const int rb = p.kmajor ? blockIdx.y : blockIdx.x, kb = p.kmajor ? blockIdx.x : blockIdx.y;
-  const int B = p.block;
-  const int per_row = B / 16;
-  const int chunks = B * per_row;  // <= 1024
-  float v[4][16];
+// One workgroup per B x B block, sixteen elements per thread in four 16-byte
+// loads: of four rows, 4 k each (k-contiguous source; half a wave covers a
+// 512-byte row segment), or of 4 k, four rows each (row-contiguous source; 8
+// threads cover 128 bytes of a row of the source), so a thread packs four
+// code words either way.  Neighbouring workgroups take neighbouring blocks
+// along the source's contiguous dimension.  HBM-bound; sixteen elements per
+// thread instead of sixty-four keep the two passes over the block (largest
+// magnitude, codes) short and the CU full: a 16384^2 operand 288 us (4.65
+// TB/s) -> 262 us (5.1 TB/s); the operands of a 1500 x 1100 x 2000 call 14.4 + 13.1
+// -> 13 us in one launch.
+template <int B, int T, bool PLAIN>
+__global__ __launch_bounds__(B * B / 16) void quantize_fp8_kernel(const QuantParams pp) {
+  constexpr int NT = B * B / 16;
+  __shared__ float sh[16];
+  __shared__ __align__(16) unsigned char qtile[PLAIN ? 1 : T][PLAIN ? 16 : 128 * QPITCH];
+  const bool first = (int)blockIdx.x < pp.grid_a;
+  const QuantOperand& p = first ? pp.a : pp.b;
+  const int id = first ? blockIdx.x : blockIdx.x - pp.grid_a;
+  const int rb = p.kmajor ? id / p.k_blocks : id % p.row_blocks;
+  const int kb = p.kmajor ? id % p.k_blocks : id / p.row_blocks;
+  const int t = threadIdx.x;
+  // word w of the thread: codes of row lr + w * row_step, k lk .. lk + 3
+  int lr, lk, row_step;
+  float v[4][4];  // [word][k]
   float amax = 0.0f;
+  if(p.kmajor) {
+    lr = t / (B / 4);
+    lk = t % (B / 4) * 4;
+    row_step = B / 4;
 #pragma unroll
-  for(int c = 0; c < 4; ++c) {
-    const int id = threadIdx.x + c * 256;
-    const int rr = p.kmajor ? id / per_row : id % B, kk = p.kmajor ? id % per_row : id / B;
-    const int r = rb * B + rr, k0 = kb * B + kk * 16;
-    const bool live = id < chunks && r < p.rows;
-    if(p.kmajor) {
-      const float* src = p.src + (int64_t)r * p.ld + k0;
-      if(live && p.vec && k0 + 16 <= p.K) {
-#pragma unroll
-        for(int q = 0; q < 4; ++q) {
-          const float4 x = reinterpret_cast<const float4*>(src)[q];
-          v[c][4 * q] = x.x;
-          v[c][4 * q + 1] = x.y;
-          v[c][4 * q + 2] = x.z;
-          v[c][4 * q + 3] = x.w;
-        }
+    for(int w = 0; w < 4; ++w) {
+      const int r = rb * B + lr + w * row_step, k = kb * B + lk;
+      const float* src = p.src + (int64_t)r * p.ld + k;
+      if(r < p.rows && p.vec && k + 4 <= p.K) {
+        const float4 x = *reinterpret_cast<const float4*>(src);
+        v[w][0] = x.x;
+        v[w][1] = x.y;
+        v[w][2] = x.z;
+        v[w][3] = x.w;
       } else {
 #pragma unroll
-        for(int e = 0; e < 16; ++e) v[c][e] = (live && k0 + e < p.K) ? src[e] : 0.0f;
+        for(int e = 0; e < 4; ++e) v[w][e] = r < p.rows && k + e < p.K ? src[e] : 0.0f;
       }
-    } else {
-#pragma unroll
-      for(int e = 0; e < 16; ++e) v[c][e] = (live && k0 + e < p.K) ? p.src[(int64_t)(k0 + e) * p.ld + r] : 0.0f;
     }
+  } else {
+    // a wave covers 32 rows x 32 k
+    constexpr int RW = B / 32;  // waves along the rows
+    const int wave = t >> 6, lane = t & 63;
+    lr = wave % RW * 32 + (lane & 7) * 4;
+    lk = wave / RW * 32 + (lane >> 3) * 4;
+    row_step = 1;
 #pragma unroll
-    for(int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(v[c][e]));
+    for(int e = 0; e < 4; ++e) {
+      const int r = rb * B + lr, k = kb * B + lk + e;
+      const float* src = p.src + (int64_t)k * p.ld + r;
+      if(k < p.K && p.vec && r + 4 <= p.rows) {
+        const float4 x = *reinterpret_cast<const float4*>(src);
+        v[0][e] = x.x;
+        v[1][e] = x.y;
+        v[2][e] = x.z;
+        v[3][e] = x.w;
+      } else {
+#pragma unroll
+        for(int w = 0; w < 4; ++w) v[w][e] = k < p.K && r + w < p.rows ? src[w] : 0.0f;
+      }
+    }
   }
-  const int ex1 = fp8_block_exponent(block_max(amax, sh));
+#pragma unroll
+  for(int w = 0; w < 4; ++w)
+#pragma unroll
+    for(int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(v[w][e]));
+  const int ex1 = fp8_block_exponent(block_max<NT>(amax, sh));
   const float inv1 = ldexpf(1.0f, -ex1), s1 = ldexpf(1.0f, ex1);
-  uint32_t w1[4][4];
+  uint32_t w1[4], w2[4];
   float amax2 = 0.0f;
 #pragma unroll
-  for(int c = 0; c < 4; ++c)
-#pragma unroll
-    for(int j = 0; j < 4; ++j) {
-      float* x = &v[c][4 * j];
-      w1[c][j] = e4m3_pack4(x[0] * inv1, x[1] * inv1, x[2] * inv1, x[3] * inv1);
-      if(p.two_term) {
-        x[0] -= e4m3_byte<0>(w1[c][j]) * s1;
-        x[1] -= e4m3_byte<1>(w1[c][j]) * s1;
-        x[2] -= e4m3_byte<2>(w1[c][j]) * s1;
-        x[3] -= e4m3_byte<3>(w1[c][j]) * s1;
-        amax2 = fmaxf(amax2, fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
-      }
-    }
-  int ex2 = 0;
-  float inv2 = 1.0f;
-  if(p.two_term) {
-    ex2 = fp8_block_exponent(block_max(amax2, sh));
-    inv2 = ldexpf(1.0f, -ex2);
-  }
-  if(threadIdx.x == 0) {
-    p.e1[rb * p.kb128s + kb] = ex1;
-    if(p.two_term) p.e2[rb * p.kb128s + kb] = ex2;
-  }
-#pragma unroll
-  for(int c = 0; c < 4; ++c) {
-    const int id = threadIdx.x + c * 256;
-    if(id >= chunks) continue;
-    const int rr = p.kmajor ? id / per_row : id % B, kk = p.kmajor ? id % per_row : id / B;
-    const int r = rb * B + rr, k0 = kb * B + kk * 16;
-    uint32_t w2[4] = {0, 0, 0, 0};
-    if(p.two_term)
-#pragma unroll
-      for(int j = 0; j < 4; ++j)
-        w2[j] = e4m3_pack4(v[c][4 * j] * inv2, v[c][4 * j + 1] * inv2, v[c][4 * j + 2] * inv2, v[c][4 * j + 3] * inv2);
-    if(p.q1) {
-      // codes of (rr, kk*16 .. kk*16+15) into the block's LDS tile
-      *reinterpret_cast<u32x4*>(&qtile[0][rr * QPITCH + kk * 16]) = (u32x4){w1[c][0], w1[c][1], w1[c][2], w1[c][3]};
-      if(p.two_term) *reinterpret_cast<u32x4*>(&qtile[1][rr * QPITCH + kk * 16]) = (u32x4){w2[0], w2[1], w2[2], w2[3]};
-    } else if(r < p.rows) {
-      for(int e = 0; e < 16 && k0 + e < p.K; ++e)
-        p.plain[(int64_t)r * p.plain_ld + k0 + e] = (uint8_t)(w1[c][e / 4] >> (8 * (e % 4)));
+  for(int w = 0; w < 4; ++w) {
+    float* x = v[w];
+    w1[w] = e4m3_pack4(x[0] * inv1, x[1] * inv1, x[2] * inv1, x[3] * inv1);
+    if constexpr(T == 2) {
+      x[0] -= e4m3_byte<0>(w1[w]) * s1;
+      x[1] -= e4m3_byte<1>(w1[w]) * s1;
+      x[2] -= e4m3_byte<2>(w1[w]) * s1;
+      x[3] -= e4m3_byte<3>(w1[w]) * s1;
+      amax2 = fmaxf(amax2, fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
     }
   }
-  if(p.q1) {
-    // The block's 1024 fragment-order chunks (block = 128 here), consecutive
-    // threads on consecutive chunks: chunk (blk, kb64, half, lane) holds the
-    // codes of row blk*32 + lane%32, k = kb64*64 + 32*(lane/32) + 16*half + 0..15.
+  if(t == 0) p.e1[(int64_t)rb * p.k_blocks + kb] = ex1;
+  if constexpr(T == 2) {
+    const int ex2 = fp8_block_exponent(block_max<NT>(amax2, sh));
+    const float inv2 = ldexpf(1.0f, -ex2);
+    if(t == 0) p.e2[(int64_t)rb * p.k_blocks + kb] = ex2;
+#pragma unroll
+    for(int w = 0; w < 4; ++w) w2[w] = e4m3_pack4(v[w][0] * inv2, v[w][1] * inv2, v[w][2] * inv2, v[w][3] * inv2);
+  }
+  if constexpr(PLAIN) {
+#pragma unroll
+    for(int w = 0; w < 4; ++w) {
+      const int r = rb * B + lr + w * row_step, k = kb * B + lk;
+      if(r < p.rows)
+        for(int e = 0; e < 4 && k + e < p.K; ++e) p.plain[(int64_t)r * p.plain_ld + k + e] = (uint8_t)(w1[w] >> (8 * e));
+    }
+  } else {
+    static_assert(B == 128, "fragment order holds 128 x 128 blocks");
+#pragma unroll
+    for(int w = 0; w < 4; ++w) {
+      *reinterpret_cast<uint32_t*>(&qtile[0][(lr + w * row_step) * QPITCH + lk]) = w1[w];
+      if constexpr(T == 2) *reinterpret_cast<uint32_t*>(&qtile[T - 1][(lr + w * row_step) * QPITCH + lk]) = w2[w];
+    }
+    // The block's 1024 fragment-order chunks, consecutive threads on
+    // consecutive chunks: chunk (blk, kb64, half, lane) holds the codes of row
+    // blk*32 + lane%32, k = kb64*64 + 32*(lane/32) + 16*half + 0..15.
     __syncthreads();
-    const int kb64s = p.kb128s * 2;
-#pragma unroll
-    for(int c = 0; c < 4; ++c) {
-      const int ch = threadIdx.x + c * 256;
-      const int lane = ch & 63, half = (ch >> 6) & 1, kb64l = (ch >> 7) & 1, blkl = ch >> 8;
-      const int row = blkl * 32 + (lane & 31), col = kb64l * 64 + 32 * (lane >> 5) + 16 * half;
-      const int64_t at = ((((int64_t)(rb * 4 + blkl)) * kb64s + kb * 2 + kb64l) * 2 + half) * 64 + lane;
-      p.q1[at] = *reinterpret_cast<const u32x4*>(&qtile[0][row * QPITCH + col]);
-      if(p.two_term) p.q2[at] = *reinterpret_cast<const u32x4*>(&qtile[1][row * QPITCH + col]);
-    }
+    const int kb64s = p.k_blocks * 2;
+    const int lane = t & 63, half = (t >> 6) & 1, kb64l = (t >> 7) & 1, blkl = t >> 8;
+    const int row = blkl * 32 + (lane & 31), col = kb64l * 64 + 32 * (lane >> 5) + 16 * half;
+    const int64_t at = ((((int64_t)(rb * 4 + blkl)) * kb64s + kb * 2 + kb64l) * 2 + half) * 64 + lane;
+    p.q1[at] = *reinterpret_cast<const u32x4*>(&qtile[0][row * QPITCH + col]);
+    if constexpr(T == 2) p.q2[at] = *reinterpret_cast<const u32x4*>(&qtile[T - 1][row * QPITCH + col]);
   }
 }
 
@@ -534,26 +551,22 @@ void launch_fp8_cfg(const Fp8Params& p, bool two_term, int grid, hipStream_t s) 
   else gemm_fp8_kernel<BM, BN, WM, WN, 1><<<grid, Fp8Cfg<BM, BN, WM, WN, 1>::NT, 0, s>>>(p);
 }
 
-mfx_status quantize(Handle* h, const float* src, int64_t ld, int rows, int K, bool kmajor, int64_t rows_pad,
-    int64_t kb128s, bool two, u32x4* q1, u32x4* q2, int* e1, int* e2, hipStream_t s) {
-  QuantParams p{};
-  p.src = src;
-  p.ld = ld;
-  p.rows = rows;
-  p.K = K;
-  p.kmajor = kmajor;
-  p.vec = kmajor && (reinterpret_cast<uintptr_t>(src) & 15u) == 0 && ld % 4 == 0;
-  p.kb128s = (int)kb128s;
-  p.two_term = two;
-  p.q1 = q1;
-  p.q2 = q2;
-  p.e1 = e1;
-  p.e2 = e2;
-  p.block = 128;
-  const unsigned rbs = (unsigned)(rows_pad / 128);
-  const dim3 grid = kmajor ? dim3((unsigned)kb128s, rbs) : dim3(rbs, (unsigned)kb128s);
-  return timed_launch(h, two ? "quantize_fp8_block2" : "quantize_fp8_block", s,
-      [&] { quantize_fp8_kernel<<<grid, 256, 0, s>>>(p); });
+QuantOperand quant_operand(const float* src, int64_t ld, int rows, int K, bool kmajor, int64_t rows_pad, int64_t kb128s,
+    u32x4* q1, u32x4* q2, int* e1, int* e2) {
+  QuantOperand o{};
+  o.src = src;
+  o.ld = ld;
+  o.rows = rows;
+  o.K = K;
+  o.kmajor = kmajor;
+  o.vec = (reinterpret_cast<uintptr_t>(src) & 15u) == 0 && ld % 4 == 0;
+  o.row_blocks = (int)(rows_pad / 128);
+  o.k_blocks = (int)kb128s;
+  o.q1 = q1;
+  o.q2 = q2;
+  o.e1 = e1;
+  o.e2 = e2;
+  return o;
 }
 
 }  // namespace
@@ -603,8 +616,15 @@ mfx_status launch_dense_fp8(Handle* h, const DenseOp& op, bool two_term, int con
     ea2 = reinterpret_cast<int*>(take(pl.e_a));
     eb2 = reinterpret_cast<int*>(take(pl.e_b));
   }
-  MFX_CHECK(quantize(h, op.A, op.lda, op.M, op.K, op.a_kmajor, pl.rows_pad_a, pl.kb128s, two_term, qa1, qa2, ea1, ea2, s));
-  MFX_CHECK(quantize(h, op.B, op.ldb, op.N, op.K, op.b_kmajor, pl.rows_pad_b, pl.kb128s, two_term, qb1, qb2, eb1, eb2, s));
+  QuantParams q;
+  q.a = quant_operand(op.A, op.lda, op.M, op.K, op.a_kmajor, pl.rows_pad_a, pl.kb128s, qa1, qa2, ea1, ea2);
+  q.b = quant_operand(op.B, op.ldb, op.N, op.K, op.b_kmajor, pl.rows_pad_b, pl.kb128s, qb1, qb2, eb1, eb2);
+  q.grid_a = q.a.row_blocks * q.a.k_blocks;
+  const int qgrid = q.grid_a + q.b.row_blocks * q.b.k_blocks;
+  MFX_CHECK(timed_launch(h, two_term ? "quantize_fp8_block2" : "quantize_fp8_block", s, [&] {
+    if(two_term) quantize_fp8_kernel<128, 2, false><<<qgrid, 1024, 0, s>>>(q);
+    else quantize_fp8_kernel<128, 1, false><<<qgrid, 1024, 0, s>>>(q);
+  }));
   const Fp8Config& c = kFp8Configs[config];
   Fp8Params p;
   p.t = Fp8TileArgs{qa1, qa2 ? qa2 : qa1, qb1, qb2 ? qb2 : qb1, ea1, ea2 ? ea2 : ea1, eb1, eb2 ? eb2 : eb1,
@@ -634,20 +654,27 @@ mfx_status launch_quantize_fp8(Handle* h, int64_t rows, int64_t cols, const floa
     uint8_t* q, int32_t* exps, hipStream_t s) {
   if(rows == 0 || cols == 0) return MFX_SUCCESS;
   QuantParams p{};
-  p.src = x;
-  p.ld = ldx;
-  p.rows = (int)rows;
-  p.K = (int)cols;
-  p.kmajor = 1;
-  p.vec = (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && ldx % 4 == 0;
-  p.kb128s = (int)ceil_div(cols, block);
-  p.two_term = 0;
-  p.e1 = exps;
-  p.plain = q;
-  p.plain_ld = cols;
-  p.block = block;
-  dim3 grid((unsigned)ceil_div(cols, block), (unsigned)ceil_div(rows, block));
-  return timed_launch(h, "quantize_fp8_block_plain", s, [&] { quantize_fp8_kernel<<<grid, 256, 0, s>>>(p); });
+  QuantOperand& o = p.a;
+  o.src = x;
+  o.ld = ldx;
+  o.rows = (int)rows;
+  o.K = (int)cols;
+  o.kmajor = 1;
+  o.vec = (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && ldx % 4 == 0;
+  o.row_blocks = (int)ceil_div(rows, block);
+  o.k_blocks = (int)ceil_div(cols, block);
+  o.e1 = exps;
+  o.plain = q;
+  o.plain_ld = cols;
+  const int64_t blocks = (int64_t)o.row_blocks * o.k_blocks;
+  if(blocks > INT32_MAX) return unsupported("quantize: more than 2^31 blocks");
+  p.grid_a = (int)blocks;
+  const unsigned grid = (unsigned)blocks;
+  return timed_launch(h, "quantize_fp8_block_plain", s, [&] {
+    if(block == 128) quantize_fp8_kernel<128, 1, true><<<grid, 1024, 0, s>>>(p);
+    else if(block == 64) quantize_fp8_kernel<64, 1, true><<<grid, 256, 0, s>>>(p);
+    else quantize_fp8_kernel<32, 1, true><<<grid, 64, 0, s>>>(p);
+  });
 }
 
 }  // namespace mfx
