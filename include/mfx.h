@@ -82,7 +82,8 @@ mfx_status mfx_device_name(mfx_handle handle, char* buf, size_t len);
 
 /* ---- dense contractions -------------------------------------------------- */
 
-/* Size of the fixed device array behind mfx_gemm_noalloc (one per device). */
+/* Packed-operand bytes of the fixed device array behind mfx_gemm_noalloc (one
+ * per device; 32 MiB for split-K partial tiles come on top). */
 #define MFX_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)
 
 /*
@@ -100,9 +101,9 @@ mfx_status mfx_gemm(mfx_handle handle, mfx_precision prec, mfx_op transA, mfx_op
 
 /*
  * mfx_gemm without any allocation: the same kernels and results as mfx_gemm
- * (FP32, SPLIT_BF16 or BF16), with the packed operands (or FP32 split-K
- * partial tiles, at most 32 MiB) in a fixed library array of
- * MFX_NOALLOC_SCRATCH_BYTES per device instead of the handle's workspace.  It calls no hipMalloc / hipFree or other allocating routine,
+ * (FP32, SPLIT_BF16 or BF16), with the packed operands (at most
+ * MFX_NOALLOC_SCRATCH_BYTES) and split-K partial tiles (at most 32 MiB) in a
+ * fixed library array per device instead of the handle's workspace.  It calls no hipMalloc / hipFree or other allocating routine,
  * so code under graph capture, tight serving loops and harnesses that
  * forbid allocation can call it.  A request whose packed operands exceed the
  * array (4 (m + n) k bytes for SPLIT_BF16, half that for BF16, about) returns

@@ -145,18 +145,13 @@ PackPlan plan(const DenseOp& op, bool split, int config, int cus, int forced_spl
   pl.split = SplitPlan{(int)pl.tiles, 1};
   pl.bytes_partial = 0;
   const int64_t steps = pl.kbs / stage * op.nprod;
-  // Partial tiles stay within kMaxPartialBytes and, where the packed operands
-  // fit the no-allocation entry point's array, within that array too, so both
-  // entry points split alike.
-  const int64_t packed = (int64_t)(pl.bytes_a + pl.bytes_b), array = (int64_t)MFX_NOALLOC_SCRATCH_BYTES;
-  const int64_t max_partial = packed <= array ? std::min(kMaxPartialBytes, array - packed) : kMaxPartialBytes;
   if(forced_splits >= 2) {
     int64_t s = std::min<int64_t>(forced_splits, steps);
-    while(s > 1 && pl.tiles * s * c.bm * c.bn * 4 > max_partial) --s;
+    while(s > 1 && pl.tiles * s * c.bm * c.bn * 4 > kMaxPartialBytes) --s;
     if(s > 1) pl.split = SplitPlan{0, (int)s};
   } else if(forced_splits < 0) {
-    plan_splits(split ? MFX_PREC_SPLIT_BF16 : MFX_PREC_BF16, config, pl.tiles, steps * stage * 16, cus, max_partial,
-        &pl.split);
+    plan_splits(split ? MFX_PREC_SPLIT_BF16 : MFX_PREC_BF16, config, pl.tiles, steps * stage * 16, cus,
+        kMaxPartialBytes, &pl.split);
   }
   if(pl.split.splits > 1)
     pl.bytes_partial = (size_t)(pl.tiles - pl.split.head) * pl.split.splits * c.bm * c.bn * sizeof(float);
@@ -212,9 +207,11 @@ bool bf_config_info(int c, bool split, int* bm, int* bn, int* bk, int* waves) {
   return true;
 }
 
-size_t dense_bf16x_workspace(const DenseOp& op, bool split, int config, int cus, int forced_splits) {
+size_t dense_bf16x_workspace(const DenseOp& op, bool split, int config, int cus, int forced_splits, size_t* partial) {
+  if(partial) *partial = 0;
   if(config < 0 || config >= kBfConfigCount) return 0;
   const PackPlan pl = plan(op, split, config, cus, forced_splits);
+  if(partial) *partial = pl.bytes_partial;
   // syrk (single operand used in both roles) still reserves two slots; the
   // second is simply unused.
   return pl.bytes_a + pl.bytes_b + pl.bytes_partial;

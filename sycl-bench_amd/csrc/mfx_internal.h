@@ -435,7 +435,9 @@ constexpr int64_t kMaxPartialBytes = (int64_t)32 << 20;
 // and the split plan behind it; partial tiles take at most max_partial bytes.
 double plan_splits(mfx_precision p, int config, int64_t tiles, int64_t k, int cus, int64_t max_partial, SplitPlan* plan);
 mfx_status launch_dense_fp8(Handle* h, const DenseOp& op, bool two_term, int config, hipStream_t s);
-size_t dense_bf16x_workspace(const DenseOp& op, bool split, int config, int cus, int forced_splits);
+// Packed operands and split-K partial tiles (*partial of them, at the end).
+size_t dense_bf16x_workspace(const DenseOp& op, bool split, int config, int cus, int forced_splits,
+    size_t* partial = nullptr);
 size_t dense_fp8_workspace(const DenseOp& op, bool two_term, int config, int cus);
 
 int config_count(mfx_precision p);

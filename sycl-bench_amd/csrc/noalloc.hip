@@ -28,7 +28,9 @@ mfx_status dispatch_dense(Handle* h, mfx_precision prec, DenseOp& op, int config
 
 namespace {
 
-static __device__ __align__(256) unsigned char scratch[MFX_NOALLOC_SCRATCH_BYTES];
+// MFX_NOALLOC_SCRATCH_BYTES for the packed operands, and room for the partial
+// tiles of any split call behind them, so a call splits exactly as mfx_gemm's.
+static __device__ __align__(256) unsigned char scratch[MFX_NOALLOC_SCRATCH_BYTES + kMaxPartialBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mutex;
@@ -97,7 +99,8 @@ mfx_status mfx_gemm_noalloc(mfx_handle handle, mfx_precision prec, mfx_op transA
     else st = launch_dense_f32_ws(h, op, cfg, ws, MFX_NOALLOC_SCRATCH_BYTES, s);
   } else {
     const bool split = prec == MFX_PREC_SPLIT_BF16;
-    const size_t need = dense_bf16x_workspace(op, split, cfg, cus_of(h), h->forced_splits);
+    size_t partial = 0;
+    const size_t need = dense_bf16x_workspace(op, split, cfg, cus_of(h), h->forced_splits, &partial) - partial;
     void* ws = scratch_of(h->device);
     if(need > MFX_NOALLOC_SCRATCH_BYTES) {
       st = unsupported("mfx_gemm_noalloc: the packed operands need " + std::to_string(need) +

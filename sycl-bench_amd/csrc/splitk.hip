@@ -82,35 +82,37 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitReduceArg
 }
 
 // Time of one tile, microseconds: `fixed` for its launch, first loads and
-// epilogue, and nanoseconds per k with few CUs busy (latency and LDS bound)
-// and with all of them busy (power, L2 and fabric shared by every CU).
-// Measured on MI355X with one tile per CU at K = 1024 and 4096.
+// epilogue, and nanoseconds per k with at most a third of the CUs busy
+// (latency and LDS bound), with all of them busy (power, L2 and fabric shared
+// by every CU) and, for tiles small enough in LDS, with two on every CU.
+// Measured on MI355X at K = 1024 and 4096.
 struct TileCost {
-  double fixed, idle, full;
+  double fixed, idle, full, twice;  // twice == 0: one tile per CU
 };
 constexpr TileCost kSplitCost[] = {
-    {6.0, 44.0, 64.0},  // 256x256, four waves
-    {5.8, 12.4, 18.0},  // 128x128, four waves
-    {4.0, 6.7, 6.8},    // 64x64
-    {7.0, 22.5, 33.0},  // 256x128, four waves
-    {6.0, 43.6, 65.0},  // 256x256, eight waves
-    {6.5, 22.6, 34.0},  // 256x128, eight waves
-    {4.9, 13.3, 19.0},  // 128x128, eight waves
+    {6.0, 44.0, 64.0, 0.0},  // 256x256, four waves
+    {5.8, 12.4, 18.0, 0.0},  // 128x128, four waves
+    {4.0, 6.7, 6.8, 13.0},   // 64x64
+    {7.0, 22.5, 33.0, 0.0},  // 256x128, four waves
+    {6.0, 43.6, 65.0, 0.0},  // 256x256, eight waves
+    {6.5, 22.6, 34.0, 0.0},  // 256x128, eight waves
+    {4.9, 13.3, 19.0, 0.0},  // 128x128, eight waves
 };
 constexpr TileCost kBf16Cost[] = {
-    {7.5, 16.0, 24.5}, {4.5, 6.2, 8.2}, {3.4, 3.87, 3.9}, {5.5, 9.7, 14.0},
-    {6.0, 15.4, 24.5}, {5.3, 9.5, 13.8}, {4.0, 6.1, 8.3},
+    {7.5, 16.0, 24.5, 0.0}, {4.5, 6.2, 8.2, 0.0},  {3.4, 3.87, 3.9, 5.5}, {5.5, 9.7, 14.0, 0.0},
+    {6.0, 15.4, 24.5, 0.0}, {5.3, 9.5, 13.8, 0.0}, {4.0, 6.1, 8.3, 0.0},
 };
 constexpr TileCost kFp8Cost[] = {
-    {16.0, 7.7, 10.8},  // 256x256, four waves
-    {6.5, 2.8, 3.5},    // 128x128
-    {10.0, 7.8, 10.9},  // 256x256, eight waves
-    {3.0, 1.6, 1.9},    // 64x64
+    {16.0, 7.7, 10.8, 0.0},  // 256x256, four waves
+    {6.5, 2.8, 3.5, 0.0},    // 128x128
+    {10.0, 7.8, 10.9, 0.0},  // 256x256, eight waves
+    {3.0, 1.6, 1.9, 2.86},   // 64x64
 };
-constexpr TileCost kFp8TwoCost[] = {{14.0, 22.5, 30.6}, {6.0, 7.7, 9.7}, {9.0, 22.7, 32.0}, {3.0, 3.9, 4.3}};
+constexpr TileCost kFp8TwoCost[] = {
+    {14.0, 22.5, 30.6, 0.0}, {6.0, 7.7, 9.7, 0.0}, {9.0, 22.7, 32.0, 0.0}, {3.0, 3.9, 4.3, 6.57}};
 
 // Reading the partials back and the launch that does it.
-constexpr double kReduceFixedUs = 4.0, kReduceBytesPerUs = 3.0e6;
+constexpr double kReduceFixedUs = 3.5, kReduceBytesPerUs = 4.0e6;
 
 bool tile_cost(mfx_precision p, int c, TileCost* out) {
   if(c < 0 || c >= config_count(p)) return false;
@@ -131,36 +133,45 @@ mfx_status launch_splitk_reduce(Handle* h, const SplitReduceArgs& a, hipStream_t
   return timed_launch(h, "splitk_reduce", s, [&] { splitk_reduce_kernel<<<(unsigned)grid, 256, 0, s>>>(a); });
 }
 
-// Whole rounds of tiles run unsplit.  The rest -- the tiles that do not fill a
-// round -- run whole or in up to 64 slices of at least two stages, whichever
-// this model makes shorter: a round costs fixed + k * (ns per k at the share of
-// CUs it keeps busy), a split adds the reduction.
+// The tiles that do not fill a round of the CUs -- all of them, or those past
+// the whole rounds -- run whole or in up to 64 slices of at least two stages,
+// whichever this model makes shorter: `count` workgroups of `len` k each cost
+// fixed + len * (ns per k at the load they put on the CUs) per round, and a
+// split adds the reduction.
 double plan_splits(mfx_precision p, int config, int64_t tiles, int64_t k, int cus, int64_t max_partial,
     SplitPlan* plan) {
   TileCost tc;
   int bm, bn, bk, w;
   if(plan) *plan = SplitPlan{(int)tiles, 1};
   if(!tile_cost(p, config, &tc) || !config_info(p, config, &bm, &bn, &bk, &w) || tiles <= 0) return 0.0;
-  auto per_k = [&](double busy) {  // us per k
-    const double x = std::max(0.0, (std::min(1.0, busy) - 0.5) / 0.5);
-    return 1e-3 * (tc.idle + (tc.full - tc.idle) * x);
+  const int64_t slots = tc.twice > 0.0 ? 2 * (int64_t)cus : cus;
+  auto span = [&](int64_t count, double len) {
+    const int64_t rounds = count / slots, rest = count - rounds * slots;
+    auto round = [&](double load) {  // load: workgroups per CU
+      const double ns = load > 1.0 ? tc.full + (tc.twice - tc.full) * (load - 1.0)
+                                   : tc.idle + (tc.full - tc.idle) * std::max(0.0, (load - 0.33) / 0.67);
+      return tc.fixed + 1e-3 * ns * len;
+    };
+    return (double)rounds * round((double)slots / cus) + (rest ? round((double)rest / cus) : 0.0);
   };
-  const int64_t rounds = tiles / cus, rest = tiles - rounds * cus, steps = ceil_div(k, bk);
-  const double head = (double)rounds * (tc.fixed + (double)k * per_k(1.0));
-  if(rest == 0) return head;
-  double best = head + tc.fixed + (double)k * per_k((double)rest / cus);
+  double best = span(tiles, (double)k);
+  const int64_t steps = ceil_div(k, bk);
   const double tile_bytes = 4.0 * bm * bn;
-  for(int64_t s = 2; s <= 64 && 2 * s <= steps; ++s) {
-    const double bytes = (double)(rest * s) * tile_bytes;
-    if(bytes > (double)max_partial) break;
-    const int64_t slice_rounds = ceil_div(rest * s, cus);
-    const double t = head + (double)slice_rounds * (tc.fixed + (double)(ceil_div(steps, s) * bk) * per_k((double)(rest * s) / cus)) +
-                     kReduceFixedUs + bytes / kReduceBytesPerUs;
-    if(t < best * 0.97) {  // a split has to be clearly ahead
-      best = t;
-      if(plan) *plan = SplitPlan{(int)(rounds * cus), (int)s};
+  auto try_split = [&](int64_t head) {
+    const int64_t rest = tiles - head;
+    const double whole = head ? span(head, (double)k) : 0.0;
+    for(int64_t s = 2; s <= 64 && 2 * s <= steps && whole < best; ++s) {
+      const double bytes = (double)(rest * s) * tile_bytes;
+      if(bytes > (double)max_partial) break;
+      const double t = whole + span(rest * s, (double)(ceil_div(steps, s) * bk)) + kReduceFixedUs + bytes / kReduceBytesPerUs;
+      if(t < best * 0.98) {  // a split has to be clearly ahead
+        best = t;
+        if(plan) *plan = SplitPlan{(int)head, (int)s};
+      }
     }
-  }
+  };
+  if(tiles % cus) try_split(tiles / cus * cus);
+  if(tiles > cus && tiles < 3 * cus) try_split(0);
   return best;
 }
 

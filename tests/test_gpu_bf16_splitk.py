@@ -105,13 +105,13 @@ def test_triangles(handle, prec, uplo, mirror, n, k, config):
 
 @pytest.mark.parametrize("prec", ["split-bf16", "bf16"])
 def test_whole_rounds_and_a_split_rest(handle, prec):
-    """One round of whole 64x64 tiles and a few tiles beyond it, which split."""
+    """One round of whole 128x128 tiles (one per CU) and a few tiles beyond it, which split."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    m, n, k = 64 * 8, 64 * (cus // 8 + 1) - 3, 2048
+    m, n, k = 128 * 8, 128 * (cus // 8 + 1) - 3, 2048
     print(f"whole round + rest {prec} {m}x{n}x{k}", flush=True)
     A, B, C0 = seeded(handle, m, k, 0), seeded(handle, k, n, 1), seeded(handle, m, n, 2)
     C = C0.clone()
-    handle.force_config(prec, 2)
+    handle.force_config(prec, 6)
     try:
         rec = recorded(handle, lambda: handle.gemm(A, B, C, alpha=1.5, beta=0.5, prec=prec))
     finally:
