@@ -327,8 +327,7 @@ __device__ __forceinline__ void fp8_tile(const Fp8TileArgs& t, int tm, int tn, i
   constexpr int SLOT = NT;                                                // ints of one buffer
   int kb_next = s0, slot_next = 0;
   auto issue_scales = [&]() __attribute__((always_inline)) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(escale + kb_next),
-        (__attribute__((address_space(3))) void*)(slots + slot_next * SLOT), 4, 0, 0);
+    lds_dma4(escale + kb_next, slots + slot_next * SLOT);
   };
   struct Scales {
     int a1, b1, a2, b2;  // biased: E8M0 bytes

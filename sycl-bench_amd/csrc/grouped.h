@@ -112,15 +112,15 @@ struct GroupedArgs {
 
 // Tile geometry of configuration C (the same ids as the single-problem
 // kernels): BM x BN per workgroup, WM x WN per wave (four waves for 0-3,
-// eight, two per SIMD, for 4-6); BK is the FP32 k-step.
+// eight, two per SIMD, for 4-6).
 template <int C> struct Geo;
-template <> struct Geo<0> { static constexpr int BM = 256, BN = 256, WM = 128, WN = 128, BK = 16; };
-template <> struct Geo<1> { static constexpr int BM = 128, BN = 128, WM = 64, WN = 64, BK = 16; };
-template <> struct Geo<2> { static constexpr int BM = 64, BN = 64, WM = 32, WN = 32, BK = 32; };
-template <> struct Geo<3> { static constexpr int BM = 256, BN = 128, WM = 128, WN = 64, BK = 16; };
-template <> struct Geo<4> { static constexpr int BM = 256, BN = 256, WM = 128, WN = 64, BK = 16; };
-template <> struct Geo<5> { static constexpr int BM = 256, BN = 128, WM = 64, WN = 64, BK = 16; };
-template <> struct Geo<6> { static constexpr int BM = 128, BN = 128, WM = 64, WN = 32, BK = 16; };
+template <> struct Geo<0> { static constexpr int BM = 256, BN = 256, WM = 128, WN = 128; };
+template <> struct Geo<1> { static constexpr int BM = 128, BN = 128, WM = 64, WN = 64; };
+template <> struct Geo<2> { static constexpr int BM = 64, BN = 64, WM = 32, WN = 32; };
+template <> struct Geo<3> { static constexpr int BM = 256, BN = 128, WM = 128, WN = 64; };
+template <> struct Geo<4> { static constexpr int BM = 256, BN = 256, WM = 128, WN = 64; };
+template <> struct Geo<5> { static constexpr int BM = 256, BN = 128, WM = 64, WN = 64; };
+template <> struct Geo<6> { static constexpr int BM = 128, BN = 128, WM = 64, WN = 32; };
 // threads of a workgroup running configuration C
 template <int C>
 constexpr int geo_threads() {

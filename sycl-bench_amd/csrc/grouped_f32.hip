@@ -9,24 +9,25 @@ namespace {
 
 template <int C, bool VEC>
 __device__ __forceinline__ void run_tile(const DenseOp& op, const GProblem& P, int tm, int tn, float* smem) {
-  constexpr int BM = Geo<C>::BM, BN = Geo<C>::BN, BK = Geo<C>::BK, WM = Geo<C>::WM, WN = Geo<C>::WN;
-  if(P.a_kmajor && !P.b_kmajor) f32_tile<BM, BN, BK, WM, WN, true, false, VEC>(op, tm, tn, smem);
-  else if(P.a_kmajor) f32_tile<BM, BN, BK, WM, WN, true, true, VEC>(op, tm, tn, smem);
-  else if(!P.b_kmajor) f32_tile<BM, BN, BK, WM, WN, false, false, VEC>(op, tm, tn, smem);
-  else f32_tile<BM, BN, BK, WM, WN, false, true, VEC>(op, tm, tn, smem);
+  constexpr int BM = Geo<C>::BM, BN = Geo<C>::BN, WM = Geo<C>::WM, WN = Geo<C>::WN;
+  const int steps = (op.K + F32_BK - 1) / F32_BK, er = tm * BM, ec = tn * BN;
+  if(P.a_kmajor && !P.b_kmajor) f32_tile<BM, BN, WM, WN, true, false, VEC>(op, tm, tn, 0, steps, op.ep, er, ec, smem);
+  else if(P.a_kmajor) f32_tile<BM, BN, WM, WN, true, true, VEC>(op, tm, tn, 0, steps, op.ep, er, ec, smem);
+  else if(!P.b_kmajor) f32_tile<BM, BN, WM, WN, false, false, VEC>(op, tm, tn, 0, steps, op.ep, er, ec, smem);
+  else f32_tile<BM, BN, WM, WN, false, true, VEC>(op, tm, tn, 0, steps, op.ep, er, ec, smem);
 }
 
-template <int C>
+template <int C, bool VEC>
 constexpr int f32_smem_floats() {
-  return F32Cfg<Geo<C>::BM, Geo<C>::BN, Geo<C>::BK, Geo<C>::WM, Geo<C>::WN>::SMEM_FLOATS;
+  return F32Cfg<Geo<C>::BM, Geo<C>::BN, Geo<C>::WM, Geo<C>::WN, VEC>::SMEM_FLOATS;
 }
 
 // VEC: every problem of the launch allows 128-bit operand loads.
 template <int BIG, int SMALL, bool VEC>
 __global__ __launch_bounds__(geo_threads<BIG>()) void grouped_f32_kernel(const GroupedArgs g) {
   static_assert(geo_threads<SMALL>() == geo_threads<BIG>(), "both tiles of a policy use the same workgroup");
-  constexpr int S0 = f32_smem_floats<BIG>(), S1 = f32_smem_floats<SMALL>();
-  __shared__ float smem[S0 > S1 ? S0 : S1];
+  constexpr int S0 = f32_smem_floats<BIG, VEC>(), S1 = f32_smem_floats<SMALL, VEC>();
+  __shared__ __align__(16) float smem[S0 > S1 ? S0 : S1];
   __shared__ int slot, ready, tried;
   if(threadIdx.x == 0) tried = 0;
   for(;;) {

@@ -156,92 +156,22 @@ double config_rate(mfx_precision p, int c) {
   return c >= 0 && c < n ? t[c] : 0.5;
 }
 
-// Heuristic used when nothing is tuned: the configuration with the least
-// estimated time, counted in rounds of tiles over the CUs (a round costs the
-// tile's area over its rate), so a last round that leaves most CUs idle is
-// paid for.  `tiles(bm, bn)` gives the tile count of the schedule (the full
-// grid, or a triangle).  Ties go to the larger tile, then more waves.
-// Exception for the power-limited BF16 / FP8 MFMAs: when the largest tile
-// fills between half and all of the CUs in one round, it is taken (the clock
-// rises as CUs idle, which the round count does not see; measured on MI355X,
-// e.g. a 4096 split-BF16 syrk: 136 large tiles beat 528 small ones by 10 %).
-template <class Tiles>
-int least_time_config(Handle* h, mfx_precision p, bool square_only, Tiles&& tiles) {
-  const int cus = h->cu_count > 0 ? h->cu_count : 256;
-  if(p != MFX_PREC_FP32) {
-    int big = -1, big_w = 0;
-    int64_t big_area = 0;
-    for(int c = 0; c < config_count(p); ++c) {
-      int bm, bn, bk, w;
-      if(!config_info(p, c, &bm, &bn, &bk, &w) || (square_only && bm != bn)) continue;
-      const int64_t area = (int64_t)bm * bn;
-      if(area > big_area || (area == big_area && w > big_w)) {
-        big = c;
-        big_area = area;
-        big_w = w;
-      }
-    }
-    if(big >= 0) {
-      int bm, bn, bk, w;
-      config_info(p, big, &bm, &bn, &bk, &w);
-      const int64_t t = tiles(bm, bn);
-      if(2 * t >= cus && t <= cus) return big;
-    }
-  }
-  int best = -1;
-  double best_t = 0.0;
-  int64_t best_area = 0;
-  int best_waves = 0;
-  for(int c = 0; c < config_count(p); ++c) {
-    int bm, bn, bk, w;
-    if(!config_info(p, c, &bm, &bn, &bk, &w) || (square_only && bm != bn)) continue;
-    const int64_t area = (int64_t)bm * bn;
-    const double t = (double)ceil_div(tiles(bm, bn), cus) * (double)area / config_rate(p, c);
-    const bool better = best < 0 || t < best_t * (1.0 - 1e-9) ||
-                        (t <= best_t * (1.0 + 1e-9) && (area > best_area || (area == best_area && w > best_waves)));
-    if(better) {
-      best = c;
-      best_t = t;
-      best_area = area;
-      best_waves = w;
-    }
-  }
-  return best < 0 ? 0 : best;
-}
-
-// The configuration whose estimated launch, split-K included, is shortest
-// (plan_splits; every precision but FP32).  `tiles(bm, bn)` as above.
-template <class Tiles>
-int least_cost_config(Handle* h, mfx_precision p, int64_t k, bool square_only, Tiles&& tiles) {
+// Used when nothing is tuned: the configuration whose estimated launch
+// (tile_span's measured model, with the k slices plan_splits or the smaller
+// tiles tri_tail would give a sparse last round) is shortest.
+int heuristic_config(Handle* h, mfx_precision p, int64_t m, int64_t n, int64_t k) {
   int best = 0;
   double best_t = -1.0;
   for(int c = 0; c < config_count(p); ++c) {
     int bm, bn, bk, w;
-    if(!config_info(p, c, &bm, &bn, &bk, &w) || (square_only && bm != bn)) continue;
-    const double t = plan_splits(p, c, tiles(bm, bn), k, cus_of(h), kMaxPartialBytes, nullptr);
+    if(!config_info(p, c, &bm, &bn, &bk, &w)) continue;
+    const double t = plan_splits(p, c, ceil_div(m, bm) * ceil_div(n, bn), k, cus_of(h), kMaxPartialBytes, nullptr);
     if(best_t < 0.0 || t < best_t) {
       best = c;
       best_t = t;
     }
   }
   return best;
-}
-
-bool has_cost_model(mfx_precision p) { return p != MFX_PREC_FP32; }
-
-// FP32 configuration with sixteen waves on a 64x64 tile (four k-groups).
-constexpr int kF32KGroupConfig = 7;
-
-int heuristic_config(Handle* h, mfx_precision p, int64_t m, int64_t n, int64_t k) {
-  auto grid = [&](int bm, int bn) { return ceil_div(m, bm) * ceil_div(n, bn); };
-  if(has_cost_model(p)) return least_cost_config(h, p, k, false, grid);
-  // FP32 grids of at most one 64x64 tile per CU: the k-grouped tile (one
-  // sixteen-wave workgroup per CU hides load latency that four-wave tiles
-  // leave exposed at this size; split-K then fills the CUs if tiles are
-  // few).  Measured on MI355X: 1024^3 in 27-30 us against 32-36 us.
-  const int cus = h->cu_count > 0 ? h->cu_count : 256;
-  if(p == MFX_PREC_FP32 && ceil_div(m, 64) * ceil_div(n, 64) <= cus) return kF32KGroupConfig;
-  return least_time_config(h, p, false, grid);
 }
 
 int choose_config(Handle* h, mfx_precision p, int64_t m, int64_t n, int64_t k) {
@@ -292,68 +222,32 @@ TriTail tri_tail(mfx_precision p, int config, int64_t T, int cus) {
   return t;
 }
 
-// Least estimated time over the square configurations for an n x n
-// triangle: rounds of T(T+1)/2 tiles over the CUs, each costing the tile's
-// area over its rate, with a sparse last round re-tiled as tri_tail does.
-// BF16 / FP8 take their largest tile when it fills between half and all of
-// the CUs in one round (the power-limited clock rises as CUs idle; see
-// least_time_config).
-static int least_time_triangle(Handle* h, mfx_precision p, int64_t n) {
-  const int cus = h->cu_count > 0 ? h->cu_count : 256;
-  auto tri = [&](int b) {
-    const int64_t t = ceil_div(n, b);
-    return t * (t + 1) / 2;
-  };
-  int best = -1, best_w = 0;
-  double best_t = 0.0;
-  int64_t best_area = 0;
-  if(p != MFX_PREC_FP32) {
-    for(int c = 0; c < config_count(p); ++c) {
-      int bm, bn, bk, w;
-      if(!config_info(p, c, &bm, &bn, &bk, &w) || bm != bn) continue;
-      if((int64_t)bm * bn > best_area || ((int64_t)bm * bn == best_area && w > best_w)) {
-        best = c;
-        best_area = (int64_t)bm * bn;
-        best_w = w;
-      }
-    }
-    if(best >= 0) {
-      int bm, bn, bk, w;
-      config_info(p, best, &bm, &bn, &bk, &w);
-      const int64_t t = tri(bm);
-      if(2 * t >= cus && t <= cus) return best;
-    }
-    best = -1;
-    best_area = 0;
-    best_w = 0;
-  }
+// The same over the square configurations for an n x n triangle.
+static int heuristic_square_config(Handle* h, mfx_precision p, int64_t n, int64_t k) {
+  const int cus = cus_of(h);
+  int best = 0;
+  double best_t = -1.0;
   for(int c = 0; c < config_count(p); ++c) {
     int bm, bn, bk, w;
     if(!config_info(p, c, &bm, &bn, &bk, &w) || bm != bn) continue;
-    const int64_t T = ceil_div(n, bm), tiles = tri(bm), area = (int64_t)bm * bn;
-    const TriTail tt = tri_tail(p, c, T, cus);
-    double t;
-    if(tt.small >= 0) {
-      const int sb = bm / tt.ratio;
-      t = (double)(tiles / cus) * area / config_rate(p, c) +
-          (double)ceil_div((tiles - tt.head) * tt.ratio * tt.ratio, cus) * sb * sb / config_rate(p, tt.small);
-    } else {
-      t = (double)ceil_div(tiles, cus) * area / config_rate(p, c);
+    const int64_t T = ceil_div(n, bm), tiles = T * (T + 1) / 2;
+    double t = plan_splits(p, c, tiles, k, cus, kMaxPartialBytes, nullptr);
+    if(p == MFX_PREC_FP32) {
+      const TriTail tail = tri_tail(p, c, T, cus);
+      if(tail.small >= 0)
+        t = std::min(t, tile_span(p, c, tail.head, (double)k, cus) +
+                            tile_span(p, tail.small, (tiles - tail.head) * tail.ratio * tail.ratio, (double)k, cus));
     }
-    const bool better = best < 0 || t < best_t * (1.0 - 1e-9) ||
-                        (t <= best_t * (1.0 + 1e-9) && (area > best_area || (area == best_area && w > best_w)));
-    if(better) {
+    if(best_t < 0.0 || t < best_t) {
       best = c;
       best_t = t;
-      best_area = area;
-      best_w = w;
     }
   }
-  return best < 0 ? 0 : best;
+  return best;
 }
 
 // Square-tile choice for the triangular schedules: a forced or tuned square
-// configuration, else least_time_triangle.
+// configuration, else the estimate.
 int choose_square_config(Handle* h, mfx_precision p, int64_t n, int64_t k) {
   int c = -1;
   if(h->forced_config[p] >= 0) {
@@ -365,9 +259,7 @@ int choose_square_config(Handle* h, mfx_precision p, int64_t n, int64_t k) {
   }
   int bm, bn, bk, w;
   if(c >= 0) return config_info(p, c, &bm, &bn, &bk, &w) && bm == bn ? c : 0;
-  if(has_cost_model(p))
-    return least_cost_config(h, p, k, true, [&](int b, int) { return ceil_div(n, b) * (ceil_div(n, b) + 1) / 2; });
-  return least_time_triangle(h, p, n);
+  return heuristic_square_config(h, p, n, k);
 }
 
 mfx_status dispatch_dense(Handle* h, mfx_precision prec, DenseOp& op, int config, hipStream_t s) {
@@ -537,11 +429,7 @@ size_t mfx_gemm_workspace_size(mfx_precision prec, int64_t m, int64_t n, int64_t
   for(int c = 0; c < config_count(prec); ++c) {
     size_t b = 0;
     if(prec == MFX_PREC_FP32) {
-      int bm, bn, bk, w;
-      config_info(prec, c, &bm, &bn, &bk, &w);
-      const int64_t tiles = ceil_div(m, bm) * ceil_div(n, bn);
-      const int splits = f32_splits(c, tiles, k, cus);
-      if(splits > 1) b = f32_splitk_workspace(c, tiles, splits);
+      b = dense_f32_workspace(op, c, cus, -1);
     } else if(prec == MFX_PREC_SPLIT_BF16 || prec == MFX_PREC_BF16)
       b = dense_bf16x_workspace(op, prec == MFX_PREC_SPLIT_BF16, c, cus, -1);
     else if(prec == MFX_PREC_FP8_BLOCK || prec == MFX_PREC_FP8_BLOCK2)

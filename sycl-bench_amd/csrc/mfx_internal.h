@@ -320,6 +320,14 @@ __device__ __forceinline__ void lds_dma16(const T* src, T* lds_wave_base) {
       (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
 
+// The same with one 4-byte value per lane (global_load_lds_dword).
+template <class T>
+__device__ __forceinline__ void lds_dma4(const T* src, T* lds_wave_base) {
+  static_assert(sizeof(T) == 4, "one 4-byte value per lane");
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+      (__attribute__((address_space(3))) void*)lds_wave_base, 4, 0, 0);
+}
+
 // Waits for this wave's outstanding memory operations, LDS transfers included.
 __device__ __forceinline__ void lds_dma_wait() { __builtin_amdgcn_s_waitcnt(0); }
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -412,11 +420,7 @@ mfx_status launch_dense_f32(Handle* h, const DenseOp& op, int config, hipStream_
 // The same with split-K partial tiles in `ws` (ws_bytes long) instead of the
 // handle's workspace; fails if a split this call makes needs more.
 mfx_status launch_dense_f32_ws(Handle* h, const DenseOp& op, int config, void* ws, size_t ws_bytes, hipStream_t s);
-// FP32 split-K pieces (gemm_f32.hip): k slices per tile for a configuration
-// (1: none), the partial buffer's size, and the launch on given buffers.
-int f32_splits(int config, int64_t tiles, int64_t K, int cus);
-size_t f32_splitk_workspace(int config, int64_t tiles, int splits);
-mfx_status launch_f32_splitk(Handle* h, const DenseOp& op, int config, int splits, float* partial, hipStream_t s);
+size_t dense_f32_workspace(const DenseOp& op, int config, int cus, int forced_splits);
 mfx_status launch_dense_bf16x(Handle* h, const DenseOp& op, bool split, int config, hipStream_t s);
 // The same on a caller-provided workspace of dense_bf16x_workspace() bytes.
 mfx_status launch_dense_bf16x_ws(Handle* h, const DenseOp& op, bool split, int config, void* ws, hipStream_t s);
@@ -433,6 +437,8 @@ mfx_status launch_splitk_reduce(Handle* h, const SplitReduceArgs& a, hipStream_t
 constexpr int64_t kMaxPartialBytes = (int64_t)32 << 20;
 // Estimated microseconds of a dense launch on `config` (tile_cost's model)
 // and the split plan behind it; partial tiles take at most max_partial bytes.
+// Estimated microseconds of `count` workgroups of `len` k each (no split).
+double tile_span(mfx_precision p, int config, int64_t count, double len, int cus);
 double plan_splits(mfx_precision p, int config, int64_t tiles, int64_t k, int cus, int64_t max_partial, SplitPlan* plan);
 mfx_status launch_dense_fp8(Handle* h, const DenseOp& op, bool two_term, int config, hipStream_t s);
 // Packed operands and split-K partial tiles (*partial of them, at the end).

@@ -89,6 +89,16 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitReduceArg
 struct TileCost {
   double fixed, idle, full, twice;  // twice == 0: one tile per CU
 };
+constexpr TileCost kF32Cost[] = {
+    {25.0, 231.0, 228.0, 0.0},  // 256x256, four waves
+    {8.0, 65.0, 64.0, 122.0},   // 128x128, four waves
+    {8.0, 20.3, 21.1, 35.0},    // 64x64 in many short slices by a rule of its own: priced out of the choice
+    {18.0, 120.0, 115.0, 0.0},  // 256x128, four waves
+    {25.0, 226.0, 220.0, 0.0},  // 256x256, eight waves
+    {18.0, 116.0, 112.0, 0.0},  // 256x128, eight waves
+    {8.0, 59.4, 62.0, 123.0},   // 128x128, eight waves
+    {4.0, 16.4, 18.2, 34.5},    // 64x64, two k-groups
+};
 constexpr TileCost kSplitCost[] = {
     {6.0, 44.0, 64.0, 0.0},  // 256x256, four waves
     {5.8, 12.4, 18.0, 0.0},  // 128x128, four waves
@@ -111,12 +121,15 @@ constexpr TileCost kFp8Cost[] = {
 constexpr TileCost kFp8TwoCost[] = {
     {14.0, 22.5, 30.6, 0.0}, {6.0, 7.7, 9.7, 0.0}, {9.0, 22.7, 32.0, 0.0}, {3.0, 3.9, 4.3, 6.57}};
 
-// Reading the partials back and the launch that does it.
-constexpr double kReduceFixedUs = 3.5, kReduceBytesPerUs = 4.0e6;
+// Reading the partials back and the launch that does it.  Below kSplitFromUs
+// a call is bound by its launches on the host (about 10 us for the first, 3.5
+// for each further one, from Python), which a split adds to.
+constexpr double kReduceFixedUs = 3.5, kReduceBytesPerUs = 4.0e6, kSplitFromUs = 11.0;
 
 bool tile_cost(mfx_precision p, int c, TileCost* out) {
   if(c < 0 || c >= config_count(p)) return false;
   switch(p) {
+    case MFX_PREC_FP32: *out = kF32Cost[c]; return true;
     case MFX_PREC_SPLIT_BF16: *out = kSplitCost[c]; return true;
     case MFX_PREC_BF16: *out = kBf16Cost[c]; return true;
     case MFX_PREC_FP8_BLOCK: *out = kFp8Cost[c]; return true;
@@ -133,34 +146,39 @@ mfx_status launch_splitk_reduce(Handle* h, const SplitReduceArgs& a, hipStream_t
   return timed_launch(h, "splitk_reduce", s, [&] { splitk_reduce_kernel<<<(unsigned)grid, 256, 0, s>>>(a); });
 }
 
+// `count` workgroups of `len` k each cost fixed + len * (ns per k at the load
+// they put on the CUs) per round.
+double tile_span(mfx_precision p, int config, int64_t count, double len, int cus) {
+  TileCost tc;
+  if(count <= 0 || !tile_cost(p, config, &tc)) return 0.0;
+  const int64_t slots = tc.twice > 0.0 ? 2 * (int64_t)cus : cus;
+  const int64_t rounds = count / slots, rest = count - rounds * slots;
+  auto round = [&](double load) {  // load: workgroups per CU
+    const double ns = load > 1.0 ? tc.twice  // the CUs that got two set the pace
+                                 : tc.idle + (tc.full - tc.idle) * std::max(0.0, (load - 0.33) / 0.67);
+    return tc.fixed + 1e-3 * ns * len;
+  };
+  return (double)rounds * round((double)slots / cus) + (rest ? round((double)rest / cus) : 0.0);
+}
+
 // The tiles that do not fill a round of the CUs -- all of them, or those past
 // the whole rounds -- run whole or in up to 64 slices of at least two stages,
-// whichever this model makes shorter: `count` workgroups of `len` k each cost
-// fixed + len * (ns per k at the load they put on the CUs) per round, and a
-// split adds the reduction.
+// whichever this model makes shorter: tile_span, and for a split the
+// reduction.
 double plan_splits(mfx_precision p, int config, int64_t tiles, int64_t k, int cus, int64_t max_partial,
     SplitPlan* plan) {
-  TileCost tc;
   int bm, bn, bk, w;
   if(plan) *plan = SplitPlan{(int)tiles, 1};
-  if(!tile_cost(p, config, &tc) || !config_info(p, config, &bm, &bn, &bk, &w) || tiles <= 0) return 0.0;
-  const int64_t slots = tc.twice > 0.0 ? 2 * (int64_t)cus : cus;
-  auto span = [&](int64_t count, double len) {
-    const int64_t rounds = count / slots, rest = count - rounds * slots;
-    auto round = [&](double load) {  // load: workgroups per CU
-      const double ns = load > 1.0 ? tc.full + (tc.twice - tc.full) * (load - 1.0)
-                                   : tc.idle + (tc.full - tc.idle) * std::max(0.0, (load - 0.33) / 0.67);
-      return tc.fixed + 1e-3 * ns * len;
-    };
-    return (double)rounds * round((double)slots / cus) + (rest ? round((double)rest / cus) : 0.0);
-  };
+  if(!config_info(p, config, &bm, &bn, &bk, &w) || tiles <= 0) return 0.0;
+  auto span = [&](int64_t count, double len) { return tile_span(p, config, count, len, cus); };
   double best = span(tiles, (double)k);
   const int64_t steps = ceil_div(k, bk);
   const double tile_bytes = 4.0 * bm * bn;
   auto try_split = [&](int64_t head) {
     const int64_t rest = tiles - head;
     const double whole = head ? span(head, (double)k) : 0.0;
-    for(int64_t s = 2; s <= 64 && 2 * s <= steps && whole < best; ++s) {
+    // few, widening candidates: this runs in every call
+    for(int64_t s = 2; s <= 64 && 2 * s <= steps && whole < best; s += s < 8 ? 1 : s / 4) {
       const double bytes = (double)(rest * s) * tile_bytes;
       if(bytes > (double)max_partial) break;
       const double t = whole + span(rest * s, (double)(ceil_div(steps, s) * bk)) + kReduceFixedUs + bytes / kReduceBytesPerUs;
@@ -170,6 +188,7 @@ double plan_splits(mfx_precision p, int config, int64_t tiles, int64_t k, int cu
       }
     }
   };
+  if(best < kSplitFromUs) return best;
   if(tiles % cus) try_split(tiles / cus * cus);
   if(tiles > cus && tiles < 3 * cus) try_split(0);
   return best;

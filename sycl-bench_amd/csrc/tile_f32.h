@@ -1,297 +1,309 @@
 // One BM x BN output tile of an FP32 contraction on v_mfma_f32_32x32x2_f32,
-// shared by the single-problem kernel (gemm_f32.hip) and the persistent
-// grouped kernel (grouped.hip).
+// shared by the single-problem kernels (gemm_f32.hip) and the persistent
+// grouped kernel (grouped_f32.hip).
 //
-// A workgroup of KG groups of (BM/WM) x (BN/WN) waves; each wave owns a
-// WM x WN sub-tile held as (WM/32) x (WN/32) 32x32 accumulator blocks.  With
-// KG > 1 every group computes the whole tile over its own 1/KG of each staged
-// k block (more waves per CU for tiles that would otherwise leave the SIMDs
-// waiting on loads), and the groups' accumulators are summed through LDS at
-// the end, group 0 first, before group 0 writes the tile.  A and B panels of BK
-// k-steps are staged in LDS with double buffering: the global loads of step
-// s+1 are issued before the MFMAs of step s and land in the other LDS buffer
-// afterwards, so one barrier per step suffices.  LDS holds both panels
-// k-major (As[k][m], Bs[k][n]) whatever the global layout, padded by 4 floats
-// per row so the transposing stores of k-contiguous operands hit distinct
-// banks.
+// A workgroup of (BM/WM) x (BN/WN) waves; each wave owns a WM x WN sub-tile
+// held as (WM/32) x (WN/32) 32x32 accumulator blocks.  The operands go from
+// global memory straight into LDS, 16 k of both panels per stage, several
+// stages in flight, in a layout the DMA writes as it is and the MFMAs read as
+// it is.  One 32-row block of an operand and stage is 512 floats:
+//   k-contiguous operand (element (r, k) at p[r*ld + k]): 128 chunks of four
+//     floats; chunk h*64 + l holds row l%32, k = 8*(l/32) + 4h .. +3;
+//   row-contiguous operand (element (r, k) at p[k*ld + r]): a 16 x 32 (k x r)
+//     array.
+// Lane l feeds row l%32 to the MFMA and supplies k slot l/32 of its two, so
+// half stage h, step e contracts k = 4h + e and 8 + 4h + e: any pairing of
+// the k's is the same sum, and this one makes a lane's values of a half stage
+// one 16-byte LDS read.
 #pragma once
 
-#include "mfx_internal.h"
+#include "lds_pipe.h"
 
 namespace mfx {
 
-template <int BM, int BN, int BK, int WM, int WN, int KG = 1>
+constexpr int F32_BK = 16;  // k per stage and k-group
+
+// Stages buffered: four, eight of the 64x64 tile (whose stage is 512 cycles of
+// MFMA per wave).
+template <int BM, int BN>
+constexpr int f32_stages() {
+  return BM * BN <= 64 * 64 ? 8 : 4;
+}
+
+// VEC: 16-byte copies into LDS, else 4-byte ones (four times as many).
+// WANT: stages to buffer, as far as their copies fit vmcnt.
+// KG: groups of waves that each contract the whole tile over their own 16 k of
+// every KG * 16 deep stage (two waves per SIMD on a tile of four sub-tiles:
+// one issues MFMAs while the other is at the barrier); their accumulators are
+// summed through LDS at the end.
+template <int BM, int BN, int WM, int WN, bool VEC, int WANT = f32_stages<BM, BN>(), int KG = 1>
 struct F32Cfg {
   static constexpr int NWM = BM / WM, NWN = BN / WN, NWG = NWM * NWN, NW = NWG * KG, NT = NW * 64;
   static constexpr int FM = WM / 32, FN = WN / 32;
-  static constexpr int LDSA = BM + 4, LDSB = BN + 4;
-  static constexpr int PANELS = 2 * BK * (LDSA + LDSB);
-  static constexpr int REDUCE = (KG - 1) * BM * BN;  // accumulators of groups 1..KG-1
-  static constexpr int SMEM_FLOATS = PANELS > REDUCE ? PANELS : REDUCE;
-  static_assert(BK % (2 * KG) == 0, "each k-group takes whole MFMA k-steps of a stage");
+  static constexpr int BK = F32_BK * KG;
+  static constexpr int FL_A = BM * BK, FL_B = BN * BK, STAGE = FL_A + FL_B;  // floats per stage
+  static constexpr int W = VEC ? 4 : 1;                                              // floats per lane and copy
+  static constexpr int PER_A = FL_A / (NT * W), PER_B = FL_B / (NT * W), PER = PER_A + PER_B;
+  static constexpr int NB = WANT < 63 / PER + 1 ? WANT : 63 / PER + 1;
+  static constexpr int SMEM_FLOATS = NB * STAGE;
+  static_assert(FL_A % (NT * W) == 0 && FL_B % (NT * W) == 0, "stage must split evenly over threads");
+  static_assert(NB >= 2 && (NB - 1) * PER < 64, "in-flight copies fit vmcnt");
+  static_assert((KG - 1) * BM * BN <= NB * STAGE, "the other groups' accumulators fit the stages");
 };
 
-// Loads the BK x ROWS panel of an operand starting at (row0, k0) into
-// registers.  kmajor: element (r, k) at P[r*ld + k]; else P[k*ld + r].
-// DEFER (128-bit loads only): load without a branch and zero the chunks
-// outside the matrix at the LDS store instead (for two prefetch sets).
-template <int ROWS, int BK, int NT, bool KMAJOR, bool DEFER = false>
-struct PanelLoader {
-  static constexpr int NV = ROWS * BK / 4;  // float4 chunks
-  static constexpr int PER = NV / NT;
-  static_assert(NV % NT == 0, "panel must split evenly over threads");
-  static_assert(PER <= 32, "in-bounds flags are one bit per chunk");
-  float4 v[PER];
-  uint32_t in = 0;  // VEC and DEFER: bit i set when chunk i lies inside the matrix
-
-  // VEC: 128-bit loads (compile-time, so the steady-state loop has no
-  // per-load branches); otherwise four bounds-checked scalar loads.
-  template <bool VEC>
-  __device__ __forceinline__ void load(const float* P, int64_t ld, int rows, int K, int row0, int k0, int tid) {
-#pragma unroll
-    for(int i = 0; i < PER; ++i) {
-      const int idx = tid + i * NT;
-      int r, k;
-      if(KMAJOR) {
-        r = idx / (BK / 4);
-        k = (idx % (BK / 4)) * 4;
-      } else {
-        k = idx / (ROWS / 4);
-        r = (idx % (ROWS / 4)) * 4;
-      }
-      const int gr = row0 + r, gk = k0 + k;
-      float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-      if constexpr(VEC && DEFER) {
-        // Unconditional load from the nearest in-bounds chunk (rows >= 1 for
-        // any scheduled tile, and the contiguous extent is a positive
-        // multiple of 4 whenever a stage is issued); store() zeroes the
-        // chunks outside the matrix.  With no branch around the load and its
-        // value first used at the LDS store, the compiler can wait for one
-        // prefetch set while a later one is still in flight.
-        if(i == 0) in = 0;
-        in |= (uint32_t)(gr < rows && gk < K) << i;
-        const int cr = KMAJOR ? min(gr, rows - 1) : min(gr, rows - 4);
-        const int ck = KMAJOR ? min(gk, K - 4) : min(gk, K - 1);
-        v[i] = *reinterpret_cast<const float4*>(KMAJOR ? P + (int64_t)cr * ld + ck : P + (int64_t)ck * ld + cr);
-      } else {
-        if(KMAJOR) {
-          const float* src = P + (int64_t)gr * ld + gk;
-          if(gr < rows) {
-            if constexpr(VEC) {
-              if(gk < K) x = *reinterpret_cast<const float4*>(src);
-            } else {
-              if(gk + 0 < K) x.x = src[0];
-              if(gk + 1 < K) x.y = src[1];
-              if(gk + 2 < K) x.z = src[2];
-              if(gk + 3 < K) x.w = src[3];
-            }
-          }
-        } else {
-          const float* src = P + (int64_t)gk * ld + gr;
-          if(gk < K) {
-            if constexpr(VEC) {
-              if(gr < rows) x = *reinterpret_cast<const float4*>(src);
-            } else {
-              if(gr + 0 < rows) x.x = src[0];
-              if(gr + 1 < rows) x.y = src[1];
-              if(gr + 2 < rows) x.z = src[2];
-              if(gr + 3 < rows) x.w = src[3];
-            }
-          }
-        }
-        v[i] = x;
-      }
-    }
-  }
-
-  // S is the [BK][LD] k-major LDS panel; VEC as in load().
-  template <int LD, bool VEC>
-  __device__ __forceinline__ void store(float (*S)[LD], int tid) const {
-#pragma unroll
-    for(int i = 0; i < PER; ++i) {
-      const int idx = tid + i * NT;
-      float4 x = v[i];
-      if constexpr(VEC && DEFER) {
-        if(!((in >> i) & 1u)) x = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-      if(KMAJOR) {
-        const int r = idx / (BK / 4), k = (idx % (BK / 4)) * 4;
-        S[k + 0][r] = x.x;
-        S[k + 1][r] = x.y;
-        S[k + 2][r] = x.z;
-        S[k + 3][r] = x.w;
-      } else {
-        const int k = idx / (ROWS / 4), r = (idx % (ROWS / 4)) * 4;
-        *reinterpret_cast<float4*>(&S[k][r]) = x;
-      }
-    }
-  }
-};
-
-// 128-bit loads need 16-byte aligned rows and a contiguous extent that is a
-// multiple of 4 (so a float4 is entirely inside or outside the matrix).
+// 128-bit copies need 16-byte aligned rows and a contiguous extent that is a
+// multiple of 4 (so a chunk is entirely inside or outside the matrix).
 inline bool f32_vec_ok(const float* P, int64_t ld, bool kmajor, int rows, int K) {
   const int contig = kmajor ? K : rows;
   return (reinterpret_cast<uintptr_t>(P) & 15u) == 0 && ld % 4 == 0 && contig % 4 == 0;
 }
 
-// Computes tile (tm, tn) of `op` (all nprod products) and writes it through
-// op.ep.  `smem` holds F32Cfg::SMEM_FLOATS floats; the caller separates two
-// calls that reuse it with a barrier.
-template <int BM, int BN, int BK, int WM, int WN, bool AK, bool BKM, bool VEC, int KG = 1>
-__device__ __forceinline__ void f32_tile(const DenseOp& op, int tm, int tn, float* smem) {
-  using Cfg = F32Cfg<BM, BN, BK, WM, WN, KG>;
-  constexpr int NT = Cfg::NT, FM = Cfg::FM, FN = Cfg::FN;
-  // LDS row strides.  A k-contiguous operand is stored transposed, one float
-  // at a time, by BK/4 threads per row: padding the row by 64/BK floats
-  // (1 from BK = 64 up) puts the 4k-strided stores of those threads in
-  // distinct banks.  Otherwise 128-bit stores need 16-byte rows (pad 4).
-  constexpr int PT = BK >= 64 ? 1 : 64 / BK;
-  constexpr int LA = AK ? BM + PT : Cfg::LDSA, LB = BKM ? BN + PT : Cfg::LDSB;
-  static_assert(LA <= Cfg::LDSA && LB <= Cfg::LDSB, "panels fit the configuration's LDS");
-  typedef float PanelA[BK][LA];
-  typedef float PanelB[BK][LB];
-  PanelA* As = reinterpret_cast<PanelA*>(smem);
-  PanelB* Bs = reinterpret_cast<PanelB*>(smem + 2 * BK * LA);
-
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int g = KG > 1 ? wid / Cfg::NWG : 0, w = wid - g * Cfg::NWG;  // k-group, wave within it
-  const int wm = w / Cfg::NWN, wn = w % Cfg::NWN;
-
-  floatx16 acc[FM][FN];
-#pragma unroll
-  for(int i = 0; i < FM; ++i)
-#pragma unroll
-    for(int j = 0; j < FN; ++j)
-#pragma unroll
-      for(int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
-
-  PanelLoader<BM, BK, NT, AK, (KG > 1)> la;
-  PanelLoader<BN, BK, NT, BKM, (KG > 1)> lb;
-  const int KT = (op.K + BK - 1) / BK;
-  const int steps = KT * op.nprod;
-
-  auto issue_to = [&](auto& xa, auto& xb, int s) __attribute__((always_inline)) {
-    const int prod = s / KT, kt = s - prod * KT;
-    const float* pa = prod ? op.B : op.A;
-    const float* pb = prod ? op.A : op.B;
-    const int64_t lda = prod ? op.ldb : op.lda, ldb = prod ? op.lda : op.ldb;
-    xa.template load<VEC>(pa, lda, op.M, op.K, m0, kt * BK, tid);
-    xb.template load<VEC>(pb, ldb, op.N, op.K, n0, kt * BK, tid);
-  };
-  auto commit_from = [&](const auto& xa, const auto& xb, int buf) __attribute__((always_inline)) {
-    xa.template store<LA, VEC>(As[buf], tid);
-    xb.template store<LB, VEC>(Bs[buf], tid);
-  };
-  auto issue = [&](int s) __attribute__((always_inline)) { issue_to(la, lb, s); };
-  auto commit = [&](int buf) __attribute__((always_inline)) { commit_from(la, lb, buf); };
-  const int lrow = lane & 31, lk = lane >> 5;
-  constexpr int KS = BK / KG;  // k of each stage per group
-  const int kg0 = g * KS;
-  auto compute = [&](int cur) __attribute__((always_inline)) {
-#pragma unroll
-    for(int kk = 0; kk < KS; kk += 2) {
-      float a[FM], b[FN];
-#pragma unroll
-      for(int i = 0; i < FM; ++i) a[i] = As[cur][kg0 + kk + lk][wm * WM + i * 32 + lrow];
-#pragma unroll
-      for(int j = 0; j < FN; ++j) b[j] = Bs[cur][kg0 + kk + lk][wn * WN + j * 32 + lrow];
-#pragma unroll
-      for(int i = 0; i < FM; ++i)
-#pragma unroll
-        for(int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-  };
-
-  if constexpr(KG == 1) {
-    // Steady state without branches around the prefetch, so the registers
-    // holding step s+1 stay live across the MFMAs of step s (no early wait).
-    if(steps > 0) {
-      issue(0);
-      commit(0);
-    }
-    __syncthreads();
-    for(int s = 0; s + 1 < steps; ++s) {
-      issue(s + 1);
-      compute(s & 1);
-      commit((s + 1) & 1);
-      __syncthreads();
-    }
-    if(steps > 0) compute((steps - 1) & 1);
+// Float f of a stage's ROWS-row panel ([16 k][32-row block][512 floats]): its
+// row within the panel and k within the stage.
+template <int ROWS, bool KMAJOR, bool VEC>
+__device__ __forceinline__ void f32_place(int f, int& r, int& k) {
+  const int sub = f / (ROWS * F32_BK), blk = f % (ROWS * F32_BK) >> 9, g = f & 511;
+  if(KMAJOR) {
+    const int chunk = g >> 2, l = chunk & 63;
+    r = blk * 32 + (l & 31);
+    k = sub * F32_BK + 8 * (l >> 5) + 4 * (chunk >> 6) + (VEC ? 0 : g & 3);
   } else {
-    // One workgroup per CU: loads run two stages ahead, in two register
-    // sets (la/lb for even stages, la1/lb1 for odd ones), so a stage's loads
-    // have two stages of MFMAs to land.  At the top of the steady loop stage
-    // s is in LDS buffer 0 and stage s+1 in flight in the odd set; the loop
-    // body has no branches, so the compiler waits only for the older set.
-    PanelLoader<BM, BK, NT, AK, true> la1;
-    PanelLoader<BN, BK, NT, BKM, true> lb1;
-    if(steps > 0) issue_to(la, lb, 0);
-    if(steps > 1) issue_to(la1, lb1, 1);
-    if(steps > 0) commit_from(la, lb, 0);
-    __syncthreads();
-    int s = 0;
-    for(; s + 3 < steps; s += 2) {
-      issue_to(la, lb, s + 2);
-      compute(0);
-      commit_from(la1, lb1, 1);
-      __syncthreads();
-      issue_to(la1, lb1, s + 3);
-      compute(1);
-      commit_from(la, lb, 0);
-      __syncthreads();
-    }
-    const int left = steps - s;  // 0 (no k at all) to 3
-    if(left == 3) {
-      issue_to(la, lb, s + 2);
-      compute(0);
-      commit_from(la1, lb1, 1);
-      __syncthreads();
-      compute(1);
-      commit_from(la, lb, 0);
-      __syncthreads();
-      compute(0);
-    } else if(left == 2) {
-      compute(0);
-      commit_from(la1, lb1, 1);
-      __syncthreads();
-      compute(1);
-    } else if(left == 1) {
-      compute(0);
-    }
+    r = blk * 32 + (g & 31);
+    k = sub * F32_BK + (g >> 5);
   }
+}
 
-  if constexpr(KG > 1) {
-    // Groups 1..KG-1 park their accumulators in LDS (over the panels, once
-    // every group is done with them), lane-contiguous; group 0 adds them in
-    // group order and alone writes the tile.
-    __syncthreads();
-    auto at = [&](int grp, int blk, int q) __attribute__((always_inline)) {
-      return ((((grp - 1) * Cfg::NWG + w) * (FM * FN) + blk) * 16 + q) * 64 + lane;
+// Contracts stages [s0, s1) of tile (tm, tn) of `op` (a product's stages are
+// ceil(K / (16 KG)), the second product's follow the first's) and writes alpha *
+// sum + beta * C through `ep` at row er, column ec.  `smem` holds
+// F32Cfg::SMEM_FLOATS floats; the caller separates two calls that reuse it
+// with a barrier.
+//
+// The pipeline is bf16_tile's (tile_bf16.h): the LDS reads of the next half
+// stage between the MFMAs of the current one, across the stage boundary too,
+// and the copies of the stage NB further on spread over the MFMAs behind the
+// barrier.  The earlier form went through registers (global loads, then
+// transposing LDS stores with both waves of a SIMD waiting at the barrier
+// behind them) and lost 15 to 20 % of the MFMA time on big tiles, a third on
+// small ones.  Measured on MI355X with a tile on every CU, ns per k before ->
+// after: 256x256 250 -> 220 (130 -> 146 TFLOP/s), 128x128 80 -> 62, 64x64
+// 20.8 -> 18.2.  With one wave per SIMD a stage costs about 300 cycles beyond
+// its MFMAs (64x64: 21.0), with two the other wave's MFMAs fill them; four
+// groups of the 64x64 tile are no better (19.6).
+//
+// Rows past the operand read its last row again and only feed outputs the
+// epilogue does not store.  k past the end (K % 16) reads k inside it again
+// and is zeroed in both operands' fragments in the last stage, so Inf and NaN
+// stay where they belong.
+template <int BM, int BN, int WM, int WN, bool AK, bool BKM, bool VEC, int WANT = f32_stages<BM, BN>(),
+    int KG = 1>
+__device__ __forceinline__ void f32_tile(const DenseOp& op, int tm, int tn, int s0, int s1, const Epilogue& ep, int er,
+    int ec, float* smem) {
+  using Cfg = F32Cfg<BM, BN, WM, WN, VEC, WANT, KG>;
+  constexpr int NT = Cfg::NT, FM = Cfg::FM, FN = Cfg::FN, NB = Cfg::NB, W = Cfg::W;
+  constexpr int STAGE = Cfg::STAGE, PER_A = Cfg::PER_A, PER = Cfg::PER, BK = Cfg::BK;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = KG > 1 ? wid / Cfg::NWG : 0, wave = wid - group * Cfg::NWG;
+  const int wm = wave / Cfg::NWN, wn = wave % Cfg::NWN;
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  // One 32x32 block per wave would make every MFMA wait for the one before:
+  // two accumulators take turns then, added at the end.
+  constexpr int NA = FM * FN == 1 ? 2 : 1;
+  floatx16 acc[NA][FM][FN];
+#pragma unroll
+  for(int n = 0; n < NA; ++n)
+#pragma unroll
+    for(int i = 0; i < FM; ++i)
+#pragma unroll
+      for(int j = 0; j < FN; ++j)
+#pragma unroll
+        for(int q = 0; q < 16; ++q) acc[n][i][j][q] = 0.0f;
+
+  const int KT = (op.K + BK - 1) / BK;
+  const int tail = op.K % BK;  // k of a partial last stage
+  const int hi = lane >> 5;
+
+  floatx4 a[2][FM], b[2][FN];
+  constexpr int NR = FM + FN;         // fragments per half stage
+  constexpr int NM = 4 * FM * FN;     // MFMAs per half stage
+  using Yes = std::true_type;
+  using No = std::false_type;
+  using Q0 = std::integral_constant<int, 0>;
+  using Q1 = std::integral_constant<int, 1>;
+
+  // fragment r of half stage h of the stage at `st` into set q
+  auto read_one = [&](const float* st, int h, auto qq, auto rr) __attribute__((always_inline)) {
+    constexpr int q = decltype(qq)::value, r = decltype(rr)::value;
+    constexpr bool is_b = r < FN, KM = is_b ? BKM : AK;
+    const float* blk = is_b ? st + Cfg::FL_A + group * BN * F32_BK + (wn * FN + r) * 512
+                            : st + group * BM * F32_BK + (wm * FM + r - FN) * 512;
+    floatx4 v;
+    if constexpr(KM) {
+      v = *reinterpret_cast<const floatx4*>(blk + (h * 64 + lane) * 4);
+    } else {
+#pragma unroll
+      for(int e = 0; e < 4; ++e) v[e] = blk[(8 * hi + 4 * h + e) * 32 + (lane & 31)];
+    }
+    if constexpr(is_b) b[q][r] = v;
+    else a[q][r - FN] = v;
+  };
+
+  // one product's stages [from, to), through the whole pipeline
+  auto run = [&](const float* A, int64_t lda, const float* B, int64_t ldb, int from, int to) __attribute__((always_inline)) {
+    const float* src[PER];
+#pragma unroll
+    for(int i = 0; i < PER; ++i) {
+      int r, k;
+      if(i < PER_A) {
+        f32_place<BM, AK, VEC>((tid + i * NT) * W, r, k);
+        src[i] = A + (AK ? (int64_t)min(m0 + r, op.M - 1) * lda + k : (int64_t)k * lda + min(m0 + r, op.M - W));
+      } else {
+        f32_place<BN, BKM, VEC>((tid + (i - PER_A) * NT) * W, r, k);
+        src[i] = B + (BKM ? (int64_t)min(n0 + r, op.N - 1) * ldb + k : (int64_t)k * ldb + min(n0 + r, op.N - W));
+      }
+    }
+    int next = from;
+    float* dst = smem;
+    // a copy's source moves on by one stage as soon as it is issued (one
+    // addition of a uniform step); past the end it stays on the last stage,
+    // which is then read again into a buffer no one reads
+    const int64_t whole_a = AK ? BK : BK * lda, whole_b = BKM ? BK : BK * ldb;
+    int64_t step_a, step_b;
+    auto steps_for = [&]() __attribute__((always_inline)) {
+      step_a = next + 1 < to ? whole_a : 0;
+      step_b = next + 1 < to ? whole_b : 0;
     };
-    if(g > 0) {
+    auto issue_one = [&](int i) __attribute__((always_inline)) {
+      float* d = dst + ((i < PER_A ? i * NT : Cfg::FL_A / W + (i - PER_A) * NT) + wid * 64) * W;
+      if constexpr(VEC) lds_dma16(reinterpret_cast<const floatx4*>(src[i]), reinterpret_cast<floatx4*>(d));
+      else lds_dma4(src[i], d);
+      src[i] += i < PER_A ? step_a : step_b;
+    };
+    // the sources of a partial last stage go back inside K
+    auto clamp_tail = [&]() __attribute__((always_inline)) {
+      if(tail == 0 || next != KT - 1) return;
 #pragma unroll
-      for(int i = 0; i < FM; ++i)
+      for(int i = 0; i < PER; ++i) {
+        const bool is_a = i < PER_A;
+        const bool km = is_a ? AK : BKM;
+        int r, k;
+        if(is_a) f32_place<BM, AK, VEC>((tid + i * NT) * W, r, k);
+        else f32_place<BN, BKM, VEC>((tid + (i - PER_A) * NT) * W, r, k);
+        const int over = max(k - (tail - (km ? W : 1)), 0);
+        src[i] -= km ? (int64_t)over : (int64_t)over * (is_a ? lda : ldb);
+      }
+    };
+    auto advance = [&]() __attribute__((always_inline)) {
+      if(next + 1 < to) {
+        ++next;
+        clamp_tail();
+      } else {
+        next = to;
+      }
+      dst = dst + STAGE == smem + NB * STAGE ? smem : dst + STAGE;
+      steps_for();
+    };
 #pragma unroll
-        for(int j = 0; j < FN; ++j)
+    for(int i = 0; i < PER; ++i) src[i] += (i < PER_A ? whole_a : whole_b) * from;
+    clamp_tail();
+    steps_for();
+    // the MFMAs of fragment set q (half q of its stage); masked: k >= `keep` of
+    // the stage zeroed
+    auto contract = [&](auto qq, const float* st, int h, auto reads, auto dma, auto masked, int keep) __attribute__((always_inline)) {
+      constexpr int q = decltype(qq)::value;
+      if constexpr(decltype(masked)::value) {
 #pragma unroll
-          for(int q = 0; q < 16; ++q) smem[at(g, i * FN + j, q)] = acc[i][j][q];
+        for(int e = 0; e < 4; ++e) {
+          const bool in = group * F32_BK + 8 * hi + 4 * q + e < keep;
+#pragma unroll
+          for(int i = 0; i < FM; ++i) a[q][i][e] = in ? a[q][i][e] : 0.0f;
+#pragma unroll
+          for(int j = 0; j < FN; ++j) b[q][j][e] = in ? b[q][j][e] : 0.0f;
+        }
+      }
+      static_for<NM>([&](auto mm) __attribute__((always_inline)) {
+        constexpr int m = decltype(mm)::value;
+        // the first at once, all of them three quarters through (64x64 tile:
+        // before the first MFMA, the only ones that hide their latency)
+        constexpr int MR = NM * 3 / 4 > 3 ? NM * 3 / 4 : 1;
+        constexpr int r0 = m < MR ? (m * NR + MR - 1) / MR : NR, r1 = m < MR ? ((m + 1) * NR + MR - 1) / MR : NR;
+        if constexpr(decltype(reads)::value)
+          static_for<r1 - r0>([&](auto x) __attribute__((always_inline)) {
+            read_one(st, h, std::integral_constant<int, 1 - q>{}, std::integral_constant<int, r0 + decltype(x)::value>{});
+          });
+        constexpr int d0 = m * PER / NM, d1 = (m + 1) * PER / NM;
+        if constexpr(decltype(dma)::value)
+          static_for<d1 - d0>([&](auto x) __attribute__((always_inline)) { issue_one(d0 + decltype(x)::value); });
+        constexpr int e = m / (FM * FN), i = m % (FM * FN) / FN, j = m % FN;
+        acc[e % NA][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][i][e], b[q][j][e], acc[e % NA][i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+
+#pragma unroll
+    for(int p = 0; p < NB; ++p) {
+#pragma unroll
+      for(int i = 0; i < PER; ++i) issue_one(i);
+      advance();
     }
-    __syncthreads();
-    if(g != 0) return;
-    for(int gg = 1; gg < KG; ++gg)
-#pragma unroll
-      for(int i = 0; i < FM; ++i)
-#pragma unroll
-        for(int j = 0; j < FN; ++j)
-#pragma unroll
-          for(int q = 0; q < 16; ++q) acc[i][j][q] += smem[at(gg, i * FN + j, q)];
+    vm_wait<(NB - 1) * PER>();  // the first stage
+    bare_barrier();
+    const float* st = smem;
+    static_for<NR>([&](auto rr) __attribute__((always_inline)) { read_one(st, 0, Q0{}, rr); });
+    for(int s = from; s + 1 < to; ++s) {
+      contract(Q0{}, st, 1, Yes{}, No{}, No{}, 0);
+      // stage s + 1 has landed (the NB - 2 issued after it may still be in
+      // flight) and this wave has read all of stage s
+      vm_wait<(NB - 2) * PER>();
+      lds_wait();
+      bare_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      st = st + STAGE == smem + NB * STAGE ? (const float*)smem : st + STAGE;
+      contract(Q1{}, st, 0, Yes{}, Yes{}, No{}, 0);
+      advance();
+    }
+    const int keep = tail != 0 && to == KT ? tail : BK;
+    contract(Q0{}, st, 1, Yes{}, No{}, Yes{}, keep);
+    contract(Q1{}, st, 0, No{}, No{}, Yes{}, keep);
+    lds_dma_wait();  // no copy into LDS is left behind
+  };
+
+  // the stages of each product that [s0, s1) covers
+  if(s1 > s0) {
+#pragma clang loop unroll(disable)
+    for(int prod = s0 >= KT ? 1 : 0;; ++prod) {
+      run(prod ? op.B : op.A, prod ? op.ldb : op.lda, prod ? op.A : op.B, prod ? op.lda : op.ldb,
+          max(s0 - prod * KT, 0), min(s1 - prod * KT, KT));
+      if(s1 <= (prod + 1) * KT) break;
+      __syncthreads();  // the first product's last reads of smem
+    }
   }
 
+  if constexpr(NA == 2) acc[0][0][0] += acc[1][0][0];
+  if constexpr(KG > 1) {
+    __syncthreads();  // every wave is done with the stages
+    float* mine = smem + (wave * FM * FN * 16) * 64 + lane;  // + (group - 1) * BM * BN, lane-contiguous
+    if(group > 0)
+      static_for<FM * FN>([&](auto ij) __attribute__((always_inline)) {
+        constexpr int ij_ = decltype(ij)::value;
+#pragma unroll
+        for(int q = 0; q < 16; ++q) mine[(group - 1) * BM * BN + (ij_ * 16 + q) * 64] = acc[0][ij_ / FN][ij_ % FN][q];
+      });
+    __syncthreads();
+    if(group > 0) return;
+#pragma unroll
+    for(int g = 0; g < KG - 1; ++g)
+      static_for<FM * FN>([&](auto ij) __attribute__((always_inline)) {
+        constexpr int ij_ = decltype(ij)::value;
+#pragma unroll
+        for(int q = 0; q < 16; ++q) acc[0][ij_ / FN][ij_ % FN][q] += mine[g * BM * BN + (ij_ * 16 + q) * 64];
+      });
+  }
   static_for<FM * FN>([&](auto ij) __attribute__((always_inline)) {
     constexpr int i = decltype(ij)::value / FN, j = decltype(ij)::value % FN;
-    store_block32(op.ep, acc[i][j], m0 + wm * WM + i * 32, n0 + wn * WN + j * 32, lane);
+    store_block32(ep, acc[0][i][j], er + wm * WM + i * 32, ec + wn * WN + j * 32, lane);
   });
 }
 
