@@ -536,7 +536,8 @@ __device__ __forceinline__ void bf16_tile_pipe(const BfTileArgs& t, int tm, int 
     if(after >= NB - 2) vm_wait<(NB - 2) * PER>();
     else if(NB > 3 && after == 1) vm_wait<PER>();
     else lds_dma_wait();
-    __syncthreads();
+    lds_wait();
+    bare_barrier();
     if(s + NB - 1 < steps) issue(s + NB - 1);
     const u32x4* sa = lds + (s % NB) * (SA + SB);
 #pragma unroll
@@ -761,7 +762,8 @@ __device__ __forceinline__ void bf16_tile_direct(const DirectTileArgs& t, int tm
       if(after >= NB - 2) vm_wait<(NB - 2) * PER>();
       else if(NB > 3 && after == 1) vm_wait<PER>();
       else lds_dma_wait();
-      __syncthreads();
+      lds_wait();
+      bare_barrier();
       if(s + NB - 1 < steps) issue(s + NB - 1);
       const u32x4* sa = lds + (s % NB) * (SA + SB);
       if(active) contract(sa, sa + SA, ak, bk, part);
