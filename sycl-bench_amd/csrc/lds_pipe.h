@@ -25,4 +25,17 @@ __device__ __forceinline__ void bare_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// LDS layout of 32 rows x 16 k of a k-contiguous FP32 operand: 128 16-byte
+// chunks, chunk c holding row c / 4, k = 4 * kq .. +3.  The four lanes of a
+// copy that share a row read its 64 bytes, so one copy of a wave touches 16
+// cache lines (rows across the lanes instead: 64, and the address path, not
+// the data, bounds the copy).  The order of a row's four chunks is permuted by
+// (row / 4) % 4, so that 16 consecutive rows' chunks of one kq fall in
+// different banks.  Measured on MI355X against the 64-line order: single BF16
+// direct tile, both operands k-contiguous, 4096^3 290 -> 222 us; FP32 64x64
+// tile 18.2 -> 17.5 ns per k.
+__device__ __forceinline__ int kchunk_row(int c) { return c >> 2; }
+__device__ __forceinline__ int kchunk_kq(int c) { return (c & 3) ^ ((c >> 4) & 3); }
+__device__ __forceinline__ int kchunk_at(int row, int kq) { return row * 4 + (kq ^ ((row >> 2) & 3)); }
+
 }  // namespace mfx

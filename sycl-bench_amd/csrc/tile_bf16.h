@@ -561,9 +561,8 @@ __device__ __forceinline__ void bf16_tile_pipe(const BfTileArgs& t, int tm, int 
 // One LDS stage holds 16 k of both panels; a 32-row (or 32-column) block of
 // an operand is 128 16-byte chunks laid out so that one DMA instruction of a
 // wave fills 64 consecutive chunks:
-//   k-major source (element (r, k) at p[r*ld + k]): chunk h*64 + l of a
-//     block holds row l%32, k = 8*(l/32) + 4h .. +3, so a lane's fragment
-//     (8 consecutive k of its row) is chunks l and 64 + l;
+//   k-major source (element (r, k) at p[r*ld + k]): kchunk_at's layout, so a
+//     lane's fragment (8 consecutive k of its row) is two chunks;
 //   row-major source (element (r, k) at p[k*ld + r]): the block is a 16 x 32
 //     (k x r) float array, row k at floats k*32 .. k*32+31, filled 4
 //     consecutive r per chunk, and a lane reads its 8 k one float each.
@@ -599,8 +598,8 @@ struct BfDirectCfg {
 __device__ __forceinline__ const float* direct_src(const DirectOp& o, int row0, int g, int l) {
   const int blk = g >> 1, h = g & 1;
   if(o.kmajor) {
-    const int r = min(row0 + blk * 32 + (l & 31), o.rows - 1);
-    return o.p + (int64_t)r * o.ld + 8 * (l >> 5) + 4 * h;
+    const int c = h * 64 + l, r = min(row0 + blk * 32 + kchunk_row(c), o.rows - 1);
+    return o.p + (int64_t)r * o.ld + 4 * kchunk_kq(c);
   }
   const int c = min(row0 + blk * 32 + (l & 7) * 4, o.rows - 4);
   return o.p + (int64_t)(h * 8 + (l >> 3)) * o.ld + c;
@@ -612,8 +611,9 @@ __device__ __forceinline__ const float* direct_src(const DirectOp& o, int row0, 
 template <bool KMAJOR>
 __device__ __forceinline__ void direct_frag(const u32x4* st, int blk, int l, float (&x)[8]) {
   if constexpr(KMAJOR) {
-    const floatx4 u = __builtin_bit_cast(floatx4, st[blk * 128 + l]);
-    const floatx4 v = __builtin_bit_cast(floatx4, st[blk * 128 + 64 + l]);
+    const int r = l & 31, kq = 2 * (l >> 5);
+    const floatx4 u = __builtin_bit_cast(floatx4, st[blk * 128 + kchunk_at(r, kq)]);
+    const floatx4 v = __builtin_bit_cast(floatx4, st[blk * 128 + kchunk_at(r, kq + 1)]);
 #pragma unroll
     for(int e = 0; e < 4; ++e) {
       x[e] = u[e];

@@ -8,7 +8,7 @@
 // stages in flight, in a layout the DMA writes as it is and the MFMAs read as
 // it is.  One 32-row block of an operand and stage is 512 floats:
 //   k-contiguous operand (element (r, k) at p[r*ld + k]): 128 chunks of four
-//     floats; chunk h*64 + l holds row l%32, k = 8*(l/32) + 4h .. +3;
+//     floats (kchunk_at);
 //   row-contiguous operand (element (r, k) at p[k*ld + r]): a 16 x 32 (k x r)
 //     array.
 // Lane l feeds row l%32 to the MFMA and supplies k slot l/32 of its two, so
@@ -64,9 +64,9 @@ template <int ROWS, bool KMAJOR, bool VEC>
 __device__ __forceinline__ void f32_place(int f, int& r, int& k) {
   const int sub = f / (ROWS * F32_BK), blk = f % (ROWS * F32_BK) >> 9, g = f & 511;
   if(KMAJOR) {
-    const int chunk = g >> 2, l = chunk & 63;
-    r = blk * 32 + (l & 31);
-    k = sub * F32_BK + 8 * (l >> 5) + 4 * (chunk >> 6) + (VEC ? 0 : g & 3);
+    const int chunk = g >> 2;
+    r = blk * 32 + kchunk_row(chunk);
+    k = sub * F32_BK + 4 * kchunk_kq(chunk) + (VEC ? 0 : g & 3);
   } else {
     r = blk * 32 + (g & 31);
     k = sub * F32_BK + (g >> 5);
@@ -87,7 +87,7 @@ __device__ __forceinline__ void f32_place(int f, int& r, int& k) {
 // behind them) and lost 15 to 20 % of the MFMA time on big tiles, a third on
 // small ones.  Measured on MI355X with a tile on every CU, ns per k before ->
 // after: 256x256 250 -> 220 (130 -> 146 TFLOP/s), 128x128 80 -> 62, 64x64
-// 20.8 -> 18.2.  With one wave per SIMD a stage costs about 300 cycles beyond
+// 20.8 -> 17.5.  With one wave per SIMD a stage costs about 300 cycles beyond
 // its MFMAs (64x64: 21.0), with two the other wave's MFMAs fill them; four
 // groups of the 64x64 tile are no better (19.6).
 //
@@ -124,6 +124,7 @@ __device__ __forceinline__ void f32_tile(const DenseOp& op, int tm, int tn, int 
   const int KT = (op.K + BK - 1) / BK;
   const int tail = op.K % BK;  // k of a partial last stage
   const int hi = lane >> 5;
+  const int chunk0 = kchunk_at(lane & 31, 2 * hi), chunk1 = kchunk_at(lane & 31, 2 * hi + 1);
 
   floatx4 a[2][FM], b[2][FN];
   constexpr int NR = FM + FN;         // fragments per half stage
@@ -141,7 +142,7 @@ __device__ __forceinline__ void f32_tile(const DenseOp& op, int tm, int tn, int 
                             : st + group * BM * F32_BK + (wm * FM + r - FN) * 512;
     floatx4 v;
     if constexpr(KM) {
-      v = *reinterpret_cast<const floatx4*>(blk + (h * 64 + lane) * 4);
+      v = *reinterpret_cast<const floatx4*>(blk + (h ? chunk1 : chunk0) * 4);
     } else {
 #pragma unroll
       for(int e = 0; e < 4; ++e) v[e] = blk[(8 * hi + 4 * h + e) * 32 + (lane & 31)];
