@@ -182,9 +182,11 @@ typedef struct mfx_dep {
 } mfx_dep;
 
 /*
- * Runs `count` problems in one persistent grouped launch.  Producers listed in
- * `deps` must come before their consumers in `problems`; a consumer tile waits
- * in-kernel (bounded) for its producers.  Precisions: FP32, SPLIT_BF16, BF16.
+ * Runs `count` problems in one persistent grouped launch (an untuned short
+ * list whose problems each fill the GPU: one dense launch per problem).
+ * Producers listed in `deps` must come before their consumers in `problems`; a
+ * consumer tile waits in-kernel (bounded) for its producers.  Precisions: FP32,
+ * SPLIT_BF16, BF16.
  * No reference counterpart: it batches the per-kernel submissions of
  * polybench/2mm.cpp:91-124, polybench/3mm.cpp:112-159 and
  * runtime/matmulchain.cpp:81-85 (whose DAG edges come from SYCL accessors).

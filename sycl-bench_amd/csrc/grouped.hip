@@ -11,8 +11,6 @@
 
 namespace mfx {
 
-double config_rate(mfx_precision p, int c);
-
 std::string tune_key(mfx_precision p, int64_t m, int64_t n, int64_t k);
 int tuned_lookup(const std::string& key);
 
@@ -72,6 +70,10 @@ constexpr GroupedPolicy kPolicies[] = {
     {4, 5, 1.34, 2, 1},  // 33
     {4, 6, 0.0, 2, 1},   // 34: independent problems on the large tile, problems with
     {4, 5, 0.0, 2, 1},   // 35:   producers (a chain's later levels) on the small one
+    {2, 2, 0.0, 0, 1},   // 36: small tiles for lists that would leave CUs idle on large ones,
+    {6, 6, 0.0, 0, 1},   // 37:   in one kernel
+    {2, 2, 0.0, 1, 1},   // 38:   and one launch per level
+    {6, 6, 0.0, 1, 1},   // 39
 };
 constexpr int kPolicyCount = sizeof(kPolicies) / sizeof(kPolicies[0]);
 
@@ -120,30 +122,115 @@ std::vector<int> assign_configs(const GroupedPolicy& pol, mfx_precision prec, co
   return cfg;
 }
 
-// Estimated duration (arbitrary units) of a launch under a policy: per level,
-// the padded tile work spread over the CUs plus half a tile of tail.
+// Microseconds of one tile of a grouped kernel: fixed + K * ns per k, the
+// latter between `idle` (a quarter of the CUs busy) and `full` (all of them),
+// by precision and configuration, measured on MI355X at K = 512 and 2048.
+// `full` lies between one-tile problems, whose panels all come from HBM (split
+// BF16 256x256: 165, 128x128: 60), and the tiles of one large problem, which
+// share them in L2 (110, 36).
+struct GroupedTileCost {
+  double fixed, idle, full;
+};
+constexpr GroupedTileCost kGroupedF32[7] = {{10.0, 228.0, 240.0}, {6.0, 71.0, 80.0},    {4.0, 23.3, 23.5}, {8.0, 120.0, 138.0},
+                                            {10.0, 228.0, 240.0}, {8.0, 117.0, 135.0}, {6.0, 68.0, 78.0}};
+constexpr GroupedTileCost kGroupedSplit[7] = {{10.0, 100.0, 160.0}, {6.0, 38.0, 48.0},  {4.0, 27.0, 27.0}, {8.0, 62.0, 90.0},
+                                              {10.0, 84.0, 140.0}, {8.0, 60.0, 85.0}, {6.0, 35.5, 46.0}};
+constexpr GroupedTileCost kGroupedBf16[7] = {{10.0, 70.0, 95.0}, {6.0, 27.0, 40.0}, {4.0, 17.0, 17.5}, {8.0, 42.0, 62.0},
+                                             {10.0, 55.0, 80.0}, {8.0, 40.0, 58.0}, {6.0, 25.0, 38.0}};
+
+// busy: tiles per CU of the level
+double grouped_tile_us(mfx_precision prec, int c, int64_t k, double busy) {
+  const GroupedTileCost& t =
+      prec == MFX_PREC_FP32 ? kGroupedF32[c] : prec == MFX_PREC_SPLIT_BF16 ? kGroupedSplit[c] : kGroupedBf16[c];
+  const double x = std::min(1.0, std::max(0.0, (busy - 0.25) / 0.75));
+  return t.fixed + 1e-3 * (t.idle + (t.full - t.idle) * x) * (double)std::max<int64_t>(k, 1);
+}
+
+// Estimated microseconds of the tiles of one level (level[i] == lv), problem i
+// on configuration of(i): whole rounds over the CUs where all tiles are alike,
+// else the work spread over the CUs plus a quarter of the longest tile.
+template <class Of>
+double level_estimate(mfx_precision prec, const mfx_gemm_problem* problems, int count, const std::vector<int>& level,
+    int lv, int cus, Of&& of) {
+  auto tiles_of = [&](int i) {
+    const auto& q = problems[i];
+    const int c = of(i);
+    return level[i] != lv || q.m <= 0 || q.n <= 0 ? (int64_t)0 : ceil_div(q.m, cfg_bm(c)) * ceil_div(q.n, cfg_bn(c));
+  };
+  int64_t tiles = 0;
+  for(int i = 0; i < count; ++i) tiles += tiles_of(i);
+  if(tiles == 0) return 0.0;
+  double work = 0.0, longest = 0.0, shortest = -1.0;
+  for(int i = 0; i < count; ++i) {
+    const int64_t n = tiles_of(i);
+    if(n == 0) continue;
+    const double t = grouped_tile_us(prec, of(i), problems[i].k, (double)tiles / cus);
+    work += t * (double)n;
+    longest = std::max(longest, t);
+    shortest = shortest < 0.0 ? t : std::min(shortest, t);
+  }
+  if(longest <= shortest * 1.001) return (double)ceil_div(tiles, cus) * longest;
+  return std::max(longest, work / cus + 0.25 * longest);
+}
+
+// The tile configuration that is estimated shortest when all of a level's
+// problems run it.
+int best_level_config(mfx_precision prec, const mfx_gemm_problem* problems, int count, const std::vector<int>& level,
+    int lv, int cus, double* us) {
+  int best = -1;
+  for(int c = 0; c < 7; ++c) {
+    if(grouped_config(prec, c) != c) continue;
+    const double t = level_estimate(prec, problems, count, level, lv, cus, [&](int) { return c; });
+    if(best < 0 || t < *us) {
+      best = c;
+      *us = t;
+    }
+  }
+  return best;
+}
+
+// What a further dependency level costs beyond its tiles: a launch of its own
+// (item fetches from cold queues, a drained pipeline), or in one kernel the
+// publication and the wait.
+constexpr double kLevelLaunchUs = 14.0, kLevelWaitUs = 8.0;
+
+// Estimated microseconds of a launch under a policy.  One launch per level:
+// the levels' sum.  One kernel: all work spread over the CUs, or the chain of
+// the levels' longest tiles where that is longer.
 double policy_estimate(const GroupedPolicy& pol, mfx_precision prec, const mfx_gemm_problem* problems, int count,
     const std::vector<int>& level, int cus) {
   const int levels = count ? *std::max_element(level.begin(), level.end()) + 1 : 0;
-  std::vector<double> work(levels, 0.0), tmax(levels, 0.0);
-  std::vector<int64_t> ntiles(levels, 0);
   const std::vector<int> cfg = assign_configs(pol, prec, problems, count, level, cus);
-  for(int i = 0; i < count; ++i) {
+  auto of = [&](int i) { return cfg[i]; };
+  if(pol.per_level == 1 && levels > 1) {
+    double est = kLevelLaunchUs * (levels - 1);
+    for(int l = 0; l < levels; ++l) {
+      double uniform = 0.0;
+      best_level_config(prec, problems, count, level, l, cus, &uniform);
+      est += std::min(level_estimate(prec, problems, count, level, l, cus, of), uniform);
+    }
+    return est;
+  }
+  if(levels == 1) return level_estimate(prec, problems, count, level, 0, cus, of);
+  int64_t tiles = 0;
+  auto tiles_of = [&](int i) {
     const auto& q = problems[i];
-    if(q.m <= 0 || q.n <= 0) continue;
-    const int c = cfg[i];
-    const int64_t tiles = ceil_div(q.m, cfg_bm(c)) * ceil_div(q.n, cfg_bn(c));
-    const double t = (double)cfg_bm(c) * cfg_bn(c) * (double)round_up(std::max<int64_t>(q.k, 1), 32) / kTileRate[c];
-    work[level[i]] += t * tiles;
-    tmax[level[i]] = std::max(tmax[level[i]], t);
-    ntiles[level[i]] += tiles;
+    return q.m <= 0 || q.n <= 0 ? (int64_t)0 : ceil_div(q.m, cfg_bm(cfg[i])) * ceil_div(q.n, cfg_bn(cfg[i]));
+  };
+  for(int i = 0; i < count; ++i) tiles += tiles_of(i);
+  std::vector<double> longest(std::max(levels, 1), 0.0);
+  double work = 0.0, last = 0.0, path = kLevelWaitUs * (levels - 1);
+  for(int i = 0; i < count; ++i) {
+    if(tiles_of(i) == 0) continue;
+    const double t = grouped_tile_us(prec, cfg[i], problems[i].k, (double)tiles / cus);
+    work += t * (double)tiles_of(i);
+    last = std::max(last, t);
+    if(level[i] > 0 || levels == 1) longest[level[i]] = std::max(longest[level[i]], t);
   }
-  double est = 0.0;
-  for(int l = 0; l < levels; ++l) {
-    if(ntiles[l] == 0) continue;
-    est += std::max(work[l] / cus + 0.5 * work[l] / ntiles[l], tmax[l]);
-  }
-  return est;
+  // the first level's linked problems are as long as its longest tile at most
+  longest[0] = last;
+  for(int l = 0; l < levels; ++l) path += longest[l];
+  return std::max(work / cus + 0.25 * last, path);
 }
 
 }  // namespace
@@ -187,29 +274,17 @@ int choose_grouped_policy(Handle* h, mfx_precision prec, const mfx_gemm_problem*
   const auto level = problem_levels(count, deps, ndeps);
   const int cus = h->cu_count > 0 ? h->cu_count : 256;
   const bool levels = count > 0 && *std::max_element(level.begin(), level.end()) > 0;
-  // With dependency levels: one launch per level, unless (BF16) at least
-  // half of the work is in problems with neither producers nor consumers --
-  // then one kernel with in-kernel waits, whose list-schedule order fills
-  // the later levels' idle CUs with that work.  Measured on MI355X: a lone
-  // 8-long 2048^2 chain 0.51 ms per level against 0.66 ms in one kernel;
-  // the same chain beside 512 uneven problems 1.61 against 1.55 ms.
-  bool one_kernel = !levels;
-  if(levels && prec != MFX_PREC_FP32) {
-    std::vector<char> linked(count, 0);
-    for(int d = 0; d < ndeps; ++d) linked[deps[d].consumer] = linked[deps[d].producer] = 1;
-    double free_work = 0.0, all_work = 0.0;
-    for(int i = 0; i < count; ++i) {
-      const double w = (double)problems[i].m * problems[i].n * problems[i].k;
-      all_work += w;
-      if(!linked[i]) free_work += w;
-    }
-    one_kernel = free_work >= 0.5 * all_work;
-  }
+  // With dependency levels: one launch per level, or one kernel with in-kernel
+  // waits, whose list-schedule order fills a chain's later levels' idle CUs
+  // with other problems' tiles, by estimate.  Measured on MI355X: a lone 8-long
+  // 2048^2 chain (split BF16) 0.45 ms per level against 0.66 ms in one kernel;
+  // 30 problems of 128 to 1024 beside a chain of four 512^2 (single BF16) 46 us
+  // in one kernel against 68 us per level.
   int best = 0;
   double best_est = -1.0;
   for(int i = 0; i < kPolicyCount; ++i) {
     // without levels the two modes are the same launch
-    if(kPolicies[i].per_level == 2 || one_kernel != (kPolicies[i].per_level == 0)) continue;
+    if(kPolicies[i].per_level == 2 || (!levels && kPolicies[i].per_level == 1)) continue;
     // BF16: the direct tiles (no packing pass; measured 1.3x faster on the
     // batched workload); FP32 has nothing to pack
     if(prec != MFX_PREC_FP32 && !kPolicies[i].direct) continue;
@@ -547,39 +622,20 @@ mfx_status plan_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* p
   } else {
     cfg = assign_configs(pol, prec, problems, count, level, cus);
   }
-  // With a launch per level, a later level whose tiles leave CUs idle (the
-  // last products of a chain) may take a smaller tile of the same workgroup
-  // size for all its problems, in a kernel of its own tile pair, when that
-  // is the least estimated time in rounds over the CUs.
+  // With a launch per level, a level may take one tile for all its problems,
+  // in a kernel of its own tile pair, when that is estimated shorter than the
+  // policy's pair: the later levels of a chain hold few problems, and all
+  // levels of a chain of small matrices would leave CUs idle on large tiles.
   std::vector<int> level_cfg(max_level + 1, -1);
   if(pl.per_level && !pl.pipelined) {
-    const int threads = cfg_threads(pl.big);
-    for(int lv = 1; lv <= max_level; ++lv) {
-      auto level_tiles = [&](int c) {
-        int64_t tiles = 0;
-        for(int i = 0; i < count; ++i)
-          if(level[i] == lv && problems[i].m > 0 && problems[i].n > 0)
-            tiles += ceil_div(problems[i].m, cfg_bm(c >= 0 ? c : cfg[i])) * ceil_div(problems[i].n, cfg_bn(c >= 0 ? c : cfg[i]));
-        return tiles;
-      };
-      if(level_tiles(-1) >= cus) continue;
-      double best_t = -1.0;
-      int best = -1;
-      for(int c = 0; c < 7; ++c) {  // tile configurations 0..6
-        if(grouped_config(prec, c) != c || cfg_threads(c) != threads) continue;
-        const double t = (double)ceil_div(level_tiles(c), cus) * cfg_bm(c) * cfg_bn(c) / config_rate(prec, c);
-        if(best < 0 || t < best_t) {
-          best_t = t;
-          best = c;
-        }
-      }
-      bool uniform = true;
-      for(int i = 0; i < count; ++i) uniform = uniform && (level[i] != lv || cfg[i] == best);
-      if(best >= 0 && !uniform) {
-        level_cfg[lv] = best;
-        for(int i = 0; i < count; ++i)
-          if(level[i] == lv) cfg[i] = best;
-      }
+    for(int lv = 0; lv <= max_level; ++lv) {
+      const double as_is = level_estimate(prec, problems, count, level, lv, cus, [&](int i) { return cfg[i]; });
+      double us = 0.0;
+      const int best = best_level_config(prec, problems, count, level, lv, cus, &us);
+      if(best < 0 || us >= 0.97 * as_is) continue;
+      level_cfg[lv] = best;
+      for(int i = 0; i < count; ++i)
+        if(level[i] == lv) cfg[i] = best;
     }
   }
 
@@ -852,7 +908,6 @@ static mfx_status launch_grouped_kernels(Handle* h, const GroupedPlan& pl, const
     zero_ints_kernel<<<(int)std::min<int64_t>(ceil_div(n, 256), 1024), 256, 0, s>>>(g.head - 1, n, g.error);
   }));
   if(pl.items.empty()) return MFX_SUCCESS;
-  const int grid = h->cu_count > 0 ? h->cu_count : 256;
   const int nhl = pl.prec == MFX_PREC_SPLIT_BF16 ? 2 : 1;
   const int segments = (int)pl.seg_items.size() - 1;
   for(int l = 0; l < segments; ++l) {
@@ -868,8 +923,79 @@ static mfx_status launch_grouped_kernels(Handle* h, const GroupedPlan& pl, const
     gl.nprejobs = pl.seg_prejobs[l + 1] - pl.seg_prejobs[l];
     if(gl.nitems == 0) continue;
     const int big = pl.seg_big[l], small = pl.seg_small[l];
+    // two persistent workgroups of the 64x64 tile (64 KiB of LDS) per CU, one
+    // of the others
+    const int grid = cus_of(h) * (big == 2 && small == 2 && gl.nitems > cus_of(h) ? 2 : 1);
     if(pl.prec == MFX_PREC_FP32) MFX_CHECK(launch_grouped_f32(h, big, small, pl.all_vec, gl, grid, s));
     else MFX_CHECK(launch_grouped_bf16(h, nhl, big, small, pl.all_vec, gl, grid, s));
+  }
+  return MFX_SUCCESS;
+}
+
+// A short list whose problems each fill the GPU runs as one dense launch per
+// problem instead (same stream, in list order, which is a topological one):
+// those kernels split k where tiles are few and reach a tile without queues
+// and problem tables.  Untuned lists only; a forced or tuned policy is kept.
+struct DenseList {
+  std::vector<DenseOp> ops;  // empty: the grouped launch is estimated shorter
+  std::vector<int> config;
+  size_t bytes = 0;  // workspace, shared by the problems in turn
+};
+constexpr int kDenseListMax = 16;
+// Uploading the tables, clearing the counters and the first item of a grouped
+// launch; a dense FP32 / packed BF16 product's floor (its launches on the
+// host); packing a BF16 problem's operands.
+constexpr double kGroupedFixedUs = 20.0, kDenseFloorUs = 9.0, kPackedFloorUs = 14.0;
+constexpr double kPackFixedUs = 4.0, kPackBytesPerUs = 4.5e6;
+
+DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count, const mfx_dep* deps,
+    int ndeps, const GroupedPlan& pl) {
+  DenseList d;
+  if(count == 0 || count > kDenseListMax || h->grouped_policy >= 0 || h->forced_config[prec] >= 0) return d;
+  if(tuned_lookup(grouped_tune_key(prec, problems, count, deps, ndeps)) >= 0) return d;
+  const int cus = cus_of(h);
+  const bool packed = prec != MFX_PREC_FP32, split = prec == MFX_PREC_SPLIT_BF16;
+  double dense = 0.0;
+  for(int i = 0; i < count; ++i) {
+    const auto& q = problems[i];
+    if(q.m == 0 || q.n == 0) continue;
+    const int c = choose_config(h, prec, q.m, q.n, q.k);
+    int bm, bn, bk, w;
+    config_info(prec, c, &bm, &bn, &bk, &w);
+    double us = plan_splits(prec, c, ceil_div(q.m, bm) * ceil_div(q.n, bn), q.k, cus, kMaxPartialBytes, nullptr);
+    if(packed) us += kPackFixedUs + 8.0 * (double)(q.m + q.n) * (double)q.k / kPackBytesPerUs;
+    dense += std::max(packed ? kPackedFloorUs : kDenseFloorUs, us);
+    DenseOp op{};
+    op.M = (int)q.m;
+    op.N = (int)q.n;
+    op.K = (int)q.k;
+    op.A = q.A;
+    op.lda = q.lda;
+    op.a_kmajor = q.transA == 0;
+    op.B = q.B;
+    op.ldb = q.ldb;
+    op.b_kmajor = q.transB == 1;
+    op.nprod = 1;
+    op.tiles = TILES_FULL;
+    op.ep = Epilogue{q.C, q.ldc, q.alpha, q.beta, (int)q.m, (int)q.n, TILES_FULL, 0};
+    d.ops.push_back(op);
+    d.config.push_back(c);
+    d.bytes = std::max(d.bytes, packed ? dense_bf16x_workspace(op, split, c, cus, h->forced_splits)
+                                       : dense_f32_workspace(op, c, cus, h->forced_splits));
+  }
+  const auto level = problem_levels(count, deps, ndeps);
+  const double grouped = kGroupedFixedUs + policy_estimate(kPolicies[pl.policy], prec, problems, count, level, cus);
+  // Clearly ahead only. A packed list pays three launches a problem, which the
+  // model knows less well: 8 chained products of 363 measured 102 us dense and
+  // 83 grouped at equal estimates, four of 1024 66 and 101.
+  if(dense >= (packed ? 0.75 : 0.9) * grouped) d.ops.clear();
+  return d;
+}
+
+mfx_status launch_dense_list(Handle* h, mfx_precision prec, const DenseList& d, void* ws, hipStream_t s) {
+  for(size_t i = 0; i < d.ops.size(); ++i) {
+    if(prec == MFX_PREC_FP32) MFX_CHECK(launch_dense_f32_ws(h, d.ops[i], d.config[i], ws, d.bytes, s));
+    else MFX_CHECK(launch_dense_bf16x_ws(h, d.ops[i], prec == MFX_PREC_SPLIT_BF16, d.config[i], ws, s));
   }
   return MFX_SUCCESS;
 }
@@ -879,6 +1005,16 @@ mfx_status run_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* pr
   GroupedPlan pl;
   MFX_CHECK(plan_grouped(h, prec, problems, count, deps, ndeps, pl));
   void* ws = nullptr;
+  const DenseList dense = dense_list(h, prec, problems, count, deps, ndeps, pl);
+  h->grouped_waits = true;
+  if(!dense.ops.empty()) {
+    // packed operands that do not fit: the grouped kernels need none
+    if(dense.bytes == 0 || workspace(h, dense.bytes, &ws) == MFX_SUCCESS) {
+      h->grouped_waits = false;
+      return launch_dense_list(h, prec, dense, ws, s);
+    }
+    (void)hipGetLastError();
+  }
   MFX_CHECK(workspace(h, pl.total_bytes, &ws));
   GroupedArgs g;
   MFX_CHECK(bind_grouped(h, pl, ws, g, s));
@@ -991,7 +1127,7 @@ mfx_status mfx_grouped_status(mfx_handle handle, mfx_stream stream) {
   Handle* h = &handle->h;
   MFX_HIP(hipSetDevice(h->device));
   MFX_HIP(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
-  if(!h->error_flag) return MFX_SUCCESS;
+  if(!h->error_flag || !h->grouped_waits) return MFX_SUCCESS;
   int err = 0;
   MFX_HIP(hipMemcpy(&err, h->error_flag, sizeof(int), hipMemcpyDeviceToHost));
   if(err) {
@@ -1015,20 +1151,26 @@ mfx_status mfx_grouped_graph_create(mfx_handle handle, mfx_precision prec, const
   gr->device = h->device;
   // The graph owns its tables, counters and packed operands, so later calls on
   // the handle (which may regrow the handle's workspace) cannot move them.
-  hipError_t ae = hipMalloc(&gr->mem, std::max<size_t>(pl.total_bytes, 256));
+  DenseList dense = dense_list(h, prec, problems, count, deps, ndeps, pl);
+  hipError_t ae = hipMalloc(&gr->mem, std::max<size_t>(dense.ops.empty() ? pl.total_bytes : dense.bytes, 256));
+  if(ae != hipSuccess && !dense.ops.empty()) {
+    (void)hipGetLastError();
+    dense.ops.clear();
+    ae = hipMalloc(&gr->mem, std::max<size_t>(pl.total_bytes, 256));
+  }
   if(ae != hipSuccess) {
     delete gr;
     return hip_fail(ae, "hipMalloc(grouped graph)");
   }
-  GroupedArgs g;
-  mfx_status bs = bind_grouped(h, pl, gr->mem, g, s);
+  GroupedArgs g{};
+  mfx_status bs = dense.ops.empty() ? bind_grouped(h, pl, gr->mem, g, s) : MFX_SUCCESS;
   hipError_t se = hipStreamSynchronize(s);  // tables resident before capture
   if(bs != MFX_SUCCESS || se != hipSuccess) {
     (void)hipFree(gr->mem);
     delete gr;
     return bs != MFX_SUCCESS ? bs : hip_fail(se, "hipStreamSynchronize");
   }
-  gr->error = g.error;
+  gr->error = g.error;  // null for dense launches, which wait for nothing
   // Capture on a private stream: the graph holds the counter reset (a
   // kernel, not a memset node) and the persistent kernel.
   hipStream_t cs = nullptr;
@@ -1044,7 +1186,7 @@ mfx_status mfx_grouped_graph_create(mfx_handle handle, mfx_precision prec, const
   mfx_status st = MFX_SUCCESS;
   hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
   if(e == hipSuccess) {
-    st = launch_grouped_kernels(h, pl, g, cs);
+    st = dense.ops.empty() ? launch_grouped_kernels(h, pl, g, cs) : launch_dense_list(h, prec, dense, gr->mem, cs);
     hipError_t e2 = hipStreamEndCapture(cs, &gr->graph);
     if(st == MFX_SUCCESS && e2 != hipSuccess) st = hip_fail(e2, "hipStreamEndCapture");
   } else {
@@ -1079,6 +1221,7 @@ mfx_status mfx_graph_status(mfx_graph graph, mfx_stream stream) {
   if(!graph) return invalid("null graph");
   MFX_HIP(hipSetDevice(graph->device));
   MFX_HIP(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
+  if(!graph->error) return MFX_SUCCESS;
   int err = 0;
   MFX_HIP(hipMemcpy(&err, graph->error, sizeof(int), hipMemcpyDeviceToHost));
   if(err) {

@@ -130,7 +130,12 @@ __device__ __forceinline__ void prepack_item(const PackJob* jobs, int njobs, int
 // Grouped tiles mostly stream panels that no other running tile shares, so
 // they run the deeper pipeline: four buffers of half a stage, three in
 // flight, in the LDS that bf16_tile uses for two.
+// The 64x64 tile, whose direct stages hold 8 KiB, buffers eight.
 constexpr int PIPE_NB = 4;
+template <int C>
+constexpr int direct_nb() {
+  return C == 2 ? 8 : PIPE_NB;
+}
 template <int NHL>
 constexpr int pipe_kb() {
   return kb_per_stage<NHL>() / 2;
@@ -143,13 +148,13 @@ __device__ __forceinline__ void run_tile(const BfTileArgs& t, int tm, int tn, u3
 
 template <int NHL, int C>
 __device__ __forceinline__ void run_direct(const DirectTileArgs& t, int tm, int tn, u32x4* lds) {
-  bf16_tile_direct<Geo<C>::BM, Geo<C>::BN, Geo<C>::WM, Geo<C>::WN, NHL, PIPE_NB>(t, tm, tn, lds);
+  bf16_tile_direct<Geo<C>::BM, Geo<C>::BN, Geo<C>::WM, Geo<C>::WN, NHL, direct_nb<C>()>(t, tm, tn, lds);
 }
 
 template <int NHL, int C>
 constexpr int bf16_smem_chunks() {
   constexpr int p = BfPipeCfg<Geo<C>::BM, Geo<C>::BN, Geo<C>::WM, Geo<C>::WN, NHL, pipe_kb<NHL>(), PIPE_NB>::SMEM_CHUNKS;
-  constexpr int d = BfDirectCfg<Geo<C>::BM, Geo<C>::BN, Geo<C>::WM, Geo<C>::WN, PIPE_NB>::SMEM_CHUNKS;
+  constexpr int d = BfDirectCfg<Geo<C>::BM, Geo<C>::BN, Geo<C>::WM, Geo<C>::WN, direct_nb<C>()>::SMEM_CHUNKS;
   return p > d ? p : d;
 }
 

@@ -67,6 +67,7 @@ struct Handle {
   size_t staging_bytes = 0;
   hipEvent_t staging_ready = nullptr;
   int* error_flag = nullptr;
+  bool grouped_waits = true;  // the last grouped call launched kernels that can time out
   int forced_splits = -1;  // split-K: -1 automatic, 1 never, >= 2 that many slices
 };
 
