@@ -177,8 +177,9 @@ int heuristic_config(Handle* h, mfx_precision p, int64_t m, int64_t n, int64_t k
 int choose_config(Handle* h, mfx_precision p, int64_t m, int64_t n, int64_t k) {
   if(h->forced_config[p] >= 0) return h->forced_config[p];
   {
+    // the key's text only where a table is there: 0.3 us of a small call's 4.6
     std::lock_guard<std::mutex> lock(g_tune_mutex);
-    auto it = g_tuned.find(tune_key(p, m, n, k));
+    auto it = g_tuned.empty() ? g_tuned.end() : g_tuned.find(tune_key(p, m, n, k));
     if(it != g_tuned.end()) return it->second;
   }
   return heuristic_config(h, p, m, n, k);
@@ -254,7 +255,7 @@ int choose_square_config(Handle* h, mfx_precision p, int64_t n, int64_t k) {
     c = h->forced_config[p];
   } else {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
-    auto it = g_tuned.find(tune_key(p, n, n, k));
+    auto it = g_tuned.empty() ? g_tuned.end() : g_tuned.find(tune_key(p, n, n, k));
     if(it != g_tuned.end()) c = it->second;
   }
   int bm, bn, bk, w;
