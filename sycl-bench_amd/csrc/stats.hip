@@ -214,9 +214,7 @@ __global__ __launch_bounds__(256) void center_kernel(int64_t m, int64_t n, const
     sd[w] = a.stddev ? stat[tx * W + w] : 1.0f;
   }
   const int64_t r1 = min(n, ((int64_t)blockIdx.y + 1) * rows_per);
-  for(int64_t i = (int64_t)blockIdx.y * rows_per + ty; i < r1; i += TY) {
-    float x[W];
-    load_cols<W>(data + i * ld + j, x);
+  auto put = [&](int64_t i, float(&x)[W]) __attribute__((always_inline)) {
 #pragma unroll
     for(int w = 0; w < W; ++w) {
       x[w] -= mu[w];
@@ -225,6 +223,19 @@ __global__ __launch_bounds__(256) void center_kernel(int64_t m, int64_t n, const
     float* o = out + i * ldo + j;
     if constexpr(W == 4) *reinterpret_cast<float4*>(o) = make_float4(x[0], x[1], x[2], x[3]);
     else o[0] = x[0];
+  };
+  int64_t i = (int64_t)blockIdx.y * rows_per + ty;
+  for(; i + 3 * TY < r1; i += 4 * TY) {
+    float x[4][W];
+#pragma unroll
+    for(int u = 0; u < 4; ++u) load_cols<W>(data + (i + u * TY) * ld + j, x[u]);
+#pragma unroll
+    for(int u = 0; u < 4; ++u) put(i + u * TY, x[u]);
+  }
+  for(; i < r1; i += TY) {
+    float x[W];
+    load_cols<W>(data + i * ld + j, x);
+    put(i, x);
   }
 }
 
