@@ -332,7 +332,6 @@ __device__ __forceinline__ void lds_dma4(const T* src, T* lds_wave_base) {
 
 // Waits for this wave's outstanding memory operations, LDS transfers included.
 __device__ __forceinline__ void lds_dma_wait() { __builtin_amdgcn_s_waitcnt(0); }
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Compile-time loop: f(std::integral_constant<int, I>) for I in [0, N).  Used
 // where an index selects an accumulator block, so the index stays a constant
@@ -345,6 +344,13 @@ __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int
 template <int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// alpha * acc + beta * old, rounded the same way wherever it is written: the two
+// halves of a mirrored square have to agree to the last bit, and left to itself
+// the compiler fuses either product into the sum.
+__device__ __forceinline__ float scaled(const Epilogue& ep, float acc, float old) {
+  return fmaf(ep.alpha, acc, ep.beta * old);
 }
 
 // Writes one 32x32 MFMA accumulator block whose top-left corner is (r0, c0).
@@ -370,7 +376,7 @@ __device__ __forceinline__ void store_block32(const Epilogue& ep, floatx16 acc, 
 #pragma unroll
       for(int q = 0; q < 16; ++q) old[q] = direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc];
 #pragma unroll
-      for(int q = 0; q < 16; ++q) direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc] = ep.alpha * acc[q] + ep.beta * old[q];
+      for(int q = 0; q < 16; ++q) direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc] = scaled(ep, acc[q], old[q]);
     } else {
 #pragma unroll
       for(int q = 0; q < 16; ++q) direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc] = ep.alpha * acc[q];
@@ -386,7 +392,7 @@ __device__ __forceinline__ void store_block32(const Epilogue& ep, floatx16 acc, 
       for(int g = 0; g < 4; ++g) {
         floatx4 v;
 #pragma unroll
-        for(int u = 0; u < 4; ++u) v[u] = ep.beta != 0.0f ? ep.alpha * acc[4 * g + u] + ep.beta * was[g][u] : ep.alpha * acc[4 * g + u];
+        for(int u = 0; u < 4; ++u) v[u] = ep.beta != 0.0f ? scaled(ep, acc[4 * g + u], was[g][u]) : ep.alpha * acc[4 * g + u];
         *reinterpret_cast<floatx4*>(mirrored + 8 * g) = v;
       }
       return;
@@ -397,33 +403,37 @@ __device__ __forceinline__ void store_block32(const Epilogue& ep, floatx16 acc, 
     }
 #pragma unroll
     for(int q = 0; q < 16; ++q)
-      mirrored[8 * (q >> 2) + (q & 3)] = ep.beta != 0.0f ? ep.alpha * acc[q] + ep.beta * old[q] : ep.alpha * acc[q];
+      mirrored[8 * (q >> 2) + (q & 3)] = ep.beta != 0.0f ? scaled(ep, acc[q], old[q]) : ep.alpha * acc[q];
     return;
   }
-  // A block at the matrix's edge or across the diagonal.
-  auto writes = [&](int row) {
-    return row < ep.M && col < ep.N && (ep.uplo == TILES_FULL || (ep.uplo == TILES_LOWER ? row >= col : row <= col));
-  };
+  // A block at the matrix's edge or across the diagonal: old values come from
+  // clamped positions without a branch (those of elements that are not written
+  // are not used), so that only the stores are predicated.
+  const int last_row = ep.M - 1, last_col = ep.N - 1, near_col = min(col, last_col);
   auto row_of = [&](int q) { return rbase + 8 * (q >> 2) + (q & 3); };
+  auto writes = [&](int row) {
+    return row <= last_row && col <= last_col && (ep.uplo == TILES_FULL || (ep.uplo == TILES_LOWER ? row >= col : row <= col));
+  };
+  const bool mirror = ep.uplo != TILES_FULL && ep.mirror;  // C is square then
   if(ep.beta != 0.0f) {
 #pragma unroll
-    for(int q = 0; q < 16; ++q)
-      if(writes(row_of(q))) old[q] = direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc];
+    for(int q = 0; q < 16; ++q) old[q] = ep.C[(int64_t)min(row_of(q), last_row) * ep.ldc + near_col];
   }
 #pragma unroll
-  for(int q = 0; q < 16; ++q)
-    if(writes(row_of(q)))
-      direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc] = ep.beta != 0.0f ? ep.alpha * acc[q] + ep.beta * old[q] : ep.alpha * acc[q];
-  if(ep.uplo == TILES_FULL || !ep.mirror) return;
+  for(int q = 0; q < 16; ++q) {
+    const float v = ep.beta != 0.0f ? scaled(ep, acc[q], old[q]) : ep.alpha * acc[q];
+    if(writes(row_of(q))) direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc] = v;
+  }
+  if(!mirror) return;
   if(ep.beta != 0.0f) {
 #pragma unroll
-    for(int q = 0; q < 16; ++q)
-      if(writes(row_of(q)) && row_of(q) != col) old[q] = mirrored[8 * (q >> 2) + (q & 3)];
+    for(int q = 0; q < 16; ++q) old[q] = ep.C[(int64_t)near_col * ep.ldc + min(row_of(q), last_row)];
   }
 #pragma unroll
-  for(int q = 0; q < 16; ++q)
-    if(writes(row_of(q)) && row_of(q) != col)
-      mirrored[8 * (q >> 2) + (q & 3)] = ep.beta != 0.0f ? ep.alpha * acc[q] + ep.beta * old[q] : ep.alpha * acc[q];
+  for(int q = 0; q < 16; ++q) {
+    const float v = ep.beta != 0.0f ? scaled(ep, acc[q], old[q]) : ep.alpha * acc[q];
+    if(writes(row_of(q)) && row_of(q) != col) mirrored[8 * (q >> 2) + (q & 3)] = v;
+  }
 }
 
 // ---------------------------------------------------------------------------

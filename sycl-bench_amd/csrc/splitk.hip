@@ -52,7 +52,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitReduceArg
   const bool inside = r0 + 32 <= ep.M && c0 + 32 <= ep.N;
   if(ep.uplo == TILES_FULL && inside && vec) {
     floatx4* c = reinterpret_cast<floatx4*>(ep.C + (int64_t)row * ep.ldc + col);
-    *c = ep.beta != 0.0f ? ep.alpha * v + ep.beta * *c : ep.alpha * v;
+    const floatx4 old = ep.beta != 0.0f ? *c : v;
+#pragma unroll
+    for(int e = 0; e < 4; ++e) v[e] = ep.beta != 0.0f ? scaled(ep, v[e], old[e]) : ep.alpha * v[e];
+    *c = v;
     return;
   }
   auto wanted = [&](int r, int c) {
@@ -62,7 +65,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitReduceArg
   for(int e = 0; e < 4; ++e)
     if(wanted(row, col + e)) {
       float* c = ep.C + (int64_t)row * ep.ldc + col + e;
-      *c = ep.beta != 0.0f ? ep.alpha * v[e] + ep.beta * *c : ep.alpha * v[e];
+      *c = ep.beta != 0.0f ? scaled(ep, v[e], *c) : ep.alpha * v[e];
     }
   if(ep.uplo == TILES_FULL || !ep.mirror) return;
   // element (row, col) of the triangle also gives (col, row), from its own C
@@ -75,8 +78,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitReduceArg
     const int r = r0 + lc + e, cc = c0 + lr;  // source element; its mirror is (cc, r)
     if(r != cc && wanted(r, cc)) {
       float* c = ep.C + (int64_t)cc * ep.ldc + r;
-      const float x = ep.alpha * tr[lc + e][lr];
-      *c = ep.beta != 0.0f ? x + ep.beta * *c : x;
+      const float x = tr[lc + e][lr];
+      *c = ep.beta != 0.0f ? scaled(ep, x, *c) : ep.alpha * x;
     }
   }
 }
