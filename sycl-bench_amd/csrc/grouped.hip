@@ -133,17 +133,20 @@ struct GroupedTileCost {
 };
 constexpr GroupedTileCost kGroupedF32[7] = {{10.0, 228.0, 240.0}, {6.0, 71.0, 80.0},    {4.0, 23.3, 23.5}, {8.0, 120.0, 138.0},
                                             {10.0, 228.0, 240.0}, {8.0, 117.0, 135.0}, {6.0, 68.0, 78.0}};
-constexpr GroupedTileCost kGroupedSplit[7] = {{10.0, 100.0, 160.0}, {6.0, 38.0, 48.0},  {4.0, 27.0, 27.0}, {8.0, 62.0, 90.0},
-                                              {10.0, 84.0, 140.0}, {8.0, 60.0, 85.0}, {6.0, 35.5, 46.0}};
-constexpr GroupedTileCost kGroupedBf16[7] = {{10.0, 70.0, 95.0}, {6.0, 27.0, 40.0}, {4.0, 17.0, 17.5}, {8.0, 42.0, 62.0},
-                                             {10.0, 55.0, 80.0}, {8.0, 40.0, 58.0}, {6.0, 25.0, 38.0}};
+constexpr GroupedTileCost kGroupedSplit[7] = {{10.0, 100.0, 160.0}, {6.0, 38.0, 48.0},  {5.0, 27.0, 27.0}, {8.0, 62.0, 90.0},
+                                              {10.0, 84.0, 140.0}, {8.0, 60.0, 85.0}, {4.0, 35.5, 46.0}};
+constexpr GroupedTileCost kGroupedBf16[7] = {{10.0, 70.0, 95.0}, {6.0, 27.0, 40.0}, {5.0, 17.0, 17.5}, {8.0, 42.0, 62.0},
+                                             {10.0, 55.0, 80.0}, {8.0, 40.0, 58.0}, {4.0, 25.0, 38.0}};
 
 // busy: tiles per CU of the level
 double grouped_tile_us(mfx_precision prec, int c, int64_t k, double busy) {
   const GroupedTileCost& t =
       prec == MFX_PREC_FP32 ? kGroupedF32[c] : prec == MFX_PREC_SPLIT_BF16 ? kGroupedSplit[c] : kGroupedBf16[c];
   const double x = std::min(1.0, std::max(0.0, (busy - 0.25) / 0.75));
-  return t.fixed + 1e-3 * (t.idle + (t.full - t.idle) * x) * (double)std::max<int64_t>(k, 1);
+  // single BF16 64x64 tiles of packed problems fall behind 128x128 ones from
+  // about K = 256 on: eight chained products of 200 57 and 66 us, of 363 79 and 74
+  const double packed = c == 2 && prec == MFX_PREC_BF16 && k % 16 != 0 && k >= 256 ? 5.0 : 0.0;
+  return t.fixed + packed + 1e-3 * (t.idle + (t.full - t.idle) * x) * (double)std::max<int64_t>(k, 1);
 }
 
 // Estimated microseconds of the tiles of one level (level[i] == lv), problem i
@@ -191,14 +194,32 @@ int best_level_config(mfx_precision prec, const mfx_gemm_problem* problems, int 
 
 // What a further dependency level costs beyond its tiles: a launch of its own
 // (item fetches from cold queues, a drained pipeline), or in one kernel the
-// publication and the wait.
-constexpr double kLevelLaunchUs = 14.0, kLevelWaitUs = 8.0;
+// publication and the wait. In a chain without other problems to fill the wait
+// it depends on the tile and on packing: nearly nothing beyond the publication
+// on 128x128 tiles read directly, but 12 us on 64x64 tiles, whose second
+// workgroup per CU polls beside the first, and more where a level packs its
+// operands first (split BF16, eight chained products of 512: 87 us on 128x128
+// tiles in one kernel, 102 in a launch per level, 99 on 64x64 tiles in one kernel).
+constexpr double kLevelLaunchUs = 16.0, kLevelWaitUs = 8.0, kLoneLevelWaitUs = 6.0, kSlowLevelWaitUs = 20.0;
+
+// Whether problems with producers or consumers hold more than half of the work.
+bool mostly_linked(const mfx_gemm_problem* problems, int count, const mfx_dep* deps, int ndeps) {
+  std::vector<char> linked(count, 0);
+  for(int d = 0; d < ndeps; ++d) linked[deps[d].consumer] = linked[deps[d].producer] = 1;
+  double free_work = 0.0, all_work = 0.0;
+  for(int i = 0; i < count; ++i) {
+    const double w = (double)problems[i].m * problems[i].n * problems[i].k;
+    all_work += w;
+    if(!linked[i]) free_work += w;
+  }
+  return free_work < 0.5 * all_work;
+}
 
 // Estimated microseconds of a launch under a policy.  One launch per level:
 // the levels' sum.  One kernel: all work spread over the CUs, or the chain of
 // the levels' longest tiles where that is longer.
 double policy_estimate(const GroupedPolicy& pol, mfx_precision prec, const mfx_gemm_problem* problems, int count,
-    const std::vector<int>& level, int cus) {
+    const std::vector<int>& level, bool lone, int cus) {
   const int levels = count ? *std::max_element(level.begin(), level.end()) + 1 : 0;
   const std::vector<int> cfg = assign_configs(pol, prec, problems, count, level, cus);
   auto of = [&](int i) { return cfg[i]; };
@@ -219,7 +240,7 @@ double policy_estimate(const GroupedPolicy& pol, mfx_precision prec, const mfx_g
   };
   for(int i = 0; i < count; ++i) tiles += tiles_of(i);
   std::vector<double> longest(std::max(levels, 1), 0.0);
-  double work = 0.0, last = 0.0, path = kLevelWaitUs * (levels - 1);
+  double work = 0.0, last = 0.0;
   for(int i = 0; i < count; ++i) {
     if(tiles_of(i) == 0) continue;
     const double t = grouped_tile_us(prec, cfg[i], problems[i].k, (double)tiles / cus);
@@ -229,6 +250,9 @@ double policy_estimate(const GroupedPolicy& pol, mfx_precision prec, const mfx_g
   }
   // the first level's linked problems are as long as its longest tile at most
   longest[0] = last;
+  bool slow = pol.small == 2;
+  for(int i = 0; i < count; ++i) slow = slow || (prec != MFX_PREC_FP32 && problems[i].k % 16 != 0);
+  double path = (!lone ? kLevelWaitUs : slow ? kSlowLevelWaitUs : kLoneLevelWaitUs) * (levels - 1);
   for(int l = 0; l < levels; ++l) path += longest[l];
   return std::max(work / cus + 0.25 * last, path);
 }
@@ -282,13 +306,14 @@ int choose_grouped_policy(Handle* h, mfx_precision prec, const mfx_gemm_problem*
   // in one kernel against 68 us per level.
   int best = 0;
   double best_est = -1.0;
+  const bool lone = mostly_linked(problems, count, deps, ndeps);
   for(int i = 0; i < kPolicyCount; ++i) {
     // without levels the two modes are the same launch
     if(kPolicies[i].per_level == 2 || (!levels && kPolicies[i].per_level == 1)) continue;
     // BF16: the direct tiles (no packing pass; measured 1.3x faster on the
     // batched workload); FP32 has nothing to pack
     if(prec != MFX_PREC_FP32 && !kPolicies[i].direct) continue;
-    const double e = policy_estimate(kPolicies[i], prec, problems, count, level, cus);
+    const double e = policy_estimate(kPolicies[i], prec, problems, count, level, lone, cus);
     if(best_est < 0 || e < best_est) {
       best_est = e;
       best = i;
@@ -945,7 +970,7 @@ constexpr int kDenseListMax = 16;
 // Uploading the tables, clearing the counters and the first item of a grouped
 // launch; a dense FP32 / packed BF16 product's floor (its launches on the
 // host); packing a BF16 problem's operands.
-constexpr double kGroupedFixedUs = 20.0, kDenseFloorUs = 9.0, kPackedFloorUs = 14.0;
+constexpr double kGroupedFixedUs = 20.0, kDenseFloorUs = 11.0, kSplitFloorUs = 14.0, kBf16FloorUs = 12.0;
 constexpr double kPackFixedUs = 4.0, kPackBytesPerUs = 4.5e6;
 
 DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count, const mfx_dep* deps,
@@ -964,7 +989,7 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
     config_info(prec, c, &bm, &bn, &bk, &w);
     double us = plan_splits(prec, c, ceil_div(q.m, bm) * ceil_div(q.n, bn), q.k, cus, kMaxPartialBytes, nullptr);
     if(packed) us += kPackFixedUs + 8.0 * (double)(q.m + q.n) * (double)q.k / kPackBytesPerUs;
-    dense += std::max(packed ? kPackedFloorUs : kDenseFloorUs, us);
+    dense += std::max(split ? kSplitFloorUs : packed ? kBf16FloorUs : kDenseFloorUs, us);
     DenseOp op{};
     op.M = (int)q.m;
     op.N = (int)q.n;
@@ -984,11 +1009,12 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
                                        : dense_f32_workspace(op, c, cus, h->forced_splits));
   }
   const auto level = problem_levels(count, deps, ndeps);
-  const double grouped = kGroupedFixedUs + policy_estimate(kPolicies[pl.policy], prec, problems, count, level, cus);
-  // Clearly ahead only. A packed list pays three launches a problem, which the
-  // model knows less well: 8 chained products of 363 measured 102 us dense and
-  // 83 grouped at equal estimates, four of 1024 66 and 101.
-  if(dense >= (packed ? 0.75 : 0.9) * grouped) d.ops.clear();
+  const double grouped = kGroupedFixedUs + policy_estimate(kPolicies[pl.policy], prec, problems, count, level,
+                                               mostly_linked(problems, count, deps, ndeps), cus);
+  // Clearly ahead only: a packed list pays two or three launches a problem,
+  // which the model knows less well. Split BF16, dense and the best grouped
+  // policy: four chained products of 500 35 and 57 us, eight of 900 143 and 174.
+  if(dense >= (packed ? 0.8 : 0.9) * grouped) d.ops.clear();
   return d;
 }
 

@@ -103,7 +103,7 @@ constexpr TileCost kF32Cost[] = {
     {4.0, 16.4, 18.2, 34.5},    // 64x64, two k-groups
 };
 constexpr TileCost kSplitCost[] = {
-    {6.0, 44.0, 64.0, 0.0},  // 256x256, four waves
+    {12.0, 44.0, 64.0, 0.0}, // 256x256, four waves: one wave per SIMD stores the tile
     {5.8, 12.4, 18.0, 0.0},  // 128x128, four waves
     {4.0, 6.7, 6.8, 13.0},   // 64x64
     {7.0, 22.5, 33.0, 0.0},  // 256x128, four waves
@@ -112,7 +112,7 @@ constexpr TileCost kSplitCost[] = {
     {4.9, 13.3, 19.0, 0.0},  // 128x128, eight waves
 };
 constexpr TileCost kBf16Cost[] = {
-    {7.5, 16.0, 24.5, 0.0}, {4.5, 6.2, 8.2, 0.0},  {3.4, 3.87, 3.9, 5.5}, {5.5, 9.7, 14.0, 0.0},
+    {13.5, 16.0, 24.5, 0.0}, {4.5, 6.2, 8.2, 0.0},  {3.4, 3.87, 3.9, 5.5}, {5.5, 9.7, 14.0, 0.0},
     {6.0, 15.4, 24.5, 0.0}, {5.3, 9.5, 13.8, 0.0}, {4.0, 6.1, 8.3, 0.0},
 };
 constexpr TileCost kFp8Cost[] = {
