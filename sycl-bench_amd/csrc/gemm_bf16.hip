@@ -60,15 +60,15 @@ struct BfParams {
   float* partial;
 };
 
-template <int BM, int BN, int WM, int WN, int NHL>
+template <int BM, int BN, int WM, int WN, int NHL, int MOST = 4>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16x_kernel(const BfParams p) {
-  using Cfg = BfCfg<BM, BN, WM, WN, NHL>;
+  using Cfg = BfCfg<BM, BN, WM, WN, NHL, MOST>;
   __shared__ u32x4 lds[Cfg::SMEM_CHUNKS];
   int tm, tn;
   const int steps = p.t.kbs / Cfg::KB * p.t.nprod;
   if((int)blockIdx.x < p.plan.head) {
     tile_of(p.mode, xcd_remap(blockIdx.x, p.plan.head), p.tiles_m, p.tiles_n, p.group, tm, tn);
-    bf16_tile<BM, BN, WM, WN, NHL>(p.t, tm, tn, 0, steps, p.t.ep, tm * BM, tn * BN, lds);
+    bf16_tile<BM, BN, WM, WN, NHL, MOST>(p.t, tm, tn, 0, steps, p.t.ep, tm * BM, tn * BN, lds);
     return;
   }
   // slice-major: an XCD's consecutive workgroups read the same k range of
@@ -80,7 +80,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_bf16x_kernel(
   const int s0 = (int)((int64_t)steps * slice / splits), s1 = (int)((int64_t)steps * (slice + 1) / splits);
   float* slot = p.partial + ((int64_t)tile * splits + slice) * (BM * BN);
   const Epilogue ep{slot, BN, 1.0f, 0.0f, BM, BN, TILES_FULL, 0};
-  bf16_tile<BM, BN, WM, WN, NHL>(p.t, tm, tn, s0, s1, ep, 0, 0, lds);
+  bf16_tile<BM, BN, WM, WN, NHL, MOST>(p.t, tm, tn, s0, s1, ep, 0, 0, lds);
 }
 
 struct BfConfig {
@@ -97,14 +97,14 @@ constexpr BfConfig kBfConfigs[] = {
 };
 constexpr int kBfConfigCount = sizeof(kBfConfigs) / sizeof(kBfConfigs[0]);
 
-template <int BM, int BN, int WM, int WN>
+template <int BM, int BN, int WM, int WN, int MOST = 4>
 mfx_status launch_bf_cfg(Handle* h, const BfParams& p, bool split, int grid, hipStream_t s) {
   if(split)
     return timed_launch(h, "gemm_split_bf16_mfma", s, [&] {
-      gemm_bf16x_kernel<BM, BN, WM, WN, 2><<<grid, BfCfg<BM, BN, WM, WN, 2>::NT, 0, s>>>(p);
+      gemm_bf16x_kernel<BM, BN, WM, WN, 2, MOST><<<grid, BfCfg<BM, BN, WM, WN, 2>::NT, 0, s>>>(p);
     });
   return timed_launch(h, "gemm_bf16_mfma", s, [&] {
-    gemm_bf16x_kernel<BM, BN, WM, WN, 1><<<grid, BfCfg<BM, BN, WM, WN, 1>::NT, 0, s>>>(p);
+    gemm_bf16x_kernel<BM, BN, WM, WN, 1, MOST><<<grid, BfCfg<BM, BN, WM, WN, 1>::NT, 0, s>>>(p);
   });
 }
 
@@ -116,7 +116,11 @@ mfx_status launch_bf_config(Handle* h, const BfParams& p, bool split, int config
     case 3: return launch_bf_cfg<256, 128, 128, 64>(h, p, split, grid, s);
     case 4: return launch_bf_cfg<256, 256, 128, 64>(h, p, split, grid, s);
     case 5: return launch_bf_cfg<256, 128, 64, 64>(h, p, split, grid, s);
-    case 6: return launch_bf_cfg<128, 128, 64, 32>(h, p, split, grid, s);
+    case 6:
+      if(p.plan.splits == 1 &&
+         bf16_two_per_cu(split ? MFX_PREC_SPLIT_BF16 : MFX_PREC_BF16, config, p.tiles, p.t.kbs * 16 * p.t.nprod, cus_of(h)))
+        return launch_bf_cfg<128, 128, 64, 32, 2>(h, p, split, grid, s);
+      return launch_bf_cfg<128, 128, 64, 32>(h, p, split, grid, s);
   }
   return invalid("unknown BF16 configuration");
 }

@@ -164,6 +164,18 @@ double tile_span(mfx_precision p, int config, int64_t count, double len, int cus
   return (double)rounds * round((double)slots / cus) + (rest ? round((double)rest / cus) : 0.0);
 }
 
+// Whether the eight-wave 128x128 BF16 tile runs with two LDS buffers instead of
+// four, which lets two workgroups share a CU: sums of at most four stages (128
+// k split, 256 single) have nothing for the third and fourth buffer, and more
+// tiles than CUs are bound by storing C, which one workgroup does while the
+// other loads and multiplies.  5524 x 7793 x 79, the
+// call: split BF16 62.6 -> 48.0 us (61.0 on the best other tile), single BF16
+// 53.6 -> 39.0 (52.4).
+bool bf16_two_per_cu(mfx_precision p, int config, int64_t tiles, int64_t k, int cus) {
+  const int64_t most = p == MFX_PREC_SPLIT_BF16 ? 128 : p == MFX_PREC_BF16 ? 256 : 0;
+  return config == 6 && k <= most && tiles > cus;
+}
+
 // The tiles that do not fill a round of the CUs -- all of them, or those past
 // the whole rounds -- run whole or in up to 64 slices of at least two stages,
 // whichever this model makes shorter: tile_span, and for a split the
@@ -173,6 +185,10 @@ double plan_splits(mfx_precision p, int config, int64_t tiles, int64_t k, int cu
   int bm, bn, bk, w;
   if(plan) *plan = SplitPlan{(int)tiles, 1};
   if(!config_info(p, config, &bm, &bn, &bk, &w) || tiles <= 0) return 0.0;
+  // two tiles per CU and round, which take turns storing: 2.5 us on the scale of
+  // the other tiles' `fixed`, which does not hold the stores of round after round
+  if(bf16_two_per_cu(p, config, tiles, k, cus))
+    return (double)ceil_div(tiles, 2 * (int64_t)cus) * (2.5 + 1e-3 * (p == MFX_PREC_SPLIT_BF16 ? 26.0 : 13.0) * (double)k);
   auto span = [&](int64_t count, double len) { return tile_span(p, config, count, len, cus); };
   double best = span(tiles, (double)k);
   const int64_t steps = ceil_div(k, bk);

@@ -216,8 +216,9 @@ __device__ __forceinline__ void pack_chunk(const PackSrc& s, int blk, int kb, in
 // four-wave 256x256 single-BF16 tile, which gains 2 % from four shorter
 // stages), and as many stages as fit the 160 KiB of LDS, at most four, are
 // buffered: the small tiles, whose stages hold little MFMA work, need that
-// many in flight to cover the global-to-LDS latency.
-template <int BM, int BN, int WM, int WN, int NHL>
+// many in flight to cover the global-to-LDS latency.  MOST: at most that many,
+// where short sums leave nothing to buffer and a second workgroup per CU helps.
+template <int BM, int BN, int WM, int WN, int NHL, int MOST = 4>
 struct BfCfg {
   static constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN, NT = NW * 64;
   static constexpr int FM = WM / 32, FN = WN / 32;
@@ -226,7 +227,7 @@ struct BfCfg {
   static constexpr int CH_B = BN / 32 * KB * NHL * 64;
   static constexpr int PER_A = CH_A / NT, PER_B = CH_B / NT;
   static constexpr int FIT = 160 * 1024 / (16 * (CH_A + CH_B));
-  static constexpr int NB = FIT < 4 ? FIT : 4;
+  static constexpr int NB = FIT < MOST ? FIT : MOST;
   static constexpr int SMEM_CHUNKS = NB * (CH_A + CH_B);
   static_assert(CH_A % NT == 0 && CH_B % NT == 0, "stage must split evenly");
   static_assert(KB % 2 == 0 && NB >= 2, "fragment sets alternate over an even number of k blocks");
@@ -316,10 +317,10 @@ __device__ __forceinline__ void zero_acc(floatx16 (&acc)[FM][FN]) {
 // read when needed: N = 8192 split BF16 2.48 -> 2.12 ms (1331 -> 1555
 // TFLOP/s), single BF16 0.947 -> 0.796 ms; 1024 x 1024 x 4096 split BF16 on
 // 64x64 tiles 75.7 -> 31.6 us.
-template <int BM, int BN, int WM, int WN, int NHL>
+template <int BM, int BN, int WM, int WN, int NHL, int MOST = 4>
 __device__ __forceinline__ void bf16_tile(const BfTileArgs& t, int tm, int tn, int s0, int s1, const Epilogue& ep,
     int er, int ec, u32x4* lds) {
-  using Cfg = BfCfg<BM, BN, WM, WN, NHL>;
+  using Cfg = BfCfg<BM, BN, WM, WN, NHL, MOST>;
   constexpr int NT = Cfg::NT, FM = Cfg::FM, FN = Cfg::FN, KB = Cfg::KB, NB = Cfg::NB;
   constexpr int SA = Cfg::CH_A, STAGE = Cfg::CH_A + Cfg::CH_B;
   constexpr int PER = Cfg::PER_A + Cfg::PER_B;  // DMA instructions per stage and wave
