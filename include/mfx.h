@@ -17,6 +17,17 @@
  *   - Functions return an mfx_status; nothing throws or aborts across the ABI.
  *   - A handle must not be used from two host threads at once; distinct
  *     handles are independent.
+ *   - One handle's FP32 calls may run on several streams at once: split-K
+ *     partial tiles have a buffer per stream (32 MiB, allocated at the first
+ *     split call of a stream, for at most 8 streams; further streams run
+ *     unsplit).  Exceptions, as they use the handle's workspace: the packed
+ *     precisions, covariance / correlation and grouped launches, whose calls on
+ *     several streams the caller orders; and FP32 products on few tiles (at most
+ *     one for two CUs) where the stream has no buffer.
+ *   - A call may be captured into the caller's graph if the workspace holds what
+ *     it needs beforehand.  FP32 calls then run unsplit and hold no library
+ *     memory, but for products on few tiles, whose slices a large enough
+ *     workspace keeps.
  */
 #ifndef MFX_H
 #define MFX_H
@@ -62,7 +73,8 @@ mfx_status mfx_destroy(mfx_handle handle);
 mfx_status mfx_reserve_workspace(mfx_handle handle, size_t bytes);
 /* Workspace bytes a gemm of this shape and precision needs under the
  * automatic choices on the current device (packed operands; split-K partial
- * tiles of a grid that does not fill the CUs, at most 32 MiB). */
+ * tiles, at most 32 MiB, which calls outside a capture keep per stream
+ * instead where the precision is FP32). */
 size_t mfx_gemm_workspace_size(mfx_precision prec, int64_t m, int64_t n, int64_t k);
 /*
  * Host-only pre-flight check (no handle, no device): the status mfx_gemm

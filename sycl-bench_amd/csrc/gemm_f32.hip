@@ -132,20 +132,84 @@ size_t partial_bytes(const SplitPlan& plan, int64_t tiles, const F32Config& c) {
   return plan.splits > 1 ? (size_t)(tiles - plan.head) * plan.splits * c.bm * c.bn * sizeof(float) : 0;
 }
 
-}  // namespace
-
 // Whether re-tiling a triangle's last round is estimated shorter than the
 // split plan of the same configuration.
-static bool tri_tail_wins(const DenseOp& op, int config, const TriTail& tail, int tiles, int cus) {
+bool tri_tail_wins(const DenseOp& op, int config, const TriTail& tail, int tiles, int cus) {
   const int64_t k = (int64_t)ceil_div(op.K, F32_BK) * F32_BK * op.nprod;
   const double retiled = tile_span(MFX_PREC_FP32, config, tail.head, k, cus) +
                          tile_span(MFX_PREC_FP32, tail.small, (int64_t)(tiles - tail.head) * tail.ratio * tail.ratio, k, cus);
   return retiled < plan_splits(MFX_PREC_FP32, config, tiles, k, cus, kMaxPartialBytes, nullptr);
 }
 
+// How a call runs on one configuration: k slices, or a triangle's re-tiled last
+// round (tail.small >= 0, the plan then whole), or neither.
+struct F32Call {
+  SplitPlan plan;
+  TriTail tail;
+  size_t partial = 0;  // bytes of partial tiles
+};
+
+F32Call f32_call(const DenseOp& op, int config, int cus, int forced_splits) {
+  F32Call c;
+  const int tiles = (int)f32_tiles(op, config);
+  c.plan = f32_split_plan(op, config, cus, forced_splits);
+  if(op.tiles != TILES_FULL && forced_splits < 2) {
+    c.tail = tri_tail(MFX_PREC_FP32, config, ceil_div(op.M, kF32Configs[config].bm), cus);
+    if(c.tail.small >= 0 && (c.plan.splits == 1 || tri_tail_wins(op, config, c.tail, tiles, cus)))
+      c.plan = SplitPlan{c.tail.head, 1};
+    else
+      c.tail.small = -1;
+  }
+  c.partial = partial_bytes(c.plan, tiles, kF32Configs[config]);
+  return c;
+}
+
+mfx_status run_f32(Handle* h, const DenseOp& op, int config, const F32Call& call, void* partial, hipStream_t s) {
+  const F32Config& c = kF32Configs[config];
+  F32Params p;
+  p.op = op;
+  p.tiles_m = (int)ceil_div(op.M, c.bm);
+  p.tiles_n = (int)ceil_div(op.N, c.bn);
+  p.group = 8;
+  // a second product swaps the operands: one load width for both
+  const bool vec = f32_vec_ok(op.A, op.lda, op.a_kmajor, op.M, op.K) && f32_vec_ok(op.B, op.ldb, op.b_kmajor, op.N, op.K);
+  if(op.tiles != TILES_FULL && (op.M != op.N || c.bm != c.bn)) return invalid("triangular schedule needs square tiles");
+  p.tiles = (int)f32_tiles(op, config);
+  if(p.tiles == 0) return MFX_SUCCESS;
+  p.plan = call.plan;
+  p.partial = static_cast<float*>(partial);
+  if(call.tail.small >= 0) {
+    // the full rounds on this tile, the last round's big tiles re-tiled
+    const TriTail& tail = call.tail;
+    MFX_CHECK(launch_f32_config(h, p, vec, config, tail.head, s));
+    F32Params q = p;
+    q.tiles_m = q.tiles_n = (int)ceil_div(op.M, kF32Configs[tail.small].bm);
+    q.tail_first = tail.head;
+    q.tail_ratio = tail.ratio;
+    q.big_tiles = p.tiles_m;
+    q.plan.head = (p.tiles - tail.head) * tail.ratio * tail.ratio;
+    return launch_f32_config(h, q, vec, tail.small, q.plan.head, s);
+  }
+  const int grid = p.plan.head + (p.tiles - p.plan.head) * p.plan.splits;
+  MFX_CHECK(launch_f32_config(h, p, vec, config, grid, s));
+  if(p.plan.splits == 1) return MFX_SUCCESS;
+  const SplitReduceArgs r{p.partial, c.bm, c.bn, p.plan.splits, p.plan.head, p.tiles, op.tiles, p.tiles_m, p.tiles_n,
+      p.group, op.ep};
+  return launch_splitk_reduce(h, r, s);
+}
+
+// Full single products on at most one tile for every two CUs, which lose most
+// unsplit: the ones that may keep their partial tiles in the handle's workspace
+// where the stream has no buffer of its own.
+bool few_tiles(const DenseOp& op, int config, int cus) {
+  return op.tiles == TILES_FULL && op.nprod == 1 && kF32Configs[config].bm <= 128 && 2 * f32_tiles(op, config) <= cus;
+}
+
+}  // namespace
+
 size_t dense_f32_workspace(const DenseOp& op, int config, int cus, int forced_splits) {
   if(config < 0 || config >= kF32ConfigCount) return 0;
-  return partial_bytes(f32_split_plan(op, config, cus, forced_splits), f32_tiles(op, config), kF32Configs[config]);
+  return f32_call(op, config, cus, forced_splits).partial;
 }
 
 int f32_config_count() { return kF32ConfigCount; }
@@ -159,53 +223,26 @@ bool f32_config_info(int c, int* bm, int* bn, int* bk, int* waves) {
 }
 
 mfx_status launch_dense_f32(Handle* h, const DenseOp& op, int config, hipStream_t s) {
-  return launch_dense_f32_ws(h, op, config, nullptr, 0, s);
+  if(config < 0 || config >= kF32ConfigCount) return invalid("FP32 tile configuration out of range");
+  F32Call call = f32_call(op, config, cus_of(h), h->forced_splits);
+  void* partial = nullptr;
+  if(call.partial > 0) {
+    partial = stream_partials(h, s);
+    if(!partial && few_tiles(op, config, cus_of(h)) && (!is_capturing(h, s) || call.partial <= h->workspace_bytes))
+      MFX_CHECK(workspace(h, call.partial, &partial));
+    if(!partial) {
+      config = whole_config(h, MFX_PREC_FP32, op, config);
+      call = f32_call(op, config, cus_of(h), 1);
+    }
+  }
+  return run_f32(h, op, config, call, partial, s);
 }
 
 mfx_status launch_dense_f32_ws(Handle* h, const DenseOp& op, int config, void* ws, size_t ws_bytes, hipStream_t s) {
   if(config < 0 || config >= kF32ConfigCount) return invalid("FP32 tile configuration out of range");
-  const F32Config& c = kF32Configs[config];
-  F32Params p;
-  p.op = op;
-  p.tiles_m = (int)ceil_div(op.M, c.bm);
-  p.tiles_n = (int)ceil_div(op.N, c.bn);
-  p.group = 8;
-  // a second product swaps the operands: one load width for both
-  const bool vec = f32_vec_ok(op.A, op.lda, op.a_kmajor, op.M, op.K) && f32_vec_ok(op.B, op.ldb, op.b_kmajor, op.N, op.K);
-  if(op.tiles != TILES_FULL && (op.M != op.N || c.bm != c.bn)) return invalid("triangular schedule needs square tiles");
-  p.tiles = (int)f32_tiles(op, config);
-  if(p.tiles == 0) return MFX_SUCCESS;
-  p.plan = f32_split_plan(op, config, cus_of(h), h->forced_splits);
-  if(op.tiles != TILES_FULL && h->forced_splits < 2) {
-    const TriTail tail = tri_tail(MFX_PREC_FP32, config, p.tiles_m, cus_of(h));
-    if(tail.small >= 0 && (p.plan.splits == 1 || tri_tail_wins(op, config, tail, p.tiles, cus_of(h)))) {
-      // the full rounds on this tile, the last round's big tiles re-tiled
-      p.plan = SplitPlan{tail.head, 1};
-      MFX_CHECK(launch_f32_config(h, p, vec, config, tail.head, s));
-      F32Params q = p;
-      q.tiles_m = q.tiles_n = (int)ceil_div(op.M, kF32Configs[tail.small].bm);
-      q.tail_first = tail.head;
-      q.tail_ratio = tail.ratio;
-      q.big_tiles = p.tiles_m;
-      q.plan.head = (p.tiles - tail.head) * tail.ratio * tail.ratio;
-      return launch_f32_config(h, q, vec, tail.small, q.plan.head, s);
-    }
-  }
-  if(p.plan.splits > 1) {
-    const size_t need = partial_bytes(p.plan, p.tiles, c);
-    if(ws) {
-      if(need > ws_bytes) return unsupported("split-K partial tiles exceed the given buffer");
-    } else {
-      MFX_CHECK(workspace(h, need, &ws));
-    }
-    p.partial = static_cast<float*>(ws);
-  }
-  const int grid = p.plan.head + (p.tiles - p.plan.head) * p.plan.splits;
-  MFX_CHECK(launch_f32_config(h, p, vec, config, grid, s));
-  if(p.plan.splits == 1) return MFX_SUCCESS;
-  const SplitReduceArgs r{p.partial, c.bm, c.bn, p.plan.splits, p.plan.head, p.tiles, op.tiles, p.tiles_m, p.tiles_n,
-      p.group, op.ep};
-  return launch_splitk_reduce(h, r, s);
+  const F32Call call = f32_call(op, config, cus_of(h), h->forced_splits);
+  if(call.partial > ws_bytes) return unsupported("split-K partial tiles exceed the given buffer");
+  return run_f32(h, op, config, call, ws, s);
 }
 
 }  // namespace mfx

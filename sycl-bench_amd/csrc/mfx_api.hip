@@ -87,6 +87,37 @@ mfx_status workspace(Handle* h, size_t bytes, void** out) {
   return MFX_SUCCESS;
 }
 
+bool is_capturing(const Handle* h, hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if(h->capturing) return true;
+  if(hipStreamIsCapturing(s, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // the null stream while another one captures
+  return true;
+}
+
+void* stream_partials(Handle* h, hipStream_t s) {
+  if(s == hipStreamPerThread || is_capturing(h, s)) return nullptr;
+  for(int i = 0; i < h->partial_streams; ++i)
+    if(h->partials[i].stream == s) return h->partials[i].p;
+  if(h->partial_streams == Handle::kPartialStreams) return nullptr;
+  // an allocation on this stream is no part of a capture on another one
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if(hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  void* p = nullptr;
+  const hipError_t e = hipMalloc(&p, (size_t)kMaxPartialBytes);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if(e != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  h->partials[h->partial_streams].stream = s;
+  h->partials[h->partial_streams++].p = p;
+  return p;
+}
+
 int config_count(mfx_precision p) {
   switch(p) {
     case MFX_PREC_FP32: return f32_config_count();
@@ -159,13 +190,13 @@ double config_rate(mfx_precision p, int c) {
 // Used when nothing is tuned: the configuration whose estimated launch
 // (tile_span's measured model, with the k slices plan_splits or the smaller
 // tiles tri_tail would give a sparse last round) is shortest.
-int heuristic_config(Handle* h, mfx_precision p, int64_t m, int64_t n, int64_t k) {
+int heuristic_config(Handle* h, mfx_precision p, int64_t m, int64_t n, int64_t k, int64_t max_partial = kMaxPartialBytes) {
   int best = 0;
   double best_t = -1.0;
   for(int c = 0; c < config_count(p); ++c) {
     int bm, bn, bk, w;
     if(!config_info(p, c, &bm, &bn, &bk, &w)) continue;
-    const double t = plan_splits(p, c, ceil_div(m, bm) * ceil_div(n, bn), k, cus_of(h), kMaxPartialBytes, nullptr);
+    const double t = plan_splits(p, c, ceil_div(m, bm) * ceil_div(n, bn), k, cus_of(h), max_partial, nullptr);
     if(best_t < 0.0 || t < best_t) {
       best = c;
       best_t = t;
@@ -224,7 +255,8 @@ TriTail tri_tail(mfx_precision p, int config, int64_t T, int cus) {
 }
 
 // The same over the square configurations for an n x n triangle.
-static int heuristic_square_config(Handle* h, mfx_precision p, int64_t n, int64_t k) {
+static int heuristic_square_config(Handle* h, mfx_precision p, int64_t n, int64_t k,
+    int64_t max_partial = kMaxPartialBytes) {
   const int cus = cus_of(h);
   int best = 0;
   double best_t = -1.0;
@@ -232,7 +264,7 @@ static int heuristic_square_config(Handle* h, mfx_precision p, int64_t n, int64_
     int bm, bn, bk, w;
     if(!config_info(p, c, &bm, &bn, &bk, &w) || bm != bn) continue;
     const int64_t T = ceil_div(n, bm), tiles = T * (T + 1) / 2;
-    double t = plan_splits(p, c, tiles, k, cus, kMaxPartialBytes, nullptr);
+    double t = plan_splits(p, c, tiles, k, cus, max_partial, nullptr);
     if(p == MFX_PREC_FP32) {
       const TriTail tail = tri_tail(p, c, T, cus);
       if(tail.small >= 0)
@@ -261,6 +293,12 @@ int choose_square_config(Handle* h, mfx_precision p, int64_t n, int64_t k) {
   int bm, bn, bk, w;
   if(c >= 0) return config_info(p, c, &bm, &bn, &bk, &w) && bm == bn ? c : 0;
   return heuristic_square_config(h, p, n, k);
+}
+
+int whole_config(Handle* h, mfx_precision p, const DenseOp& op, int config) {
+  const int64_t k = (int64_t)op.K * op.nprod;
+  if(h->forced_config[p] >= 0 || tuned_lookup(tune_key(p, op.M, op.N, k)) >= 0) return config;
+  return op.tiles == TILES_FULL ? heuristic_config(h, p, op.M, op.N, k, 0) : heuristic_square_config(h, p, op.N, k, 0);
 }
 
 mfx_status dispatch_dense(Handle* h, mfx_precision prec, DenseOp& op, int config, hipStream_t s) {
@@ -393,6 +431,7 @@ mfx_status mfx_destroy(mfx_handle handle) {
   }
   for(auto e : h->free_events) keep(hipEventDestroy(e));
   if(h->workspace) keep(hipFree(h->workspace));
+  for(int i = 0; i < h->partial_streams; ++i) keep(hipFree(h->partials[i].p));
   if(h->staging) keep(hipHostFree(h->staging));
   if(h->staging_ready) keep(hipEventDestroy(h->staging_ready));
   if(h->error_flag) keep(hipFree(h->error_flag));

@@ -69,6 +69,13 @@ struct Handle {
   int* error_flag = nullptr;
   bool grouped_waits = true;  // the last grouped call launched kernels that can time out
   int forced_splits = -1;  // split-K: -1 automatic, 1 never, >= 2 that many slices
+  // split-K partial tiles, one buffer of kMaxPartialBytes per stream (stream_partials)
+  static constexpr int kPartialStreams = 8;
+  struct {
+    hipStream_t stream;
+    void* p;
+  } partials[kPartialStreams] = {};
+  int partial_streams = 0;
 };
 
 inline int cus_of(const Handle* h) { return h->cu_count > 0 ? h->cu_count : 256; }
@@ -80,6 +87,18 @@ mfx_status noalloc_init(int device);
 // Returns a workspace pointer of at least `bytes` (grows the arena; growing
 // synchronises the device, so it must not happen under graph capture).
 mfx_status workspace(Handle* h, size_t bytes, void** out);
+
+// Stream s's own buffer of kMaxPartialBytes for split-K partial tiles, allocated
+// at its first use and kept until mfx_destroy, so that two streams' calls on one
+// handle do not meet in it and no later call moves it (a stream whose value an
+// ended one had before finds it idle: hipStreamDestroy waits for the work). Null where there is none
+// (the caller then runs unsplit): the stream is being captured, whose graph may
+// replay beside anything; it is hipStreamPerThread, one value for several
+// streams; kPartialStreams others hold one; or the memory is not to be had.
+void* stream_partials(Handle* h, hipStream_t s);
+
+// Whether a call on s is being captured into a caller's or the library's graph.
+bool is_capturing(const Handle* h, hipStream_t s);
 
 // Records an event pair around `launch()` when timing is on, and converts a
 // launch error into MFX_ERROR_HIP.
@@ -464,7 +483,7 @@ TriTail tri_tail(mfx_precision p, int config, int64_t tiles_per_side, int cus);
 
 mfx_status launch_dense_f32(Handle* h, const DenseOp& op, int config, hipStream_t s);
 // The same with split-K partial tiles in `ws` (ws_bytes long) instead of the
-// handle's workspace; fails if a split this call makes needs more.
+// stream's buffer; fails if a split this call makes needs more.
 mfx_status launch_dense_f32_ws(Handle* h, const DenseOp& op, int config, void* ws, size_t ws_bytes, hipStream_t s);
 size_t dense_f32_workspace(const DenseOp& op, int config, int cus, int forced_splits);
 mfx_status launch_dense_bf16x(Handle* h, const DenseOp& op, bool split, int config, hipStream_t s);
@@ -481,6 +500,9 @@ struct SplitReduceArgs {
 };
 mfx_status launch_splitk_reduce(Handle* h, const SplitReduceArgs& a, hipStream_t s);
 constexpr int64_t kMaxPartialBytes = (int64_t)32 << 20;
+// The configuration for `op` without k slices, in place of `config` (chosen with
+// them): `config` itself where it was forced or tuned.
+int whole_config(Handle* h, mfx_precision p, const DenseOp& op, int config);
 // Estimated microseconds of a dense launch on `config` (tile_cost's model)
 // and the split plan behind it; partial tiles take at most max_partial bytes.
 // Estimated microseconds of `count` workgroups of `len` k each (no split).
