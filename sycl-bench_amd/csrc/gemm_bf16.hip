@@ -221,23 +221,15 @@ size_t dense_bf16x_workspace(const DenseOp& op, bool split, int config, int cus,
   return pl.bytes_a + pl.bytes_b + pl.bytes_partial;
 }
 
-mfx_status launch_dense_bf16x(Handle* h, const DenseOp& op, bool split, int config, hipStream_t s) {
-  if(config < 0 || config >= kBfConfigCount) return invalid("BF16 tile configuration out of range");
-  if(op.M == 0 || op.N == 0) return MFX_SUCCESS;
-  void* ws = nullptr;
-  MFX_CHECK(workspace(h, dense_bf16x_workspace(op, split, config, cus_of(h), h->forced_splits), &ws));
-  return launch_dense_bf16x_ws(h, op, split, config, ws, s);
-}
+namespace {
 
 // The pack kernels write every chunk of both padded panels (zeros past the
 // matrix) and the slices every partial tile, so `ws` needs no clearing and
 // may hold anything on entry.
-mfx_status launch_dense_bf16x_ws(Handle* h, const DenseOp& op, bool split, int config, void* ws, hipStream_t s) {
-  if(config < 0 || config >= kBfConfigCount) return invalid("BF16 tile configuration out of range");
+mfx_status run_bf16x(Handle* h, const DenseOp& op, bool split, int config, const PackPlan& pl, void* ws, void* partials,
+    hipStream_t s) {
   const BfConfig& c = kBfConfigs[config];
-  if(op.M == 0 || op.N == 0) return MFX_SUCCESS;
   const int nhl = split ? 2 : 1;
-  const PackPlan pl = plan(op, split, config, cus_of(h), h->forced_splits);
   const bool same = op.A == op.B && op.lda == op.ldb && op.a_kmajor == op.b_kmajor && op.M == op.N &&
                     pl.rows_pad_a == pl.rows_pad_b;
   if(op.nprod == 2 && pl.rows_pad_a != pl.rows_pad_b) return invalid("two-product form needs equal operand shapes");
@@ -263,13 +255,37 @@ mfx_status launch_dense_bf16x_ws(Handle* h, const DenseOp& op, bool split, int c
   p.mode = op.tiles;
   p.plan = pl.split;
   p.tiles = (int)pl.tiles;
-  p.partial = reinterpret_cast<float*>(w + pl.bytes_a + pl.bytes_b);
+  p.partial = static_cast<float*>(partials);
   const int grid = p.plan.head + (p.tiles - p.plan.head) * p.plan.splits;
   MFX_CHECK(launch_bf_config(h, p, split, config, grid, s));
   if(p.plan.splits == 1) return MFX_SUCCESS;
   const SplitReduceArgs r{p.partial, c.bm, c.bn, p.plan.splits, p.plan.head, p.tiles, p.mode, p.tiles_m, p.tiles_n,
       p.group, op.ep};
   return launch_splitk_reduce(h, r, s);
+}
+
+}  // namespace
+
+mfx_status launch_dense_bf16x(Handle* h, const DenseOp& op, bool split, int config, hipStream_t s) {
+  if(config < 0 || config >= kBfConfigCount) return invalid("BF16 tile configuration out of range");
+  if(op.M == 0 || op.N == 0) return MFX_SUCCESS;
+  PackPlan pl = plan(op, split, config, cus_of(h), h->forced_splits);
+  void *ws = nullptr, *partials = nullptr;
+  MFX_CHECK(packed_workspace(h, pl.bytes_a + pl.bytes_b, pl.bytes_partial, s, &ws, &partials));
+  if(pl.bytes_partial > 0 && !partials) {
+    config = whole_config(h, split ? MFX_PREC_SPLIT_BF16 : MFX_PREC_BF16, op, config);
+    pl = plan(op, split, config, cus_of(h), 1);
+  }
+  return run_bf16x(h, op, split, config, pl, ws, partials, s);
+}
+
+mfx_status launch_dense_bf16x_ws(Handle* h, const DenseOp& op, bool split, int config, void* ws, hipStream_t s,
+    void* partials) {
+  if(config < 0 || config >= kBfConfigCount) return invalid("BF16 tile configuration out of range");
+  if(op.M == 0 || op.N == 0) return MFX_SUCCESS;
+  const PackPlan pl = plan(op, split, config, cus_of(h), h->forced_splits);
+  if(!partials) partials = static_cast<char*>(ws) + pl.bytes_a + pl.bytes_b;
+  return run_bf16x(h, op, split, config, pl, ws, partials, s);
 }
 
 // Element-wise split used by mfx_split_bf16 (a test and tooling utility).

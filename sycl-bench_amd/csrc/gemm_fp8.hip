@@ -580,23 +580,29 @@ bool fp8_config_info(int c, int* bm, int* bn, int* bk, int* waves) {
   return true;
 }
 
-static size_t fp8_workspace(const Fp8Plan& pl, bool two_term) {
+// Bytes of the packed operands and their exponents.
+static size_t fp8_packed(const Fp8Plan& pl, bool two_term) {
   const int terms = two_term ? 2 : 1;
-  return terms * (round_up(pl.q_a, 256) + round_up(pl.q_b, 256) + round_up(pl.e_a, 256) + round_up(pl.e_b, 256)) + pl.partial;
+  return terms * (round_up(pl.q_a, 256) + round_up(pl.q_b, 256) + round_up(pl.e_a, 256) + round_up(pl.e_b, 256));
 }
 
 size_t dense_fp8_workspace(const DenseOp& op, bool two_term, int config, int cus) {
   if(config < 0 || config >= kFp8ConfigCount) return 0;
-  return fp8_workspace(fp8_plan(op, two_term, config, cus, -1), two_term);
+  const Fp8Plan pl = fp8_plan(op, two_term, config, cus, -1);
+  return fp8_packed(pl, two_term) + pl.partial;
 }
 
 mfx_status launch_dense_fp8(Handle* h, const DenseOp& op, bool two_term, int config, hipStream_t s) {
   if(config < 0 || config >= kFp8ConfigCount) return invalid("FP8 tile configuration out of range");
   if(op.nprod != 1 || op.tiles != TILES_FULL) return unsupported("FP8 is built for plain gemm (not syrk / syr2k)");
   if(op.M == 0 || op.N == 0) return MFX_SUCCESS;
-  const Fp8Plan pl = fp8_plan(op, two_term, config, cus_of(h), h->forced_splits);
-  void* ws = nullptr;
-  MFX_CHECK(workspace(h, fp8_workspace(pl, two_term), &ws));
+  Fp8Plan pl = fp8_plan(op, two_term, config, cus_of(h), h->forced_splits);
+  void *ws = nullptr, *partials = nullptr;
+  MFX_CHECK(packed_workspace(h, fp8_packed(pl, two_term), pl.partial, s, &ws, &partials));
+  if(pl.partial > 0 && !partials) {
+    config = whole_config(h, two_term ? MFX_PREC_FP8_BLOCK2 : MFX_PREC_FP8_BLOCK, op, config);
+    pl = fp8_plan(op, two_term, config, cus_of(h), 1);
+  }
   char* w = static_cast<char*>(ws);
   auto take = [&](size_t bytes) {
     char* p = w;
@@ -632,7 +638,7 @@ mfx_status launch_dense_fp8(Handle* h, const DenseOp& op, bool two_term, int con
   p.tiles_n = (int)ceil_div(op.N, c.bn);
   p.group = 8;
   p.plan = pl.split;
-  p.partial = reinterpret_cast<float*>(w);
+  p.partial = static_cast<float*>(partials);
   p.ep = op.ep;
   const int grid = p.plan.head + ((int)pl.tiles - p.plan.head) * p.plan.splits;
   MFX_CHECK(timed_launch(h, two_term ? "gemm_fp8_block2_mfma" : "gemm_fp8_block_mfma", s, [&] {

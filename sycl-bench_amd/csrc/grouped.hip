@@ -964,7 +964,7 @@ static mfx_status launch_grouped_kernels(Handle* h, const GroupedPlan& pl, const
 struct DenseList {
   std::vector<DenseOp> ops;  // empty: the grouped launch is estimated shorter
   std::vector<int> config;
-  size_t bytes = 0;  // workspace, shared by the problems in turn
+  size_t packed = 0, partial = 0;  // bytes of packed operands and partial tiles, shared by the problems in turn
 };
 constexpr int kDenseListMax = 16;
 // Uploading the tables, clearing the counters and the first item of a grouped
@@ -1005,8 +1005,10 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
     op.ep = Epilogue{q.C, q.ldc, q.alpha, q.beta, (int)q.m, (int)q.n, TILES_FULL, 0};
     d.ops.push_back(op);
     d.config.push_back(c);
-    d.bytes = std::max(d.bytes, packed ? dense_bf16x_workspace(op, split, c, cus, h->forced_splits)
-                                       : dense_f32_workspace(op, c, cus, h->forced_splits));
+    size_t partial = 0;
+    if(packed) d.packed = std::max(d.packed, dense_bf16x_workspace(op, split, c, cus, h->forced_splits, &partial) - partial);
+    else partial = dense_f32_workspace(op, c, cus, h->forced_splits);
+    d.partial = std::max(d.partial, partial);
   }
   const auto level = problem_levels(count, deps, ndeps);
   const double grouped = kGroupedFixedUs + policy_estimate(kPolicies[pl.policy], prec, problems, count, level,
@@ -1018,10 +1020,10 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
   return d;
 }
 
-mfx_status launch_dense_list(Handle* h, mfx_precision prec, const DenseList& d, void* ws, hipStream_t s) {
+mfx_status launch_dense_list(Handle* h, mfx_precision prec, const DenseList& d, void* ws, void* partials, hipStream_t s) {
   for(size_t i = 0; i < d.ops.size(); ++i) {
-    if(prec == MFX_PREC_FP32) MFX_CHECK(launch_dense_f32_ws(h, d.ops[i], d.config[i], ws, d.bytes, s));
-    else MFX_CHECK(launch_dense_bf16x_ws(h, d.ops[i], prec == MFX_PREC_SPLIT_BF16, d.config[i], ws, s));
+    if(prec == MFX_PREC_FP32) MFX_CHECK(launch_dense_f32_ws(h, d.ops[i], d.config[i], partials, d.partial, s));
+    else MFX_CHECK(launch_dense_bf16x_ws(h, d.ops[i], prec == MFX_PREC_SPLIT_BF16, d.config[i], ws, s, partials));
   }
   return MFX_SUCCESS;
 }
@@ -1033,11 +1035,12 @@ mfx_status run_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* pr
   void* ws = nullptr;
   const DenseList dense = dense_list(h, prec, problems, count, deps, ndeps, pl);
   h->grouped_waits = true;
-  if(!dense.ops.empty()) {
-    // packed operands that do not fit: the grouped kernels need none
-    if(dense.bytes == 0 || workspace(h, dense.bytes, &ws) == MFX_SUCCESS) {
+  if(!dense.ops.empty() && !is_capturing(h, s)) {
+    // memory that is not to be had: the grouped kernels need less
+    void* partials = dense.partial > 0 ? stream_partials(h, s) : nullptr;
+    if((partials || dense.partial == 0) && (dense.packed == 0 || list_workspace(h, dense.packed, &ws) == MFX_SUCCESS)) {
       h->grouped_waits = false;
-      return launch_dense_list(h, prec, dense, ws, s);
+      return launch_dense_list(h, prec, dense, ws, partials, s);
     }
     (void)hipGetLastError();
   }
@@ -1178,7 +1181,7 @@ mfx_status mfx_grouped_graph_create(mfx_handle handle, mfx_precision prec, const
   // The graph owns its tables, counters and packed operands, so later calls on
   // the handle (which may regrow the handle's workspace) cannot move them.
   DenseList dense = dense_list(h, prec, problems, count, deps, ndeps, pl);
-  hipError_t ae = hipMalloc(&gr->mem, std::max<size_t>(dense.ops.empty() ? pl.total_bytes : dense.bytes, 256));
+  hipError_t ae = hipMalloc(&gr->mem, std::max<size_t>(dense.ops.empty() ? pl.total_bytes : dense.packed + dense.partial, 256));
   if(ae != hipSuccess && !dense.ops.empty()) {
     (void)hipGetLastError();
     dense.ops.clear();
@@ -1212,7 +1215,8 @@ mfx_status mfx_grouped_graph_create(mfx_handle handle, mfx_precision prec, const
   mfx_status st = MFX_SUCCESS;
   hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
   if(e == hipSuccess) {
-    st = dense.ops.empty() ? launch_grouped_kernels(h, pl, g, cs) : launch_dense_list(h, prec, dense, gr->mem, cs);
+    st = dense.ops.empty() ? launch_grouped_kernels(h, pl, g, cs) : launch_dense_list(h, prec, dense, gr->mem,
+                                                                          static_cast<char*>(gr->mem) + dense.packed, cs);
     hipError_t e2 = hipStreamEndCapture(cs, &gr->graph);
     if(st == MFX_SUCCESS && e2 != hipSuccess) st = hip_fail(e2, "hipStreamEndCapture");
   } else {

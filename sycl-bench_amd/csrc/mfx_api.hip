@@ -65,25 +65,38 @@ hipEvent_t take_event(Handle* h) {
   return e;
 }
 
-mfx_status workspace(Handle* h, size_t bytes, void** out) {
-  if(bytes <= h->workspace_bytes && h->workspace) {
-    *out = h->workspace;
+static mfx_status grow(Handle* h, void** memory, size_t* held, size_t bytes, void** out) {
+  if(bytes <= *held && *memory) {
+    *out = *memory;
     return MFX_SUCCESS;
   }
   if(h->capturing) return invalid("workspace must be reserved before graph capture");
-  if(h->workspace) {
+  if(*memory) {
     MFX_HIP(hipDeviceSynchronize());
-    MFX_HIP(hipFree(h->workspace));
-    h->workspace = nullptr;
-    h->workspace_bytes = 0;
+    MFX_HIP(hipFree(*memory));
+    *memory = nullptr;
+    *held = 0;
   }
   const size_t want = (size_t)round_up((int64_t)bytes, 1 << 21);
   void* p = nullptr;
   hipError_t e = hipMalloc(&p, want);
   if(e != hipSuccess) return hip_fail(e, "hipMalloc(workspace)");
-  h->workspace = p;
-  h->workspace_bytes = want;
+  *memory = p;
+  *held = want;
   *out = p;
+  return MFX_SUCCESS;
+}
+
+mfx_status workspace(Handle* h, size_t bytes, void** out) { return grow(h, &h->workspace, &h->workspace_bytes, bytes, out); }
+
+mfx_status list_workspace(Handle* h, size_t bytes, void** out) { return grow(h, &h->list_memory, &h->list_bytes, bytes, out); }
+
+mfx_status packed_workspace(Handle* h, size_t packed, size_t partial, hipStream_t s, void** ws, void** partials) {
+  *partials = nullptr;
+  const bool behind = partial > 0 && h->workspace && packed + partial <= h->workspace_bytes;
+  if(partial > 0 && !behind) *partials = stream_partials(h, s);
+  MFX_CHECK(workspace(h, packed, ws));
+  if(behind) *partials = static_cast<char*>(*ws) + packed;
   return MFX_SUCCESS;
 }
 
@@ -431,6 +444,7 @@ mfx_status mfx_destroy(mfx_handle handle) {
   }
   for(auto e : h->free_events) keep(hipEventDestroy(e));
   if(h->workspace) keep(hipFree(h->workspace));
+  if(h->list_memory) keep(hipFree(h->list_memory));
   for(int i = 0; i < h->partial_streams; ++i) keep(hipFree(h->partials[i].p));
   if(h->staging) keep(hipHostFree(h->staging));
   if(h->staging_ready) keep(hipEventDestroy(h->staging_ready));

@@ -76,6 +76,9 @@ struct Handle {
     void* p;
   } partials[kPartialStreams] = {};
   int partial_streams = 0;
+  // packed operands of lists that run as dense launches (list_workspace)
+  void* list_memory = nullptr;
+  size_t list_bytes = 0;
 };
 
 inline int cus_of(const Handle* h) { return h->cu_count > 0 ? h->cu_count : 256; }
@@ -87,6 +90,10 @@ mfx_status noalloc_init(int device);
 // Returns a workspace pointer of at least `bytes` (grows the arena; growing
 // synchronises the device, so it must not happen under graph capture).
 mfx_status workspace(Handle* h, size_t bytes, void** out);
+// The same in memory of its own, which no caller's graph holds: a list that runs
+// as dense launches needs more than its tables, and must not regrow the
+// workspace that a captured call points into.
+mfx_status list_workspace(Handle* h, size_t bytes, void** out);
 
 // Stream s's own buffer of kMaxPartialBytes for split-K partial tiles, allocated
 // at its first use and kept until mfx_destroy, so that two streams' calls on one
@@ -96,6 +103,13 @@ mfx_status workspace(Handle* h, size_t bytes, void** out);
 // replay beside anything; it is hipStreamPerThread, one value for several
 // streams; kPartialStreams others hold one; or the memory is not to be had.
 void* stream_partials(Handle* h, hipStream_t s);
+
+// Memory of a packed call: *ws for its packed operands, *partials for its
+// partial tiles, behind them where the workspace already holds both, else the
+// stream's buffer, else null (none, or not to be had: the caller runs unsplit).
+// Partial tiles never regrow the workspace, so one that holds the packed operands
+// stays where a captured call found it.
+mfx_status packed_workspace(Handle* h, size_t packed, size_t partial, hipStream_t s, void** ws, void** partials);
 
 // Whether a call on s is being captured into a caller's or the library's graph.
 bool is_capturing(const Handle* h, hipStream_t s);
@@ -487,8 +501,10 @@ mfx_status launch_dense_f32(Handle* h, const DenseOp& op, int config, hipStream_
 mfx_status launch_dense_f32_ws(Handle* h, const DenseOp& op, int config, void* ws, size_t ws_bytes, hipStream_t s);
 size_t dense_f32_workspace(const DenseOp& op, int config, int cus, int forced_splits);
 mfx_status launch_dense_bf16x(Handle* h, const DenseOp& op, bool split, int config, hipStream_t s);
-// The same on a caller-provided workspace of dense_bf16x_workspace() bytes.
-mfx_status launch_dense_bf16x_ws(Handle* h, const DenseOp& op, bool split, int config, void* ws, hipStream_t s);
+// The same on a caller-provided workspace of dense_bf16x_workspace() bytes, or
+// with its partial tiles in `partials` and the packed operands alone in ws.
+mfx_status launch_dense_bf16x_ws(Handle* h, const DenseOp& op, bool split, int config, void* ws, hipStream_t s,
+    void* partials = nullptr);
 
 // Sums the partial tiles of a split launch and applies op's epilogue.
 struct SplitReduceArgs {

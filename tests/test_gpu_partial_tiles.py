@@ -1,14 +1,14 @@
 """Where split-K partial tiles live (GPU, through the C ABI): calls of one
 handle on several streams at once, calls captured into a caller's graph, on a
 fresh handle and with a reserved workspace. Bar: relative Frobenius error
-against FP64 on U[-1, 1) inputs, 2e-6 (FP32)."""
+against FP64 on U[-1, 1) inputs, 2e-6 (FP32) or 1e-5 / 1e-2 (split / single BF16)."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda"
-TOL = {"fp32": 2e-6}
+TOL = {"fp32": 2e-6, "split-bf16": 1e-5, "bf16": 1e-2}
 
 
 def seeded(h, rows, cols, mid):
@@ -135,5 +135,52 @@ def test_capture_of_few_tiles(mfx, handle, reserve):
         h.reserve_workspace(h.lib.mfx_gemm_workspace_size(mfx.FP32, m, n, k))
     g = captured(h, c)
     assert not reserve or torch.equal(c.C, eager)
+    del g
+    h.close()
+
+
+@pytest.mark.parametrize("prec,kind,n,k", [("split-bf16", "syr2k", 4096, 1024), ("split-bf16", "syr2k", 3000, 700),
+                                           ("split-bf16", "syrk", 3000, 2500), ("bf16", "syr2k", 3000, 2500)])
+def test_workspace_of_the_query_is_enough(mfx, handle, prec, kind, n, k):
+    """With the workspace that the product query names, the symmetric calls of the same sizes are captured,
+    and eager ones take no further memory than their stream's buffer."""
+    c = Call(handle, kind, prec, n, n, k, 0)
+    assert "splitk_reduce" in c.recorded(handle)
+    c.check()
+    h = mfx.Handle(0)
+    h.reserve_workspace(h.lib.mfx_gemm_workspace_size(mfx.PRECISIONS[prec], n, n, k))
+    others = [c, Call(handle, "syrk", prec, n, n, k, 4), Call(handle, "gemm", prec, n, n, k, 8)]
+    g = captured(h, c)
+    c.run(h)
+    for other in others:
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        other.run(h)
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free, other.kind
+        other.check()
+    del g
+    h.close()
+
+
+def test_captured_call_outlives_later_eager_calls(mfx, handle):
+    """A captured product's packed operands stay where they are while symmetric calls and lists of the same sizes run."""
+    n, k = 4096, 1024
+    c = Call(handle, "gemm", "split-bf16", n, n, k, 0)
+    two = Call(handle, "syr2k", "split-bf16", n, n, k, 4)
+    mats = [seeded(handle, 1024, 1024, 10 + i) for i in range(4)]
+    scratch, out = [torch.empty((1024, 1024), device=DEV) for _ in range(2)], torch.empty((1024, 1024), device=DEV)
+    c.run(handle)
+    h = mfx.Handle(0)
+    h.reserve_workspace(h.lib.mfx_gemm_workspace_size(mfx.SPLIT_BF16, n, n, k))
+    g = captured(h, c)
+    for _ in range(3):
+        two.run(h)
+        two.check()
+        h.chain(mats, scratch, out, prec="split-bf16")
+        c.C.fill_(float("nan"))
+        g.replay()
+        c.check()
+        assert rel(out, mats[0].double() @ mats[1].double() @ mats[2].double() @ mats[3].double()) < 2 * TOL["split-bf16"]
     del g
     h.close()
