@@ -251,6 +251,7 @@ struct GroupedPlan {
   const PackJob* dev_jobs = nullptr;          // the job table in device memory
   size_t total_bytes = 0;
   int policy = 0, big = 0, small = 0;  // tile policy and its configurations
+  double estimate = -1.0;              // microseconds estimated for it; -1: forced or tuned
   bool all_vec = true;                 // every problem allows 128-bit operand loads
   double flops = 0.0;
 };

@@ -2,9 +2,12 @@
 // grouped.h): planning, workspace binding, the tile policy, chains, the
 // hipGraph form and the C entry points.
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
+#include <memory>
 #include <numeric>
+#include <optional>
 #include <queue>
 
 #include "grouped.h"
@@ -13,6 +16,7 @@ namespace mfx {
 
 std::string tune_key(mfx_precision p, int64_t m, int64_t n, int64_t k);
 int tuned_lookup(const std::string& key);
+bool tuned_any();
 
 namespace {
 
@@ -92,13 +96,18 @@ int problem_config(const GroupedPolicy& pol, mfx_precision prec, int64_t m, int6
   return padded <= pol.bound * (double)m * (double)n ? big : small;
 }
 
-// Topological level of every problem (producers come first, so one pass).
+// Topological level of every problem. Producers come first in `problems`, so one
+// pass in consumer order; the pairs are sorted only where the caller's are not.
 std::vector<int> problem_levels(int count, const mfx_dep* deps, int ndeps) {
   std::vector<int> level(count, 0);
-  std::vector<std::vector<int>> prod(count);
-  for(int d = 0; d < ndeps; ++d) prod[deps[d].consumer].push_back(deps[d].producer);
-  for(int i = 0; i < count; ++i)
-    for(int p : prod[i]) level[i] = std::max(level[i], level[p] + 1);
+  auto by_consumer = [](const mfx_dep& a, const mfx_dep& b) { return a.consumer < b.consumer; };
+  std::vector<mfx_dep> sorted;
+  if(!std::is_sorted(deps, deps + ndeps, by_consumer)) {
+    sorted.assign(deps, deps + ndeps);
+    std::sort(sorted.begin(), sorted.end(), by_consumer);
+    deps = sorted.data();
+  }
+  for(int d = 0; d < ndeps; ++d) level[deps[d].consumer] = std::max(level[deps[d].consumer], level[deps[d].producer] + 1);
   return level;
 }
 
@@ -138,59 +147,173 @@ constexpr GroupedTileCost kGroupedSplit[7] = {{10.0, 100.0, 160.0}, {6.0, 38.0, 
 constexpr GroupedTileCost kGroupedBf16[7] = {{10.0, 70.0, 95.0}, {6.0, 27.0, 40.0}, {5.0, 17.0, 17.5}, {8.0, 42.0, 62.0},
                                              {10.0, 55.0, 80.0}, {8.0, 40.0, 58.0}, {4.0, 25.0, 38.0}};
 
-// busy: tiles per CU of the level
-double grouped_tile_us(mfx_precision prec, int c, int64_t k, double busy) {
-  const GroupedTileCost& t =
-      prec == MFX_PREC_FP32 ? kGroupedF32[c] : prec == MFX_PREC_SPLIT_BF16 ? kGroupedSplit[c] : kGroupedBf16[c];
-  const double x = std::min(1.0, std::max(0.0, (busy - 0.25) / 0.75));
-  // single BF16 64x64 tiles of packed problems fall behind 128x128 ones from
-  // about K = 256 on: eight chained products of 200 57 and 66 us, of 363 79 and 74
-  const double packed = c == 2 && prec == MFX_PREC_BF16 && k % 16 != 0 && k >= 256 ? 5.0 : 0.0;
-  return t.fixed + packed + 1e-3 * (t.idle + (t.full - t.idle) * x) * (double)std::max<int64_t>(k, 1);
+double ns_per_k(const GroupedTileCost& t, double busy) {  // busy: tiles per CU
+  return t.idle + (t.full - t.idle) * std::min(1.0, std::max(0.0, (busy - 0.25) / 0.75));
+}
+const GroupedTileCost& tile_cost(mfx_precision prec, int c) {
+  return prec == MFX_PREC_FP32 ? kGroupedF32[c] : prec == MFX_PREC_SPLIT_BF16 ? kGroupedSplit[c] : kGroupedBf16[c];
+}
+// Single BF16 64x64 tiles of packed problems fall behind 128x128 ones from
+// about K = 256 on: eight chained products of 200 57 and 66 us, of 363 79 and 74.
+constexpr double kPackedSmallUs = 5.0;
+bool packed_small(mfx_precision prec, int64_t k) { return prec == MFX_PREC_BF16 && k % 16 != 0 && k >= 256; }
+
+// The tiles that some problems take on one configuration: what their estimate
+// needs of them, so that no estimate walks the problems again.
+struct TileSums {
+  int64_t tiles = 0, packed = 0;  // packed: of problems with packed_small
+  double tiles_k = 0.0;           // K summed over the tiles
+  double kmin[2], kmax[2] = {-1.0, -1.0};  // of problems without and with packed_small
+  void add(int64_t n, double k, bool slow) {
+    kmin[slow] = kmax[slow] < 0.0 ? k : std::min(kmin[slow], k);
+    kmax[slow] = std::max(kmax[slow], k);
+    tiles += n;
+    packed += slow ? n : 0;
+    tiles_k += k * (double)n;
+  }
+  void add(const TileSums& o) {
+    for(int s = 0; s < 2; ++s) {
+      if(o.kmax[s] < 0.0) continue;
+      kmin[s] = kmax[s] < 0.0 ? o.kmin[s] : std::min(kmin[s], o.kmin[s]);
+      kmax[s] = std::max(kmax[s], o.kmax[s]);
+    }
+    tiles += o.tiles;
+    packed += o.packed;
+    tiles_k += o.tiles_k;
+  }
+};
+
+// Microseconds of all of these tiles on one CU, and of the longest and shortest
+// one (kept where `longest` / `shortest` are beyond it already).
+double sum_us(mfx_precision prec, int c, const TileSums& t, double busy, double* longest, double* shortest) {
+  if(t.tiles == 0) return 0.0;
+  const GroupedTileCost& cost = tile_cost(prec, c);
+  const double ns = ns_per_k(cost, busy), slow = c == 2 ? kPackedSmallUs : 0.0;
+  for(int s = 0; s < 2; ++s) {
+    if(t.kmax[s] < 0.0) continue;
+    const double fixed = cost.fixed + (s ? slow : 0.0);
+    *longest = std::max(*longest, fixed + 1e-3 * ns * t.kmax[s]);
+    *shortest = *shortest < 0.0 ? fixed + 1e-3 * ns * t.kmin[s] : std::min(*shortest, fixed + 1e-3 * ns * t.kmin[s]);
+  }
+  return cost.fixed * (double)t.tiles + slow * (double)t.packed + 1e-3 * ns * t.tiles_k;
 }
 
-// Estimated microseconds of the tiles of one level (level[i] == lv), problem i
-// on configuration of(i): whole rounds over the CUs where all tiles are alike,
-// else the work spread over the CUs plus a quarter of the longest tile.
-template <class Of>
-double level_estimate(mfx_precision prec, const mfx_gemm_problem* problems, int count, const std::vector<int>& level,
-    int lv, int cus, Of&& of) {
-  auto tiles_of = [&](int i) {
-    const auto& q = problems[i];
-    const int c = of(i);
-    return level[i] != lv || q.m <= 0 || q.n <= 0 ? (int64_t)0 : ceil_div(q.m, cfg_bm(c)) * ceil_div(q.n, cfg_bn(c));
-  };
-  int64_t tiles = 0;
-  for(int i = 0; i < count; ++i) tiles += tiles_of(i);
+// Estimated microseconds of one level's tiles on configuration a, and b: whole
+// rounds over the CUs where all tiles are alike, else the work spread over the
+// CUs plus a quarter of the longest tile.
+double level_estimate(mfx_precision prec, int a, const TileSums& ta, int b, const TileSums& tb, int cus) {
+  const int64_t tiles = ta.tiles + tb.tiles;
   if(tiles == 0) return 0.0;
-  double work = 0.0, longest = 0.0, shortest = -1.0;
-  for(int i = 0; i < count; ++i) {
-    const int64_t n = tiles_of(i);
-    if(n == 0) continue;
-    const double t = grouped_tile_us(prec, of(i), problems[i].k, (double)tiles / cus);
-    work += t * (double)n;
-    longest = std::max(longest, t);
-    shortest = shortest < 0.0 ? t : std::min(shortest, t);
-  }
+  double longest = 0.0, shortest = -1.0;
+  const double busy = (double)tiles / cus;
+  const double work = sum_us(prec, a, ta, busy, &longest, &shortest) + sum_us(prec, b, tb, busy, &longest, &shortest);
   if(longest <= shortest * 1.001) return (double)ceil_div(tiles, cus) * longest;
   return std::max(longest, work / cus + 0.25 * longest);
 }
 
-// The tile configuration that is estimated shortest when all of a level's
-// problems run it.
-int best_level_config(mfx_precision prec, const mfx_gemm_problem* problems, int count, const std::vector<int>& level,
-    int lv, int cus, double* us) {
-  int best = -1;
-  for(int c = 0; c < 7; ++c) {
-    if(grouped_config(prec, c) != c) continue;
-    const double t = level_estimate(prec, problems, count, level, lv, cus, [&](int) { return c; });
-    if(best < 0 || t < *us) {
-      best = c;
-      *us = t;
-    }
+// Tile shapes, and the shape of each configuration.
+constexpr int kShapes = 4, kShapeBm[kShapes] = {256, 128, 64, 256}, kShapeBn[kShapes] = {256, 128, 64, 128};
+constexpr int kShapeOf[7] = {0, 1, 2, 3, 0, 3, 1};
+
+// A problem list as the estimates see it, gathered in one pass: choosing among
+// the policies of a list took four times as long as planning the chosen one
+// while each walked the problems for every level and configuration (519
+// problems, FP32: 1.07 ms, against 0.26 for the whole plan now; 1000 problems
+// in a row 65 ms).
+struct ListSummary {
+  mfx_precision prec;
+  const mfx_gemm_problem* problems;
+  int count, levels = 0, cus;
+  std::vector<int> level;
+  bool lone = false;      // problems with producers or consumers hold more than half of the work
+  bool slow_wait = false; // some problem has its operands packed
+  std::vector<std::array<TileSums, kShapes>> all;  // per level: every problem on one shape
+  std::vector<int> best;        // per level: the configuration estimated shortest for all of its problems
+  std::vector<double> best_us;  // and that estimate
+
+  ListSummary(mfx_precision p, const mfx_gemm_problem* q, int n, const mfx_dep* deps, int ndeps, int cu)
+      : prec(p), problems(q), count(n), cus(cu), level(problem_levels(n, deps, ndeps)) {
+    if(count > 0) levels = *std::max_element(level.begin(), level.end()) + 1;
   }
-  return best;
-}
+
+  void gather(const mfx_dep* deps, int ndeps) {
+    std::vector<char> linked(count, 0);
+    for(int d = 0; d < ndeps; ++d) linked[deps[d].consumer] = linked[deps[d].producer] = 1;
+    double free_work = 0.0, all_work = 0.0;
+    all.resize(levels);
+    for(int i = 0; i < count; ++i) {
+      const mfx_gemm_problem& q = problems[i];
+      const double w = (double)q.m * q.n * q.k;
+      all_work += w;
+      if(!linked[i]) free_work += w;
+      slow_wait = slow_wait || (prec != MFX_PREC_FP32 && q.k % 16 != 0);
+      if(q.m <= 0 || q.n <= 0) continue;
+      const double k = (double)std::max<int64_t>(q.k, 1);
+      const bool slow = packed_small(prec, q.k);
+      for(int s = 0; s < kShapes; ++s) all[level[i]][s].add(tiles(i, s), k, slow);
+    }
+    lone = free_work < 0.5 * all_work;
+    best.assign(levels, -1);
+    best_us.assign(levels, 0.0);
+    for(int l = 0; l < levels; ++l)
+      for(int c = 0; c < 7; ++c) {
+        if(grouped_config(prec, c) != c) continue;
+        const double t = uniform(l, c);
+        if(best[l] < 0 || t < best_us[l]) {
+          best[l] = c;
+          best_us[l] = t;
+        }
+      }
+  }
+
+  int64_t tiles(int i, int shape) const {  // the sides are powers of two
+    const mfx_gemm_problem& q = problems[i];
+    const int bm = kShapeBm[shape] == 256 ? 8 : kShapeBm[shape] == 128 ? 7 : 6;
+    const int bn = kShapeBn[shape] == 256 ? 8 : kShapeBn[shape] == 128 ? 7 : 6;
+    return ((q.m + kShapeBm[shape] - 1) >> bm) * ((q.n + kShapeBn[shape] - 1) >> bn);
+  }
+
+  double uniform(int l, int c) const { return level_estimate(prec, c, all[l][kShapeOf[c]], c, TileSums{}, cus); }
+
+  // The tiles of each level on the large and the small configuration of `pol`,
+  // as assign_configs gives them out: one pass for all policies of the same
+  // shapes and bound.
+  using Assigned = std::vector<std::array<TileSums, 2>>;
+  struct Sharing {
+    int sb, ss;
+    double bound;
+    Assigned sums;
+  };
+  std::vector<std::unique_ptr<Sharing>> known;
+
+  const Assigned& assigned(const GroupedPolicy& pol) {
+    const int sb = kShapeOf[grouped_config(prec, pol.big)], ss = kShapeOf[grouped_config(prec, pol.small)];
+    for(const auto& k : known)
+      if(k->sb == sb && k->ss == ss && (k->bound == pol.bound || sb == ss)) return k->sums;
+    known.emplace_back(new Sharing{sb, ss, pol.bound, Assigned(levels)});
+    Assigned& sums = known.back()->sums;
+    if(sb == ss || pol.bound <= 0.0) {
+      for(int l = 0; l < levels; ++l) sums[l][0] = all[l][sb];
+    } else {
+      const double area = (double)kShapeBm[sb] * kShapeBn[sb];
+      for(int i = 0; i < count; ++i) {
+        const mfx_gemm_problem& q = problems[i];
+        if(q.m <= 0 || q.n <= 0) continue;
+        const int64_t n = tiles(i, sb);
+        const bool is_big = area * (double)n <= pol.bound * (double)q.m * (double)q.n;
+        sums[level[i]][is_big ? 0 : 1].add(is_big ? n : tiles(i, ss), (double)std::max<int64_t>(q.k, 1),
+            packed_small(prec, q.k));
+      }
+    }
+    if(sb != ss)
+      for(int l = 1; l < levels; ++l)
+        if(sums[l][0].tiles + sums[l][1].tiles < cus) {
+          sums[l][0] = TileSums{};
+          sums[l][1] = all[l][ss];
+        }
+    return sums;
+  }
+};
 
 // What a further dependency level costs beyond its tiles: a launch of its own
 // (item fetches from cold queues, a drained pipeline), or in one kernel the
@@ -202,59 +325,46 @@ int best_level_config(mfx_precision prec, const mfx_gemm_problem* problems, int 
 // tiles in one kernel, 102 in a launch per level, 99 on 64x64 tiles in one kernel).
 constexpr double kLevelLaunchUs = 16.0, kLevelWaitUs = 8.0, kLoneLevelWaitUs = 6.0, kSlowLevelWaitUs = 20.0;
 
-// Whether problems with producers or consumers hold more than half of the work.
-bool mostly_linked(const mfx_gemm_problem* problems, int count, const mfx_dep* deps, int ndeps) {
-  std::vector<char> linked(count, 0);
-  for(int d = 0; d < ndeps; ++d) linked[deps[d].consumer] = linked[deps[d].producer] = 1;
-  double free_work = 0.0, all_work = 0.0;
-  for(int i = 0; i < count; ++i) {
-    const double w = (double)problems[i].m * problems[i].n * problems[i].k;
-    all_work += w;
-    if(!linked[i]) free_work += w;
-  }
-  return free_work < 0.5 * all_work;
-}
-
 // Estimated microseconds of a launch under a policy.  One launch per level:
 // the levels' sum.  One kernel: all work spread over the CUs, or the chain of
 // the levels' longest tiles where that is longer.
-double policy_estimate(const GroupedPolicy& pol, mfx_precision prec, const mfx_gemm_problem* problems, int count,
-    const std::vector<int>& level, bool lone, int cus) {
-  const int levels = count ? *std::max_element(level.begin(), level.end()) + 1 : 0;
-  const std::vector<int> cfg = assign_configs(pol, prec, problems, count, level, cus);
-  auto of = [&](int i) { return cfg[i]; };
-  if(pol.per_level == 1 && levels > 1) {
-    double est = kLevelLaunchUs * (levels - 1);
-    for(int l = 0; l < levels; ++l) {
-      double uniform = 0.0;
-      best_level_config(prec, problems, count, level, l, cus, &uniform);
-      est += std::min(level_estimate(prec, problems, count, level, l, cus, of), uniform);
-    }
+double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
+  const mfx_precision prec = list.prec;
+  const int big = grouped_config(prec, pol.big), small = grouped_config(prec, pol.small), cus = list.cus;
+  const auto& sums = list.assigned(pol);
+  if(pol.per_level == 1 && list.levels > 1) {
+    double est = kLevelLaunchUs * (list.levels - 1);
+    for(int l = 0; l < list.levels; ++l)
+      est += std::min(level_estimate(prec, big, sums[l][0], small, sums[l][1], cus), list.best_us[l]);
     return est;
   }
-  if(levels == 1) return level_estimate(prec, problems, count, level, 0, cus, of);
-  int64_t tiles = 0;
-  auto tiles_of = [&](int i) {
-    const auto& q = problems[i];
-    return q.m <= 0 || q.n <= 0 ? (int64_t)0 : ceil_div(q.m, cfg_bm(cfg[i])) * ceil_div(q.n, cfg_bn(cfg[i]));
-  };
-  for(int i = 0; i < count; ++i) tiles += tiles_of(i);
-  std::vector<double> longest(std::max(levels, 1), 0.0);
-  double work = 0.0, last = 0.0;
-  for(int i = 0; i < count; ++i) {
-    if(tiles_of(i) == 0) continue;
-    const double t = grouped_tile_us(prec, cfg[i], problems[i].k, (double)tiles / cus);
-    work += t * (double)tiles_of(i);
-    last = std::max(last, t);
-    if(level[i] > 0 || levels == 1) longest[level[i]] = std::max(longest[level[i]], t);
+  if(list.levels == 1) return level_estimate(prec, big, sums[0][0], small, sums[0][1], cus);
+  TileSums total[2];
+  for(const auto& s : sums) {
+    total[0].add(s[0]);
+    total[1].add(s[1]);
   }
-  // the first level's linked problems are as long as its longest tile at most
-  longest[0] = last;
-  bool slow = pol.small == 2;
-  for(int i = 0; i < count; ++i) slow = slow || (prec != MFX_PREC_FP32 && problems[i].k % 16 != 0);
-  double path = (!lone ? kLevelWaitUs : slow ? kSlowLevelWaitUs : kLoneLevelWaitUs) * (levels - 1);
-  for(int l = 0; l < levels; ++l) path += longest[l];
+  const double busy = (double)(total[0].tiles + total[1].tiles) / cus;
+  double last = 0.0, any = -1.0;
+  const double work = sum_us(prec, big, total[0], busy, &last, &any) + sum_us(prec, small, total[1], busy, &last, &any);
+  const bool slow = pol.small == 2 || list.slow_wait;
+  double path = (!list.lone ? kLevelWaitUs : slow ? kSlowLevelWaitUs : kLoneLevelWaitUs) * (list.levels - 1);
+  // the first level's linked problems are as long as the longest tile at most
+  path += last;
+  for(int l = 1; l < list.levels; ++l) {
+    double longest = 0.0;
+    sum_us(prec, big, sums[l][0], busy, &longest, &any);
+    sum_us(prec, small, sums[l][1], busy, &longest, &any);
+    path += longest;
+  }
   return std::max(work / cus + 0.25 * last, path);
+}
+
+// Policies that run the same launch for `prec`: FP32 has no direct form, and one
+// tile for two configurations (grouped_config).
+bool same_launch(mfx_precision prec, const GroupedPolicy& a, const GroupedPolicy& b) {
+  return grouped_config(prec, a.big) == grouped_config(prec, b.big) && grouped_config(prec, a.small) == grouped_config(prec, b.small) &&
+         a.bound == b.bound && a.per_level == b.per_level && (prec == MFX_PREC_FP32 || a.direct == b.direct);
 }
 
 }  // namespace
@@ -285,37 +395,38 @@ std::string grouped_tune_key(mfx_precision p, const mfx_gemm_problem* problems, 
 
 // Policy of a grouped launch: the tuner's override, a forced configuration,
 // a tuned entry, or the estimate.
-int choose_grouped_policy(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
-    const mfx_dep* deps, int ndeps) {
+// *us: the estimate, where the policy is not forced or tuned (-1).
+static int choose_grouped_policy(Handle* h, ListSummary& list, const mfx_dep* deps, int ndeps, double* us) {
+  const mfx_precision prec = list.prec;
+  *us = -1.0;
   if(h->grouped_policy >= 0) return h->grouped_policy;
   int forced = h->forced_config[prec];
   if(forced >= 0) {
     for(int i = 0; i < kPolicyCount; ++i)
       if(kPolicies[i].big == forced && kPolicies[i].small == forced && !kPolicies[i].per_level) return i;
   }
-  const int tuned = tuned_lookup(grouped_tune_key(prec, problems, count, deps, ndeps));
+  const int tuned = tuned_any() ? tuned_lookup(grouped_tune_key(prec, list.problems, list.count, deps, ndeps)) : -1;
   if(tuned >= 0 && tuned < kPolicyCount) return tuned;
-  const auto level = problem_levels(count, deps, ndeps);
-  const int cus = h->cu_count > 0 ? h->cu_count : 256;
-  const bool levels = count > 0 && *std::max_element(level.begin(), level.end()) > 0;
   // With dependency levels: one launch per level, or one kernel with in-kernel
   // waits, whose list-schedule order fills a chain's later levels' idle CUs
   // with other problems' tiles, by estimate.  Measured on MI355X: a lone 8-long
   // 2048^2 chain (split BF16) 0.45 ms per level against 0.66 ms in one kernel;
   // 30 problems of 128 to 1024 beside a chain of four 512^2 (single BF16) 46 us
   // in one kernel against 68 us per level.
+  list.gather(deps, ndeps);
   int best = 0;
-  double best_est = -1.0;
-  const bool lone = mostly_linked(problems, count, deps, ndeps);
   for(int i = 0; i < kPolicyCount; ++i) {
     // without levels the two modes are the same launch
-    if(kPolicies[i].per_level == 2 || (!levels && kPolicies[i].per_level == 1)) continue;
+    if(kPolicies[i].per_level == 2 || (list.levels <= 1 && kPolicies[i].per_level == 1)) continue;
     // BF16: the direct tiles (no packing pass; measured 1.3x faster on the
     // batched workload); FP32 has nothing to pack
     if(prec != MFX_PREC_FP32 && !kPolicies[i].direct) continue;
-    const double e = policy_estimate(kPolicies[i], prec, problems, count, level, lone, cus);
-    if(best_est < 0 || e < best_est) {
-      best_est = e;
+    bool seen = false;
+    for(int j = 0; j < i && !seen; ++j) seen = same_launch(prec, kPolicies[i], kPolicies[j]);
+    if(seen) continue;
+    const double e = policy_estimate(kPolicies[i], list);
+    if(*us < 0 || e < *us) {
+      *us = e;
       best = i;
     }
   }
@@ -514,27 +625,49 @@ std::vector<GItem> critical_path_items(const std::vector<int>& at, const std::ve
   std::vector<int> next(count, 0);
   for(int i : at)
     if(wait_for[i] == 0) pending.push({0.0, i});
-  std::priority_queue<double, std::vector<double>, std::greater<double>> free_at;
-  for(int w = 0; w < std::max(1, workers); ++w) free_at.push(0.0);
+  // workgroups that are free from the same time on, taken together: a problem's
+  // tiles are all alike, so they hand it out as one by one
+  using Free = std::pair<double, int>;  // (time, workgroups)
+  std::priority_queue<Free, std::vector<Free>, std::greater<Free>> free_at;
+  free_at.push({0.0, std::max(1, workers)});
   std::vector<GItem> out;
-  while(!ready.empty() || !pending.empty()) {
-    double t = free_at.top();
+  size_t total = 0;
+  for(int i : at) total += (size_t)P[i].tiles_m * P[i].tiles_n;
+  out.reserve(total);
+  auto take = [&](int p, int n) {  // the next n tiles of problem p
+    for(int tm = next[p] / P[p].tiles_n, tn = next[p] % P[p].tiles_n, i = 0; i < n; ++i) {
+      out.push_back({ITEM_TILE, p, tm, tn});
+      if(++tn == P[p].tiles_n) {
+        tn = 0;
+        ++tm;
+      }
+    }
+    next[p] += n;
+  };
+  size_t to_come = at.size();  // problems that have not become ready
+  auto arrives = [&] {
+    ready.push(pending.top().second);
+    pending.pop();
+    --to_come;
+  };
+  while(to_come > 0) {
+    double t = free_at.top().first;
+    int group = free_at.top().second;
     free_at.pop();
-    while(!pending.empty() && pending.top().first <= t) {
-      ready.push(pending.top().second);
-      pending.pop();
-    }
-    if(ready.empty()) {  // nothing due yet: this workgroup waits for the earliest
+    while(!pending.empty() && pending.top().first <= t) arrives();
+    if(ready.empty()) {  // nothing due yet: one workgroup waits for the earliest
+      if(group > 1) free_at.push({t, group - 1});
+      group = 1;
       t = pending.top().first;
-      ready.push(pending.top().second);
-      pending.pop();
+      arrives();
     }
-    const int p = ready.top();
-    const int tile = next[p]++;
-    out.push_back({ITEM_TILE, p, tile / P[p].tiles_n, tile % P[p].tiles_n});
+    const int p = ready.top(), tiles = P[p].tiles_m * P[p].tiles_n;
+    const int taken = std::min(group, tiles - next[p]);
+    if(taken < group) free_at.push({t, group - taken});
+    take(p, taken);
     finish[p] = std::max(finish[p], t + dur[p]);
-    free_at.push(t + dur[p]);
-    if(next[p] == P[p].tiles_m * P[p].tiles_n) {
+    free_at.push({t + dur[p], taken});
+    if(next[p] == tiles) {
       ready.pop();
       for(int c : cons[p]) {
         due[c] = std::max(due[c], finish[p]);
@@ -542,6 +675,8 @@ std::vector<GItem> critical_path_items(const std::vector<int>& at, const std::ve
       }
     }
   }
+  // no further arrival can change the order, whatever the times
+  for(; !ready.empty(); ready.pop()) take(ready.top(), P[ready.top()].tiles_m * P[ready.top()].tiles_n - next[ready.top()]);
   return out;
 }
 
@@ -599,14 +734,15 @@ PackJob make_job(const GProblem& P, bool is_a, int first_block) {
 
 }  // namespace
 
-mfx_status plan_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
-    const mfx_dep* deps, int ndeps, GroupedPlan& pl) {
+// The checks of a list, its dependencies and its policy: what is needed to tell
+// whether it runs as dense launches, before any table is laid out.
+static mfx_status choose_plan(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
+    const mfx_dep* deps, int ndeps, GroupedPlan& pl, std::optional<ListSummary>& list) {
   if(prec != MFX_PREC_FP32 && prec != MFX_PREC_SPLIT_BF16 && prec != MFX_PREC_BF16)
     return unsupported("grouped launch supports FP32, SPLIT_BF16 and BF16");
   MFX_CHECK(validate(prec, problems, count, deps, ndeps));
   pl.prec = prec;
   pl.problems.resize(count);
-  std::vector<int> level(count, 0);
   for(int i = 0; i < count; ++i) pl.problems[i].ndeps = pl.problems[i].consumed = 0;
   for(int d = 0; d < ndeps; ++d) {
     GProblem& c = pl.problems[deps[d].consumer];
@@ -617,18 +753,25 @@ mfx_status plan_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* p
     c.deps[c.ndeps++] = deps[d].producer;
     pl.problems[deps[d].producer].consumed = 1;
   }
-  for(int i = 0; i < count; ++i)
-    for(int e = 0; e < pl.problems[i].ndeps; ++e) level[i] = std::max(level[i], level[pl.problems[i].deps[e]] + 1);
+  list.emplace(prec, problems, count, deps, ndeps, cus_of(h));
+  pl.policy = choose_grouped_policy(h, *list, deps, ndeps, &pl.estimate);
+  return MFX_SUCCESS;
+}
+
+static void plan_tables(Handle* h, ListSummary& list, const mfx_dep* deps, int ndeps, GroupedPlan& pl) {
+  const mfx_precision prec = pl.prec;
+  const mfx_gemm_problem* problems = list.problems;
+  const int count = list.count;
+  const std::vector<int>& level = list.level;
   std::vector<char> has_prod(count), linked(count);
   for(int i = 0; i < count; ++i) {
     has_prod[i] = pl.problems[i].ndeps > 0;
     linked[i] = has_prod[i] || pl.problems[i].consumed;
   }
-  pl.policy = choose_grouped_policy(h, prec, problems, count, deps, ndeps);
   const GroupedPolicy& pol = kPolicies[pl.policy];
   pl.big = grouped_config(prec, pol.big);
   pl.small = grouped_config(prec, pol.small);
-  const int cus = h->cu_count > 0 ? h->cu_count : 256;
+  const int cus = cus_of(h);
   const bool packed = prec != MFX_PREC_FP32;
   const int nhl = prec == MFX_PREC_SPLIT_BF16 ? 2 : 1;
   const int max_level = count ? *std::max_element(level.begin(), level.end()) : 0;
@@ -653,15 +796,14 @@ mfx_status plan_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* p
   // levels of a chain of small matrices would leave CUs idle on large tiles.
   std::vector<int> level_cfg(max_level + 1, -1);
   if(pl.per_level && !pl.pipelined) {
+    if(list.best.empty()) list.gather(deps, ndeps);  // a forced or tuned policy
+    const auto& sums = list.assigned(pol);
     for(int lv = 0; lv <= max_level; ++lv) {
-      const double as_is = level_estimate(prec, problems, count, level, lv, cus, [&](int i) { return cfg[i]; });
-      double us = 0.0;
-      const int best = best_level_config(prec, problems, count, level, lv, cus, &us);
-      if(best < 0 || us >= 0.97 * as_is) continue;
-      level_cfg[lv] = best;
-      for(int i = 0; i < count; ++i)
-        if(level[i] == lv) cfg[i] = best;
+      const double as_is = level_estimate(prec, pl.big, sums[lv][0], pl.small, sums[lv][1], cus);
+      if(list.best_us[lv] < 0.97 * as_is) level_cfg[lv] = list.best[lv];
     }
+    for(int i = 0; i < count; ++i)
+      if(level_cfg[level[i]] >= 0) cfg[i] = level_cfg[level[i]];
   }
 
   size_t packed_bytes = 0;
@@ -867,6 +1009,13 @@ mfx_status plan_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* p
   pl.counter_ints = 1 + (size_t)segments * GROUPED_QUEUES + (size_t)count + (size_t)panels;
   pl.off_packed = pl.off_counters + round_up(pl.counter_ints * sizeof(int), 256);
   pl.total_bytes = pl.off_packed + packed_bytes;
+}
+
+mfx_status plan_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
+    const mfx_dep* deps, int ndeps, GroupedPlan& pl) {
+  std::optional<ListSummary> list;
+  MFX_CHECK(choose_plan(h, prec, problems, count, deps, ndeps, pl, list));
+  plan_tables(h, *list, deps, ndeps, pl);
   return MFX_SUCCESS;
 }
 
@@ -973,11 +1122,9 @@ constexpr int kDenseListMax = 16;
 constexpr double kGroupedFixedUs = 20.0, kDenseFloorUs = 11.0, kSplitFloorUs = 14.0, kBf16FloorUs = 12.0;
 constexpr double kPackFixedUs = 4.0, kPackBytesPerUs = 4.5e6;
 
-DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count, const mfx_dep* deps,
-    int ndeps, const GroupedPlan& pl) {
+DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count, const GroupedPlan& pl) {
   DenseList d;
-  if(count == 0 || count > kDenseListMax || h->grouped_policy >= 0 || h->forced_config[prec] >= 0) return d;
-  if(tuned_lookup(grouped_tune_key(prec, problems, count, deps, ndeps)) >= 0) return d;
+  if(count == 0 || count > kDenseListMax || pl.estimate < 0.0 || h->forced_config[prec] >= 0) return d;
   const int cus = cus_of(h);
   const bool packed = prec != MFX_PREC_FP32, split = prec == MFX_PREC_SPLIT_BF16;
   double dense = 0.0;
@@ -1010,9 +1157,7 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
     else partial = dense_f32_workspace(op, c, cus, h->forced_splits);
     d.partial = std::max(d.partial, partial);
   }
-  const auto level = problem_levels(count, deps, ndeps);
-  const double grouped = kGroupedFixedUs + policy_estimate(kPolicies[pl.policy], prec, problems, count, level,
-                                               mostly_linked(problems, count, deps, ndeps), cus);
+  const double grouped = kGroupedFixedUs + pl.estimate;
   // Clearly ahead only: a packed list pays two or three launches a problem,
   // which the model knows less well. Split BF16, dense and the best grouped
   // policy: four chained products of 500 35 and 57 us, eight of 900 143 and 174.
@@ -1031,9 +1176,10 @@ mfx_status launch_dense_list(Handle* h, mfx_precision prec, const DenseList& d, 
 mfx_status run_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
     const mfx_dep* deps, int ndeps, hipStream_t s) {
   GroupedPlan pl;
-  MFX_CHECK(plan_grouped(h, prec, problems, count, deps, ndeps, pl));
+  std::optional<ListSummary> list;
+  MFX_CHECK(choose_plan(h, prec, problems, count, deps, ndeps, pl, list));
   void* ws = nullptr;
-  const DenseList dense = dense_list(h, prec, problems, count, deps, ndeps, pl);
+  const DenseList dense = dense_list(h, prec, problems, count, pl);
   h->grouped_waits = true;
   if(!dense.ops.empty() && !is_capturing(h, s)) {
     // memory that is not to be had: the grouped kernels need less
@@ -1044,6 +1190,7 @@ mfx_status run_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* pr
     }
     (void)hipGetLastError();
   }
+  plan_tables(h, *list, deps, ndeps, pl);
   MFX_CHECK(workspace(h, pl.total_bytes, &ws));
   GroupedArgs g;
   MFX_CHECK(bind_grouped(h, pl, ws, g, s));
@@ -1180,7 +1327,7 @@ mfx_status mfx_grouped_graph_create(mfx_handle handle, mfx_precision prec, const
   gr->device = h->device;
   // The graph owns its tables, counters and packed operands, so later calls on
   // the handle (which may regrow the handle's workspace) cannot move them.
-  DenseList dense = dense_list(h, prec, problems, count, deps, ndeps, pl);
+  DenseList dense = dense_list(h, prec, problems, count, pl);
   hipError_t ae = hipMalloc(&gr->mem, std::max<size_t>(dense.ops.empty() ? pl.total_bytes : dense.packed + dense.partial, 256));
   if(ae != hipSuccess && !dense.ops.empty()) {
     (void)hipGetLastError();

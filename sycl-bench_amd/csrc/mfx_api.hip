@@ -236,6 +236,11 @@ int tuned_lookup(const std::string& key) {
   return it == g_tuned.end() ? -1 : it->second;
 }
 
+bool tuned_any() {
+  std::lock_guard<std::mutex> lock(g_tune_mutex);
+  return !g_tuned.empty();
+}
+
 // The square configuration a triangle's sparse last round is re-tiled with:
 // half or a quarter of the big tile's side.
 static int tri_small_config(mfx_precision p, int side) {
