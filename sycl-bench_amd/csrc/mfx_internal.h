@@ -391,21 +391,26 @@ __device__ __forceinline__ float scaled(const Epilogue& ep, float acc, float old
 // row 8*(q/4) + 4*(l/32) + q%4, column l%32.
 // Always inlined and taking the block by value: a call would force the whole
 // accumulator array into scratch memory.
-// All old values of a block are loaded before the first store, which the
-// compiler may not do by itself (C may alias C): with one load, wait and store
-// per element the triangle blocks of a 1024 x 1024 FP32 syrk took 7 us of its
-// 29.  A mirrored block's transposed value is four consecutive floats of a row
-// in each lane, written 16 bytes wide where C's rows are aligned for it.
+// All old values of a block are loaded, and all new ones computed, before its
+// first store, which the compiler may not do by itself (C may alias C): with one
+// load, wait and store per element the triangle blocks of a 1024 x 1024 FP32 syrk
+// took 7 us of its 29. The value is chosen by beta first and stored by position
+// afterwards: a predicated store that chose it itself waited, even without beta,
+// for every memory operation before it, the previous store among them, which cost
+// a block at the matrix's edge 2.4 us. A mirrored block's transposed value is four
+// consecutive floats of a row in each lane, written 16 bytes wide where C's rows
+// are aligned for it.
 __device__ __forceinline__ void store_block32(const Epilogue& ep, floatx16 acc, int r0, int c0, int lane) {
   const int col = c0 + (lane & 31);
   const int rbase = r0 + 4 * (lane >> 5);
   const bool inside = ep.uplo == TILES_FULL || (ep.uplo == TILES_LOWER ? r0 >= c0 + 32 : c0 >= r0 + 32);
   float* const direct = ep.C + (int64_t)rbase * ep.ldc + col;
   float* const mirrored = ep.C + (int64_t)col * ep.ldc + rbase;
-  float old[16];
+  float v[16];
   if(inside && r0 + 32 <= ep.M && c0 + 32 <= ep.N) {
     // Interior block: each register q is one 32-float row segment per half wave.
     if(ep.beta != 0.0f) {
+      float old[16];
 #pragma unroll
       for(int q = 0; q < 16; ++q) old[q] = direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc];
 #pragma unroll
@@ -415,58 +420,73 @@ __device__ __forceinline__ void store_block32(const Epilogue& ep, floatx16 acc, 
       for(int q = 0; q < 16; ++q) direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc] = ep.alpha * acc[q];
     }
     if(ep.uplo == TILES_FULL || !ep.mirror) return;
-    if(ep.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(ep.C) & 15u) == 0) {
-      floatx4 was[4] = {};
-      if(ep.beta != 0.0f) {
-#pragma unroll
-        for(int g = 0; g < 4; ++g) was[g] = *reinterpret_cast<const floatx4*>(mirrored + 8 * g);
-      }
-#pragma unroll
-      for(int g = 0; g < 4; ++g) {
-        floatx4 v;
-#pragma unroll
-        for(int u = 0; u < 4; ++u) v[u] = ep.beta != 0.0f ? scaled(ep, acc[4 * g + u], was[g][u]) : ep.alpha * acc[4 * g + u];
-        *reinterpret_cast<floatx4*>(mirrored + 8 * g) = v;
-      }
-      return;
-    }
+    const bool wide = ep.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(ep.C) & 15u) == 0;
     if(ep.beta != 0.0f) {
+      float old[16];
+      if(wide) {
 #pragma unroll
-      for(int q = 0; q < 16; ++q) old[q] = mirrored[8 * (q >> 2) + (q & 3)];
+        for(int g = 0; g < 4; ++g) {
+          const floatx4 was = *reinterpret_cast<const floatx4*>(mirrored + 8 * g);
+#pragma unroll
+          for(int u = 0; u < 4; ++u) old[4 * g + u] = was[u];
+        }
+      } else {
+#pragma unroll
+        for(int q = 0; q < 16; ++q) old[q] = mirrored[8 * (q >> 2) + (q & 3)];
+      }
+#pragma unroll
+      for(int q = 0; q < 16; ++q) v[q] = scaled(ep, acc[q], old[q]);
+    } else {
+#pragma unroll
+      for(int q = 0; q < 16; ++q) v[q] = ep.alpha * acc[q];
     }
+    if(wide) {
 #pragma unroll
-    for(int q = 0; q < 16; ++q)
-      mirrored[8 * (q >> 2) + (q & 3)] = ep.beta != 0.0f ? scaled(ep, acc[q], old[q]) : ep.alpha * acc[q];
+      for(int g = 0; g < 4; ++g)
+        *reinterpret_cast<floatx4*>(mirrored + 8 * g) = (floatx4){v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+    } else {
+#pragma unroll
+      for(int q = 0; q < 16; ++q) mirrored[8 * (q >> 2) + (q & 3)] = v[q];
+    }
     return;
   }
+  // nothing of the block is wanted: a small problem's tile has many of these
+  if(r0 >= ep.M || c0 >= ep.N || (ep.uplo == TILES_LOWER && r0 + 31 < c0) || (ep.uplo == TILES_UPPER && c0 + 31 < r0)) return;
   // A block at the matrix's edge or across the diagonal: old values come from
   // clamped positions without a branch (those of elements that are not written
-  // are not used), so that only the stores are predicated.
-  const int last_row = ep.M - 1, last_col = ep.N - 1, near_col = min(col, last_col);
+  // are not used), so that only the stores are predicated, by the rows [lo, hi)
+  // that this lane's column has (a test of uplo for each element was five
+  // branches).
+  const int last_row = ep.M - 1, near_col = min(col, ep.N - 1);
+  const int lo = ep.uplo == TILES_LOWER ? col : 0;
+  const int hi = col >= ep.N ? 0 : ep.uplo == TILES_UPPER ? min(col + 1, ep.M) : ep.M;
   auto row_of = [&](int q) { return rbase + 8 * (q >> 2) + (q & 3); };
-  auto writes = [&](int row) {
-    return row <= last_row && col <= last_col && (ep.uplo == TILES_FULL || (ep.uplo == TILES_LOWER ? row >= col : row <= col));
-  };
-  const bool mirror = ep.uplo != TILES_FULL && ep.mirror;  // C is square then
   if(ep.beta != 0.0f) {
+    float old[16];
 #pragma unroll
     for(int q = 0; q < 16; ++q) old[q] = ep.C[(int64_t)min(row_of(q), last_row) * ep.ldc + near_col];
+#pragma unroll
+    for(int q = 0; q < 16; ++q) v[q] = scaled(ep, acc[q], old[q]);
+  } else {
+#pragma unroll
+    for(int q = 0; q < 16; ++q) v[q] = ep.alpha * acc[q];
   }
 #pragma unroll
-  for(int q = 0; q < 16; ++q) {
-    const float v = ep.beta != 0.0f ? scaled(ep, acc[q], old[q]) : ep.alpha * acc[q];
-    if(writes(row_of(q))) direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc] = v;
-  }
-  if(!mirror) return;
-  if(ep.beta != 0.0f) {
+  for(int q = 0; q < 16; ++q)
+    if(row_of(q) >= lo && row_of(q) < hi) direct[(int64_t)(8 * (q >> 2) + (q & 3)) * ep.ldc] = v[q];
+  if(ep.uplo == TILES_FULL || !ep.mirror) return;
+  // C is square; the diagonal has no mirror
+  const int mlo = ep.uplo == TILES_LOWER ? col + 1 : 0, mhi = ep.uplo == TILES_UPPER ? min(col, hi) : hi;
+  if(ep.beta != 0.0f) {  // without it the transposed value is the same
+    float old[16];
 #pragma unroll
     for(int q = 0; q < 16; ++q) old[q] = ep.C[(int64_t)near_col * ep.ldc + min(row_of(q), last_row)];
+#pragma unroll
+    for(int q = 0; q < 16; ++q) v[q] = scaled(ep, acc[q], old[q]);
   }
 #pragma unroll
-  for(int q = 0; q < 16; ++q) {
-    const float v = ep.beta != 0.0f ? scaled(ep, acc[q], old[q]) : ep.alpha * acc[q];
-    if(writes(row_of(q)) && row_of(q) != col) mirrored[8 * (q >> 2) + (q & 3)] = v;
-  }
+  for(int q = 0; q < 16; ++q)
+    if(row_of(q) >= mlo && row_of(q) < mhi) mirrored[8 * (q >> 2) + (q & 3)] = v[q];
 }
 
 // ---------------------------------------------------------------------------
