@@ -1133,7 +1133,7 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
     if(q.m == 0 || q.n == 0) continue;
     const int c = choose_config(h, prec, q.m, q.n, q.k);
     int bm, bn, bk, w;
-    config_info(prec, c, &bm, &bn, &bk, &w);
+    if(!config_info(prec, c, &bm, &bn, &bk, &w)) return DenseList{};  // an id of a loaded table that this library lacks
     double us = plan_splits(prec, c, ceil_div(q.m, bm) * ceil_div(q.n, bn), q.k, cus, kMaxPartialBytes, nullptr);
     if(packed) us += kPackFixedUs + 8.0 * (double)(q.m + q.n) * (double)q.k / kPackBytesPerUs;
     dense += std::max(split ? kSplitFloorUs : packed ? kBf16FloorUs : kDenseFloorUs, us);

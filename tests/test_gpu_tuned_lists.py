@@ -1,0 +1,53 @@
+"""Short lists under a loaded or measured tuning table (GPU, through the C ABI)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+TOL = {"fp32": 2e-6, "split-bf16": 1e-5, "bf16": 1e-2}
+
+
+@pytest.fixture
+def table(mfx, tmp_path):
+    """load(entries) replaces the tuning table; the empty one comes back afterwards."""
+    path = str(tmp_path / "tune.json")
+
+    def load(entries):
+        text = ",\n".join(f'    "{k}": {v}' for k, v in entries.items())
+        open(path, "w").write('{\n  "format": "mfx-autotune-2",\n  "entries": {\n' + text + "\n  }\n}\n")
+        assert mfx.load().mfx_autotune_load(path.encode()) == 0
+
+    yield load
+    load({})
+
+
+def chain(h, n, count=4):
+    mats = [torch.empty((n, n), device=DEV) for _ in range(count)]
+    for i, x in enumerate(mats):
+        h.fill_uniform(x, 37, i)
+    return mats, [torch.empty((n, n), device=DEV) for _ in range(count - 2)], torch.full((n, n), float("nan"), device=DEV)
+
+
+def recorded(h, mats, scratch, out, prec):
+    h.timing_begin()
+    h.chain(mats, scratch, out, prec=prec)
+    rec = h.timing_end()
+    h.grouped_status()
+    want = mats[0].double() @ mats[1].double() @ mats[2].double() @ mats[3].double()
+    assert torch.linalg.norm(out.double() - want) < 2 * TOL[prec] * torch.linalg.norm(want)
+    return rec
+
+
+@pytest.mark.parametrize("prec,key", [("fp32", "0:9:9:9"), ("split-bf16", "1:9:9:9"), ("bf16", "2:9:9:9")])
+def test_unknown_configuration_in_the_table(handle, mfx, table, prec, key):
+    """A product refuses such an id; a list of such products runs as the grouped launch, which does not use it."""
+    print(f"unknown configuration {prec}", flush=True)
+    mats, scratch, out = chain(handle, 500)
+    assert not any(x.startswith("grouped_") for x in recorded(handle, mats, scratch, out, prec))
+    table({key: 60})
+    out.fill_(float("nan"))
+    assert any(x.startswith("grouped_") for x in recorded(handle, mats, scratch, out, prec))
+    with pytest.raises(mfx.MfxError) as e:
+        handle.gemm(mats[0], mats[1], out, prec=prec)
+    assert e.value.status == 1
