@@ -194,8 +194,8 @@ typedef struct mfx_dep {
 } mfx_dep;
 
 /*
- * Runs `count` problems in one persistent grouped launch (an untuned short
- * list whose problems each fill the GPU: one dense launch per problem).
+ * Runs `count` problems in one persistent grouped launch (a short list that is
+ * estimated, or was tuned, faster so: one dense launch per problem).
  * Producers listed in `deps` must come before their consumers in `problems`; a
  * consumer tile waits in-kernel (bounded) for its producers.  Precisions: FP32,
  * SPLIT_BF16, BF16.
@@ -334,7 +334,9 @@ mfx_status mfx_autotune(mfx_handle handle, mfx_precision prec, int64_t m, int64_
  * times the launch under every policy (see mfx_grouped_policy_info), records
  * the fastest for launches with the same key (precision, problem count,
  * contraction volume and dependency depth, in power-of-two buckets) and
- * returns its id.  Each policy's launch is planned once and timed over
+ * returns its id.  A list short enough to run as one dense launch per problem
+ * is timed in that form too; if it is the fastest, that is what is recorded, and
+ * the id returned is that of the fastest policy.  Each policy's launch is planned once and timed over
  * back-to-back launches of the same tables (as a captured graph replays it),
  * in two rounds over the policies, the faster kept.  Runs the launch several
  * times on the given buffers (C is overwritten).  Blocking.

@@ -14,7 +14,7 @@
 #include <tuple>
 #include <vector>
 
-#include "mfx_internal.h"
+#include "grouped.h"
 
 namespace mfx {
 
@@ -28,8 +28,6 @@ bool grouped_policy_info(int id, int* big, int* small, double* bound, int* per_l
 bool grouped_policy_direct(int id);
 std::string grouped_tune_key(mfx_precision p, const mfx_gemm_problem* problems, int count, const mfx_dep* deps,
     int ndeps);
-mfx_status time_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
-    const mfx_dep* deps, int ndeps, int reps, hipStream_t s, double* ms);
 mfx_status launch_fill_uniform(Handle* h, int64_t rows, int64_t cols, float* p, int64_t ld, uint64_t seed,
     uint32_t mid, hipStream_t s);
 
@@ -174,14 +172,19 @@ mfx_status mfx_autotune_grouped(mfx_handle handle, mfx_precision prec, const mfx
   // policy's faster round kept (the first round's early candidates can run
   // while the clock is still ramping up).
   std::vector<double> cand_ms(cand.size(), 0.0);
+  double dense_ms = -1.0;
   mfx_status st = MFX_SUCCESS;
-  for(int round = 0; round < 2 && st == MFX_SUCCESS; ++round)
+  for(int round = 0; round < 2 && st == MFX_SUCCESS; ++round) {
     for(size_t i = 0; i < cand.size() && st == MFX_SUCCESS; ++i) {
       h->grouped_policy = cand[i];
       double ms = 0.0;
       st = time_grouped(h, prec, problems, count, deps, ndeps, 5, s, &ms);
       if(st == MFX_SUCCESS && (round == 0 || ms < cand_ms[i])) cand_ms[i] = ms;
     }
+    double ms = -1.0;
+    if(st == MFX_SUCCESS) st = time_dense_list(h, prec, problems, count, 5, s, &ms);
+    if(st == MFX_SUCCESS && ms >= 0.0 && (dense_ms < 0.0 || ms < dense_ms)) dense_ms = ms;
+  }
   int best = -1;
   double best_ms = 0.0;
   for(size_t i = 0; i < cand.size(); ++i)
@@ -192,7 +195,8 @@ mfx_status mfx_autotune_grouped(mfx_handle handle, mfx_precision prec, const mfx
   h->grouped_policy = forced_policy;
   h->timing = timing;
   MFX_CHECK(st);
-  record_tuned(grouped_tune_key(prec, problems, count, deps, ndeps), best);
+  const bool dense = dense_ms >= 0.0 && dense_ms < best_ms;
+  record_tuned(grouped_tune_key(prec, problems, count, deps, ndeps), dense ? kDenseListPolicy : best);
   if(best_policy) *best_policy = best;
   return MFX_SUCCESS;
 }

@@ -252,6 +252,7 @@ struct GroupedPlan {
   size_t total_bytes = 0;
   int policy = 0, big = 0, small = 0;  // tile policy and its configurations
   double estimate = -1.0;              // microseconds estimated for it; -1: forced or tuned
+  bool tuned_dense = false;            // tuned: dense launches instead (kDenseListPolicy)
   bool all_vec = true;                 // every problem allows 128-bit operand loads
   double flops = 0.0;
 };
@@ -260,12 +261,20 @@ struct GroupedPlan {
 mfx_status plan_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
     const mfx_dep* deps, int ndeps, GroupedPlan& pl);
 
+// Entry of the tuning table for a list that ran fastest as dense launches; not
+// a policy (a library without this form estimates one).
+constexpr int kDenseListPolicy = 64;
+
 // Plans and binds a grouped launch once, launches it once untimed, then
 // returns in *ms the average time of `reps` back-to-back launches of the same
 // bound tables (what a captured graph replays: no host planning between
 // launches, so the GPU never idles between them).
 mfx_status time_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
     const mfx_dep* deps, int ndeps, int reps, hipStream_t s, double* ms);
+
+// The same for the list as dense launches; *ms = -1 if it has no such form.
+mfx_status time_dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count, int reps,
+    hipStream_t s, double* ms);
 
 // Pre-pass: packs every job's operand (one chunk per thread).
 mfx_status launch_pack_jobs(Handle* h, int nhl, const PackJob* jobs, int njobs, int blocks, hipStream_t s);

@@ -395,10 +395,12 @@ std::string grouped_tune_key(mfx_precision p, const mfx_gemm_problem* problems, 
 
 // Policy of a grouped launch: the tuner's override, a forced configuration,
 // a tuned entry, or the estimate.
-// *us: the estimate, where the policy is not forced or tuned (-1).
-static int choose_grouped_policy(Handle* h, ListSummary& list, const mfx_dep* deps, int ndeps, double* us) {
+// *us: the estimate, where the policy is not forced or tuned (-1).  *dense: the
+// table says that dense launches were faster than any policy.
+static int choose_grouped_policy(Handle* h, ListSummary& list, const mfx_dep* deps, int ndeps, double* us, bool* dense) {
   const mfx_precision prec = list.prec;
   *us = -1.0;
+  *dense = false;
   if(h->grouped_policy >= 0) return h->grouped_policy;
   int forced = h->forced_config[prec];
   if(forced >= 0) {
@@ -407,6 +409,7 @@ static int choose_grouped_policy(Handle* h, ListSummary& list, const mfx_dep* de
   }
   const int tuned = tuned_any() ? tuned_lookup(grouped_tune_key(prec, list.problems, list.count, deps, ndeps)) : -1;
   if(tuned >= 0 && tuned < kPolicyCount) return tuned;
+  *dense = tuned == kDenseListPolicy;
   // With dependency levels: one launch per level, or one kernel with in-kernel
   // waits, whose list-schedule order fills a chain's later levels' idle CUs
   // with other problems' tiles, by estimate.  Measured on MI355X: a lone 8-long
@@ -754,7 +757,7 @@ static mfx_status choose_plan(Handle* h, mfx_precision prec, const mfx_gemm_prob
     pl.problems[deps[d].producer].consumed = 1;
   }
   list.emplace(prec, problems, count, deps, ndeps, cus_of(h));
-  pl.policy = choose_grouped_policy(h, *list, deps, ndeps, &pl.estimate);
+  pl.policy = choose_grouped_policy(h, *list, deps, ndeps, &pl.estimate, &pl.tuned_dense);
   return MFX_SUCCESS;
 }
 
@@ -1109,7 +1112,8 @@ static mfx_status launch_grouped_kernels(Handle* h, const GroupedPlan& pl, const
 // A short list whose problems each fill the GPU runs as one dense launch per
 // problem instead (same stream, in list order, which is a topological one):
 // those kernels split k where tiles are few and reach a tile without queues
-// and problem tables.  Untuned lists only; a forced or tuned policy is kept.
+// and problem tables.  By estimate for untuned lists, by measurement for tuned
+// ones (kDenseListPolicy); a forced or tuned policy is kept.
 struct DenseList {
   std::vector<DenseOp> ops;  // empty: the grouped launch is estimated shorter
   std::vector<int> config;
@@ -1122,9 +1126,10 @@ constexpr int kDenseListMax = 16;
 constexpr double kGroupedFixedUs = 20.0, kDenseFloorUs = 11.0, kSplitFloorUs = 14.0, kBf16FloorUs = 12.0;
 constexpr double kPackFixedUs = 4.0, kPackBytesPerUs = 4.5e6;
 
-DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count, const GroupedPlan& pl) {
+// The dense launches of a list (none if it has no such form) and their estimate.
+DenseList dense_form(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count, double* estimate) {
   DenseList d;
-  if(count == 0 || count > kDenseListMax || pl.estimate < 0.0 || h->forced_config[prec] >= 0) return d;
+  if(count == 0 || count > kDenseListMax || h->forced_config[prec] >= 0) return d;
   const int cus = cus_of(h);
   const bool packed = prec != MFX_PREC_FP32, split = prec == MFX_PREC_SPLIT_BF16;
   double dense = 0.0;
@@ -1157,11 +1162,20 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
     else partial = dense_f32_workspace(op, c, cus, h->forced_splits);
     d.partial = std::max(d.partial, partial);
   }
+  *estimate = dense;
+  return d;
+}
+
+DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count, const GroupedPlan& pl) {
+  DenseList d;
+  if(pl.estimate < 0.0) return d;
+  double dense = 0.0;
+  d = dense_form(h, prec, problems, count, &dense);
   const double grouped = kGroupedFixedUs + pl.estimate;
   // Clearly ahead only: a packed list pays two or three launches a problem,
   // which the model knows less well. Split BF16, dense and the best grouped
   // policy: four chained products of 500 35 and 57 us, eight of 900 143 and 174.
-  if(dense >= (packed ? 0.8 : 0.9) * grouped) d.ops.clear();
+  if(!pl.tuned_dense && dense >= (prec == MFX_PREC_FP32 ? 0.9 : 0.8) * grouped) d.ops.clear();
   return d;
 }
 
@@ -1173,6 +1187,15 @@ mfx_status launch_dense_list(Handle* h, mfx_precision prec, const DenseList& d, 
   return MFX_SUCCESS;
 }
 
+// Memory of an eager dense list; false where it is not to be had.
+bool dense_memory(Handle* h, const DenseList& d, hipStream_t s, void** ws, void** partials) {
+  *ws = nullptr;
+  *partials = d.partial > 0 ? stream_partials(h, s) : nullptr;
+  if((*partials || d.partial == 0) && (d.packed == 0 || list_workspace(h, d.packed, ws) == MFX_SUCCESS)) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 mfx_status run_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
     const mfx_dep* deps, int ndeps, hipStream_t s) {
   GroupedPlan pl;
@@ -1181,14 +1204,11 @@ mfx_status run_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* pr
   void* ws = nullptr;
   const DenseList dense = dense_list(h, prec, problems, count, pl);
   h->grouped_waits = true;
-  if(!dense.ops.empty() && !is_capturing(h, s)) {
-    // memory that is not to be had: the grouped kernels need less
-    void* partials = dense.partial > 0 ? stream_partials(h, s) : nullptr;
-    if((partials || dense.partial == 0) && (dense.packed == 0 || list_workspace(h, dense.packed, &ws) == MFX_SUCCESS)) {
-      h->grouped_waits = false;
-      return launch_dense_list(h, prec, dense, ws, partials, s);
-    }
-    (void)hipGetLastError();
+  void* partials = nullptr;
+  // without the memory: the grouped kernels need less
+  if(!dense.ops.empty() && !is_capturing(h, s) && dense_memory(h, dense, s, &ws, &partials)) {
+    h->grouped_waits = false;
+    return launch_dense_list(h, prec, dense, ws, partials, s);
   }
   plan_tables(h, *list, deps, ndeps, pl);
   MFX_CHECK(workspace(h, pl.total_bytes, &ws));
@@ -1198,6 +1218,29 @@ mfx_status run_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* pr
   if(!h->error_flag) MFX_HIP(hipMalloc(&h->error_flag, 256));
   g.error = h->error_flag;
   return launch_grouped_kernels(h, pl, g, s);
+}
+
+// Average milliseconds of `reps` back-to-back calls of `launch` after an untimed one.
+template <class F>
+static mfx_status time_launches(F&& launch, int reps, hipStream_t s, double* ms) {
+  MFX_CHECK(launch());
+  hipEvent_t a = nullptr, b = nullptr;
+  MFX_HIP(hipEventCreate(&a));
+  hipError_t e = hipEventCreate(&b);
+  mfx_status st = e == hipSuccess ? MFX_SUCCESS : hip_fail(e, "hipEventCreate");
+  if(st == MFX_SUCCESS && (e = hipEventRecord(a, s)) != hipSuccess) st = hip_fail(e, "hipEventRecord");
+  for(int r = 0; r < reps && st == MFX_SUCCESS; ++r) st = launch();
+  float t = 0.0f;
+  if(st == MFX_SUCCESS) {
+    e = hipEventRecord(b, s);
+    if(e == hipSuccess) e = hipEventSynchronize(b);
+    if(e == hipSuccess) e = hipEventElapsedTime(&t, a, b);
+    if(e != hipSuccess) st = hip_fail(e, "grouped timing");
+  }
+  (void)hipEventDestroy(a);
+  if(b) (void)hipEventDestroy(b);
+  *ms = t / std::max(reps, 1);
+  return st;
 }
 
 mfx_status time_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count,
@@ -1210,24 +1253,18 @@ mfx_status time_grouped(Handle* h, mfx_precision prec, const mfx_gemm_problem* p
   MFX_CHECK(bind_grouped(h, pl, ws, g, s));
   if(!h->error_flag) MFX_HIP(hipMalloc(&h->error_flag, 256));
   g.error = h->error_flag;
-  MFX_CHECK(launch_grouped_kernels(h, pl, g, s));  // untimed
-  hipEvent_t a = nullptr, b = nullptr;
-  MFX_HIP(hipEventCreate(&a));
-  hipError_t e = hipEventCreate(&b);
-  mfx_status st = e == hipSuccess ? MFX_SUCCESS : hip_fail(e, "hipEventCreate");
-  if(st == MFX_SUCCESS && (e = hipEventRecord(a, s)) != hipSuccess) st = hip_fail(e, "hipEventRecord");
-  for(int r = 0; r < reps && st == MFX_SUCCESS; ++r) st = launch_grouped_kernels(h, pl, g, s);
-  float t = 0.0f;
-  if(st == MFX_SUCCESS) {
-    e = hipEventRecord(b, s);
-    if(e == hipSuccess) e = hipEventSynchronize(b);
-    if(e == hipSuccess) e = hipEventElapsedTime(&t, a, b);
-    if(e != hipSuccess) st = hip_fail(e, "grouped timing");
-  }
-  (void)hipEventDestroy(a);
-  if(b) (void)hipEventDestroy(b);
-  *ms = t / std::max(reps, 1);
-  return st;
+  h->grouped_waits = true;
+  return time_launches([&] { return launch_grouped_kernels(h, pl, g, s); }, reps, s, ms);
+}
+
+mfx_status time_dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* problems, int count, int reps,
+    hipStream_t s, double* ms) {
+  *ms = -1.0;
+  double estimate = 0.0;
+  void *ws = nullptr, *partials = nullptr;
+  const DenseList d = dense_form(h, prec, problems, count, &estimate);
+  if(d.ops.empty() || is_capturing(h, s) || !dense_memory(h, d, s, &ws, &partials)) return MFX_SUCCESS;
+  return time_launches([&] { return launch_dense_list(h, prec, d, ws, partials, s); }, reps, s, ms);
 }
 
 // Balanced-tree product of `count` n x n matrices as grouped problems.

@@ -51,3 +51,34 @@ def test_unknown_configuration_in_the_table(handle, mfx, table, prec, key):
     with pytest.raises(mfx.MfxError) as e:
         handle.gemm(mats[0], mats[1], out, prec=prec)
     assert e.value.status == 1
+
+
+@pytest.mark.parametrize("prec", ["fp32", "split-bf16", "bf16"])
+def test_tuning_keeps_the_dense_form(handle, mfx, table, tmp_path, prec):
+    """A list that runs as dense launches by a wide margin still does once it is tuned, also from a saved table."""
+    print(f"tuned list {prec}", flush=True)
+    mats, scratch, out = chain(handle, 1024)
+    pairs = [(mats[0], mats[1], scratch[0]), (mats[2], mats[3], scratch[1]), (scratch[0], scratch[1], out)]
+    policy = handle.autotune_grouped([mfx.problem(*p) for p in pairs], [(2, 0), (2, 1)], prec=prec)
+    assert 0 <= policy < mfx.grouped_policy_count()
+    assert not any(x.startswith("grouped_") for x in recorded(handle, mats, scratch, out, prec))
+    path = str(tmp_path / "saved.json").encode()
+    assert mfx.load().mfx_autotune_save(path) == 0
+    table({})
+    assert mfx.load().mfx_autotune_load(path) == 0
+    out.fill_(float("nan"))
+    assert not any(x.startswith("grouped_") for x in recorded(handle, mats, scratch, out, prec))
+    handle.force_grouped_policy(policy)  # a forced policy is still one
+    try:
+        assert any(x.startswith("grouped_") for x in recorded(handle, mats, scratch, out, prec))
+    finally:
+        handle.force_grouped_policy(-1)
+
+
+def test_a_tuned_policy_is_kept(handle, mfx, table):
+    """A table's policy still takes the list from the dense form."""
+    mats, scratch, out = chain(handle, 1024)
+    assert not any(x.startswith("grouped_") for x in recorded(handle, mats, scratch, out, "fp32"))
+    # three problems, the square root of their volume in the bucket of 2^16, two levels
+    table({"g0:2:16:1": 20})
+    assert any(x.startswith("grouped_") for x in recorded(handle, mats, scratch, out, "fp32"))
