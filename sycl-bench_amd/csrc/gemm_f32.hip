@@ -121,7 +121,7 @@ SplitPlan f32_split_plan(const DenseOp& op, int config, int cus, int forced_spli
     // eight slices
     int64_t s = std::min<int64_t>(std::min<int64_t>(8, 4 * cus / std::max<int64_t>(tiles, 1)), op.K / 128);
     while(s > 1 && tiles * s * c.bm * c.bn * 4 > kMaxPartialBytes) --s;
-    if(s > 1 && op.tiles == TILES_FULL && op.nprod == 1) plan = SplitPlan{0, (int)s};
+    if(s > 1 && op.nprod == 1) plan = SplitPlan{0, (int)s};
   } else if(forced_splits < 0) {
     plan_splits(MFX_PREC_FP32, config, tiles, steps * c.bk, cus, kMaxPartialBytes, &plan);
   }
@@ -130,15 +130,6 @@ SplitPlan f32_split_plan(const DenseOp& op, int config, int cus, int forced_spli
 
 size_t partial_bytes(const SplitPlan& plan, int64_t tiles, const F32Config& c) {
   return plan.splits > 1 ? (size_t)(tiles - plan.head) * plan.splits * c.bm * c.bn * sizeof(float) : 0;
-}
-
-// Whether re-tiling a triangle's last round is estimated shorter than the
-// split plan of the same configuration.
-bool tri_tail_wins(const DenseOp& op, int config, const TriTail& tail, int tiles, int cus) {
-  const int64_t k = (int64_t)ceil_div(op.K, F32_BK) * F32_BK * op.nprod;
-  const double retiled = tile_span(MFX_PREC_FP32, config, tail.head, k, cus) +
-                         tile_span(MFX_PREC_FP32, tail.small, (int64_t)(tiles - tail.head) * tail.ratio * tail.ratio, k, cus);
-  return retiled < plan_splits(MFX_PREC_FP32, config, tiles, k, cus, kMaxPartialBytes, nullptr);
 }
 
 // How a call runs on one configuration: k slices, or a triangle's re-tiled last
@@ -151,15 +142,12 @@ struct F32Call {
 
 F32Call f32_call(const DenseOp& op, int config, int cus, int forced_splits) {
   F32Call c;
-  const int tiles = (int)f32_tiles(op, config);
-  c.plan = f32_split_plan(op, config, cus, forced_splits);
-  if(op.tiles != TILES_FULL && forced_splits < 2) {
-    c.tail = tri_tail(MFX_PREC_FP32, config, ceil_div(op.M, kF32Configs[config].bm), cus);
-    if(c.tail.small >= 0 && (c.plan.splits == 1 || tri_tail_wins(op, config, c.tail, tiles, cus)))
-      c.plan = SplitPlan{c.tail.head, 1};
-    else
-      c.tail.small = -1;
-  }
+  const int64_t tiles = f32_tiles(op, config);
+  if(op.tiles != TILES_FULL && forced_splits < 2)
+    plan_f32_triangle(config, ceil_div(op.M, kF32Configs[config].bm), (int64_t)op.K * op.nprod, cus,
+        forced_splits == 1 ? 0 : kMaxPartialBytes, &c.plan, &c.tail);
+  else
+    c.plan = f32_split_plan(op, config, cus, forced_splits);
   c.partial = partial_bytes(c.plan, tiles, kF32Configs[config]);
   return c;
 }
@@ -206,6 +194,18 @@ bool few_tiles(const DenseOp& op, int config, int cus) {
 }
 
 }  // namespace
+
+double plan_f32_triangle(int config, int64_t T, int64_t k, int cus, int64_t max_partial, SplitPlan* plan, TriTail* tail) {
+  SplitPlan slices;
+  const int64_t tiles = T * (T + 1) / 2;
+  const double us = plan_splits(MFX_PREC_FP32, config, tiles, k, cus, config == kF32Crowded ? 0 : max_partial, &slices);
+  TriTail t = tri_tail(MFX_PREC_FP32, config, T, cus, k);
+  const bool retile = t.small >= 0 && t.us < us;
+  if(!retile) t.small = -1;
+  if(plan) *plan = retile ? SplitPlan{t.head, 1} : slices;
+  if(tail) *tail = t;
+  return retile ? t.us : us;
+}
 
 size_t dense_f32_workspace(const DenseOp& op, int config, int cus, int forced_splits) {
   if(config < 0 || config >= kF32ConfigCount) return 0;

@@ -187,19 +187,6 @@ void replace_tuned(const std::map<std::string, int>& t) {
   g_tuned = t;
 }
 
-// Per-flop rate of each tile configuration relative to the best one, on
-// large problems (the best configuration's time over this one's, measured on
-// MI355X at M = N = K = 8192).
-double config_rate(mfx_precision p, int c) {
-  static const double f32[] = {0.886, 0.868, 0.817, 0.859, 1.0, 0.97, 0.913, 0.81};
-  static const double split[] = {0.894, 0.846, 0.645, 0.70, 1.0, 0.80, 0.854};
-  static const double bf16[] = {0.844, 0.730, 0.508, 0.662, 1.0, 0.724, 0.814};
-  static const double fp8[] = {0.866, 0.69, 1.0};
-  const double* t = p == MFX_PREC_FP32 ? f32 : p == MFX_PREC_SPLIT_BF16 ? split : p == MFX_PREC_BF16 ? bf16 : fp8;
-  const int n = p == MFX_PREC_FP32 ? 8 : p == MFX_PREC_SPLIT_BF16 || p == MFX_PREC_BF16 ? 7 : 3;
-  return c >= 0 && c < n ? t[c] : 0.5;
-}
-
 // Used when nothing is tuned: the configuration whose estimated launch
 // (tile_span's measured model, with the k slices plan_splits or the smaller
 // tiles tri_tail would give a sparse last round) is shortest.
@@ -241,34 +228,26 @@ bool tuned_any() {
   return !g_tuned.empty();
 }
 
-// The square configuration a triangle's sparse last round is re-tiled with:
-// half or a quarter of the big tile's side.
-static int tri_small_config(mfx_precision p, int side) {
-  if(p == MFX_PREC_FP32) return side == 128 ? 6 : side == 64 ? 7 : -1;
-  if(p == MFX_PREC_SPLIT_BF16 || p == MFX_PREC_BF16) return side == 128 ? 6 : side == 64 ? 2 : -1;
-  return -1;
-}
-
-TriTail tri_tail(mfx_precision p, int config, int64_t T, int cus) {
+// FP32 alone: the packed precisions split such a round along k instead.
+TriTail tri_tail(mfx_precision p, int config, int64_t T, int cus, int64_t k) {
   TriTail t;
   int bm, bn, bk, w;
   if(!config_info(p, config, &bm, &bn, &bk, &w) || bm != bn || cus <= 0) return t;
   const int64_t tiles = T * (T + 1) / 2, rounds = tiles / cus, tail = tiles - rounds * cus;
   t.head = (int)tiles;
-  if(rounds == 0 || tail == 0 || 2 * tail > cus) return t;
-  // one more round of big tiles, against ceil(tail r^2 / cus) rounds of small ones
-  double best = (double)bm * bm / config_rate(p, config);
+  t.us = tile_span(p, config, tiles, (double)k, cus);
+  if(p != MFX_PREC_FP32 || rounds == 0 || tail == 0 || 2 * tail > cus) return t;
   for(int r : {2, 4}) {
-    const int s = tri_small_config(p, bm / r);
+    const int s = bm / r == 128 ? 6 : bm / r == 64 ? 7 : -1;  // the eight-wave configuration of that side
     if(s < 0) continue;
-    const double cost = (double)ceil_div(tail * r * r, cus) * (double)(bm / r) * (bm / r) / config_rate(p, s);
-    if(cost < best) {
-      best = cost;
+    const double us = tile_span(p, config, rounds * cus, (double)k, cus) + tile_span(p, s, tail * r * r, (double)k, cus);
+    if(us < t.us) {
+      t.us = us;
       t.small = s;
       t.ratio = r;
+      t.head = (int)(rounds * cus);
     }
   }
-  if(t.small >= 0) t.head = (int)(rounds * cus);
   return t;
 }
 
@@ -281,14 +260,9 @@ static int heuristic_square_config(Handle* h, mfx_precision p, int64_t n, int64_
   for(int c = 0; c < config_count(p); ++c) {
     int bm, bn, bk, w;
     if(!config_info(p, c, &bm, &bn, &bk, &w) || bm != bn) continue;
-    const int64_t T = ceil_div(n, bm), tiles = T * (T + 1) / 2;
-    double t = plan_splits(p, c, tiles, k, cus, max_partial, nullptr);
-    if(p == MFX_PREC_FP32) {
-      const TriTail tail = tri_tail(p, c, T, cus);
-      if(tail.small >= 0)
-        t = std::min(t, tile_span(p, c, tail.head, (double)k, cus) +
-                            tile_span(p, tail.small, (tiles - tail.head) * tail.ratio * tail.ratio, (double)k, cus));
-    }
+    const int64_t T = ceil_div(n, bm);
+    const double t = p == MFX_PREC_FP32 ? plan_f32_triangle(c, T, k, cus, max_partial, nullptr, nullptr)
+                                        : plan_splits(p, c, T * (T + 1) / 2, k, cus, max_partial, nullptr);
     if(best_t < 0.0 || t < best_t) {
       best = c;
       best_t = t;

@@ -503,17 +503,23 @@ struct DenseOp {
   int tiles;                                    // TILES_FULL / LOWER / UPPER
 };
 
-// Triangular schedules whose last round of tiles leaves most CUs idle: the
+// FP32 triangular schedules whose last round of tiles leaves most CUs idle: the
 // full rounds run on the chosen square tile, and the big tiles of the last
 // round are re-tiled `ratio` x `ratio` into a smaller square configuration
 // in a second launch, when that is estimated faster than one more round of
-// big tiles (small == -1: no split).
+// big tiles (small == -1: no re-tiling).
 struct TriTail {
-  int head = 0;    // big tiles of the first launch (all of them without a split)
-  int small = -1;  // configuration of the second launch
-  int ratio = 1;   // big tile side / small tile side
+  int head = 0;     // big tiles of the first launch (all of them without re-tiling)
+  int small = -1;   // configuration of the second launch
+  int ratio = 1;    // big tile side / small tile side
+  double us = 0.0;  // estimated microseconds of both
 };
-TriTail tri_tail(mfx_precision p, int config, int64_t tiles_per_side, int cus);
+TriTail tri_tail(mfx_precision p, int config, int64_t tiles_per_side, int cus, int64_t k = 4096);
+// How an FP32 triangle runs on `config`: its k slices or its re-tiled last round,
+// whichever is estimated shorter, and that estimate. The one place that decides,
+// for the choice of the configuration, the memory and the launch.
+double plan_f32_triangle(int config, int64_t tiles_per_side, int64_t k, int cus, int64_t max_partial, SplitPlan* plan,
+    TriTail* tail);
 
 mfx_status launch_dense_f32(Handle* h, const DenseOp& op, int config, hipStream_t s);
 // The same with split-K partial tiles in `ws` (ws_bytes long) instead of the
