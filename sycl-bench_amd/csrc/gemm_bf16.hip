@@ -100,10 +100,10 @@ constexpr int kBfConfigCount = sizeof(kBfConfigs) / sizeof(kBfConfigs[0]);
 template <int BM, int BN, int WM, int WN, int MOST = 4>
 mfx_status launch_bf_cfg(Handle* h, const BfParams& p, bool split, int grid, hipStream_t s) {
   if(split)
-    return timed_launch(h, "gemm_split_bf16_mfma", s, [&] {
+    return timed_launch(h, MOST == 2 ? "gemm_split_bf16_short_k" : "gemm_split_bf16_mfma", s, [&] {
       gemm_bf16x_kernel<BM, BN, WM, WN, 2, MOST><<<grid, BfCfg<BM, BN, WM, WN, 2>::NT, 0, s>>>(p);
     });
-  return timed_launch(h, "gemm_bf16_mfma", s, [&] {
+  return timed_launch(h, MOST == 2 ? "gemm_bf16_short_k" : "gemm_bf16_mfma", s, [&] {
     gemm_bf16x_kernel<BM, BN, WM, WN, 1, MOST><<<grid, BfCfg<BM, BN, WM, WN, 1>::NT, 0, s>>>(p);
   });
 }
