@@ -226,7 +226,7 @@ struct ListSummary {
   int count, levels = 0, cus;
   std::vector<int> level;
   bool lone = false;      // problems with producers or consumers hold more than half of the work
-  bool slow_wait = false; // some problem has its operands packed
+  bool slow_wait = false; // a problem with producers or consumers has its operands packed
   std::vector<std::array<TileSums, kShapes>> all;  // per level: every problem on one shape
   std::vector<int> best;        // per level: the configuration estimated shortest for all of its problems
   std::vector<double> best_us;  // and that estimate
@@ -246,7 +246,7 @@ struct ListSummary {
       const double w = (double)q.m * q.n * q.k;
       all_work += w;
       if(!linked[i]) free_work += w;
-      slow_wait = slow_wait || (prec != MFX_PREC_FP32 && q.k % 16 != 0);
+      slow_wait = slow_wait || (linked[i] && prec != MFX_PREC_FP32 && q.k % 16 != 0);
       if(q.m <= 0 || q.n <= 0) continue;
       const double k = (double)std::max<int64_t>(q.k, 1);
       const bool slow = packed_small(prec, q.k);

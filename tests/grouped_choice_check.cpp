@@ -1,0 +1,38 @@
+// Host-only check of the untuned choice of a grouped launch: small problems that
+// are packed, beside a chain that is read directly and holds nearly all of the
+// work, do not change the chain's policy. Prints "OK" or the list that differs.
+#include <cstdio>
+#include <vector>
+
+#include "grouped.h"
+
+using namespace mfx;
+
+static mfx_gemm_problem prob(int64_t m, int64_t n, int64_t k) {
+  float* p = reinterpret_cast<float*>(uintptr_t(0x100000));  // planning reads no operand
+  return mfx_gemm_problem{m, n, k, 1.0f, 0.0f, p, (k + 3) / 4 * 4, 0, p, n, 0, p, n};
+}
+
+int main() {
+  const std::vector<mfx_dep> deps = {{4, 0}, {4, 1}, {5, 2}, {5, 3}, {6, 4}, {6, 5}};
+  for(mfx_precision prec : {MFX_PREC_SPLIT_BF16, MFX_PREC_BF16})
+    for(int64_t n : {384, 448, 512}) {
+      int policy[2];
+      for(int extra : {0, 1}) {
+        std::vector<mfx_gemm_problem> list(7, prob(n, n, n));
+        if(extra) list.push_back(prob(100, 90, 77));
+        Handle h;
+        h.cu_count = 256;
+        GroupedPlan pl;
+        if(plan_grouped(&h, prec, list.data(), (int)list.size(), deps.data(), (int)deps.size(), pl) != MFX_SUCCESS) return 1;
+        policy[extra] = pl.policy;
+      }
+      if(policy[0] != policy[1]) {
+        std::printf("FAILED precision %d, chain of %d: policy %d, %d with a packed problem beside it\n", (int)prec, (int)n,
+            policy[0], policy[1]);
+        return 1;
+      }
+    }
+  std::printf("OK\n");
+  return 0;
+}
