@@ -326,8 +326,12 @@ struct ListSummary {
 constexpr double kLevelLaunchUs = 16.0, kLevelWaitUs = 8.0, kLoneLevelWaitUs = 6.0, kSlowLevelWaitUs = 20.0;
 
 // Estimated microseconds of a launch under a policy.  One launch per level:
-// the levels' sum.  One kernel: all work spread over the CUs, or the chain of
-// the levels' longest tiles where that is longer.
+// the levels' sum.  One kernel: the same where the chain holds most of the work,
+// as nothing else fills a level's last round of tiles (spread over the CUs
+// instead, eight chained products of 768 were estimated at 95 us on 64x64 tiles,
+// single BF16, beside thirty small problems, and took 211; 87 on 128x128); else
+// all work spread over the CUs, or the chain of the levels' longest tiles where
+// that is longer.
 double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
   const mfx_precision prec = list.prec;
   const int big = grouped_config(prec, pol.big), small = grouped_config(prec, pol.small), cus = list.cus;
@@ -339,6 +343,12 @@ double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
     return est;
   }
   if(list.levels == 1) return level_estimate(prec, big, sums[0][0], small, sums[0][1], cus);
+  if(list.lone) {
+    const bool slow = pol.small == 2 || list.slow_wait;
+    double est = (slow ? kSlowLevelWaitUs : kLoneLevelWaitUs) * (list.levels - 1);
+    for(const auto& s : sums) est += level_estimate(prec, big, s[0], small, s[1], cus);
+    return est;
+  }
   TileSums total[2];
   for(const auto& s : sums) {
     total[0].add(s[0]);
@@ -347,8 +357,7 @@ double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
   const double busy = (double)(total[0].tiles + total[1].tiles) / cus;
   double last = 0.0, any = -1.0;
   const double work = sum_us(prec, big, total[0], busy, &last, &any) + sum_us(prec, small, total[1], busy, &last, &any);
-  const bool slow = pol.small == 2 || list.slow_wait;
-  double path = (!list.lone ? kLevelWaitUs : slow ? kSlowLevelWaitUs : kLoneLevelWaitUs) * (list.levels - 1);
+  double path = kLevelWaitUs * (list.levels - 1);
   // the first level's linked problems are as long as the longest tile at most
   path += last;
   for(int l = 1; l < list.levels; ++l) {
@@ -1172,10 +1181,13 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
   double dense = 0.0;
   d = dense_form(h, prec, problems, count, &dense);
   const double grouped = kGroupedFixedUs + pl.estimate;
-  // Clearly ahead only: a packed list pays two or three launches a problem,
-  // which the model knows less well. Split BF16, dense and the best grouped
-  // policy: four chained products of 500 35 and 57 us, eight of 900 143 and 174.
-  if(!pl.tuned_dense && dense >= (prec == MFX_PREC_FP32 ? 0.9 : 0.8) * grouped) d.ops.clear();
+  // Ahead by more than the estimates' error. FP32, dense and the best grouped
+  // policy: estimated at 0.91 of it, eight chained products of 300 take 1.27 of
+  // its time. The fixed times of packed problems are estimated high, so that
+  // every packed list estimated below 1.0 (twenty, 2 to 16 problems) took 0.65
+  // to 0.94: split BF16, four chained products of 500 35 and 57 us, eight of 640
+  // (estimated at 0.86) 91 and 105, eight of 900 143 and 174.
+  if(!pl.tuned_dense && dense >= (prec == MFX_PREC_FP32 ? 0.9 : 0.92) * grouped) d.ops.clear();
   return d;
 }
 

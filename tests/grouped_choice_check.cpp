@@ -1,6 +1,8 @@
 // Host-only check of the untuned choice of a grouped launch: small problems that
 // are packed, beside a chain that is read directly and holds nearly all of the
-// work, do not change the chain's policy. Prints "OK" or the list that differs.
+// work, do not change the chain's policy; and a chain with several rounds of 64x64
+// tiles a level does not take them in one kernel, where nothing fills the last
+// round. Prints "OK" or the list that differs.
 #include <cstdio>
 #include <vector>
 
@@ -33,6 +35,22 @@ int main() {
         return 1;
       }
     }
+  // fifteen products of 640 in four levels: 238 us on 64x64 tiles in one kernel,
+  // 138 on 128x128 (split BF16; 217 and 100 single)
+  for(mfx_precision prec : {MFX_PREC_SPLIT_BF16, MFX_PREC_BF16}) {
+    std::vector<mfx_dep> chain;
+    for(int i = 8; i < 15; ++i)
+      for(int j : {2 * i - 16, 2 * i - 15}) chain.push_back({i, j});
+    const std::vector<mfx_gemm_problem> list(15, prob(640, 640, 640));
+    Handle h;
+    h.cu_count = 256;
+    GroupedPlan pl;
+    if(plan_grouped(&h, prec, list.data(), 15, chain.data(), (int)chain.size(), pl) != MFX_SUCCESS) return 1;
+    if(!pl.per_level && pl.small == 2) {
+      std::printf("FAILED precision %d: policy %d for the chain of 640\n", (int)prec, pl.policy);
+      return 1;
+    }
+  }
   std::printf("OK\n");
   return 0;
 }
