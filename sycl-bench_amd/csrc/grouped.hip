@@ -82,8 +82,8 @@ constexpr GroupedPolicy kPolicies[] = {
 constexpr int kPolicyCount = sizeof(kPolicies) / sizeof(kPolicies[0]);
 
 // Relative per-CU contraction rate of each tile configuration on large
-// problems (larger tiles reuse each loaded panel more), used by the
-// untuned policy estimate.
+// problems (larger tiles reuse each loaded panel more), used by the list
+// schedule's tile times (tile_ms).
 constexpr double kTileRate[7] = {1.0, 0.6, 0.2, 0.85, 1.15, 0.95, 0.65};
 
 // The configuration a grouped launch of `prec` runs for configuration c.
@@ -154,7 +154,8 @@ const GroupedTileCost& tile_cost(mfx_precision prec, int c) {
   return prec == MFX_PREC_FP32 ? kGroupedF32[c] : prec == MFX_PREC_SPLIT_BF16 ? kGroupedSplit[c] : kGroupedBf16[c];
 }
 // Single BF16 64x64 tiles of packed problems fall behind 128x128 ones from
-// about K = 256 on: eight chained products of 200 57 and 66 us, of 363 79 and 74.
+// about K = 256 on: in one kernel eight chained products of 200 take 52 and 51
+// us, of 363 87 and 73.
 constexpr double kPackedSmallUs = 5.0;
 bool packed_small(mfx_precision prec, int64_t k) { return prec == MFX_PREC_BF16 && k % 16 != 0 && k >= 256; }
 
@@ -235,6 +236,9 @@ struct ListSummary {
       : prec(p), problems(q), count(n), cus(cu), level(problem_levels(n, deps, ndeps)) {
     if(count > 0) levels = *std::max_element(level.begin(), level.end()) + 1;
   }
+
+  // one kernel is estimated by the sum of the levels
+  bool summed() const { return lone && levels > 1 && prec != MFX_PREC_FP32; }
 
   void gather(const mfx_dep* deps, int ndeps) {
     std::vector<char> linked(count, 0);
@@ -322,16 +326,18 @@ struct ListSummary {
 // on 128x128 tiles read directly, but 12 us on 64x64 tiles, whose second
 // workgroup per CU polls beside the first, and more where a level packs its
 // operands first (split BF16, eight chained products of 512: 87 us on 128x128
-// tiles in one kernel, 102 in a launch per level, 99 on 64x64 tiles in one kernel).
+// tiles in one kernel, 100 in a launch per level, 111 on 64x64 tiles in one kernel).
 constexpr double kLevelLaunchUs = 16.0, kLevelWaitUs = 8.0, kLoneLevelWaitUs = 6.0, kSlowLevelWaitUs = 20.0;
 
 // Estimated microseconds of a launch under a policy.  One launch per level:
-// the levels' sum.  One kernel: the same where the chain holds most of the work,
-// as nothing else fills a level's last round of tiles (spread over the CUs
-// instead, eight chained products of 768 were estimated at 95 us on 64x64 tiles,
-// single BF16, beside thirty small problems, and took 211; 87 on 128x128); else
-// all work spread over the CUs, or the chain of the levels' longest tiles where
-// that is longer.
+// the levels' sum.  One kernel: all work spread over the CUs, or the chain of
+// the levels' longest tiles where that is longer; but the levels' sum too for a
+// BF16 chain that holds most of the work, as nothing else fills a level's last
+// round of tiles (spread over the CUs, eight chained products of 768 beside
+// thirty small problems were estimated at 95 us on 64x64 tiles, single BF16, and
+// took 211; 87 on 128x128). FP32 chains keep the spread: summed, some were
+// chosen better (eight of 768 195 -> 122 us), others worse (sixteen of 400 101 ->
+// 134, thirty-two of 768 367 -> 475), as launches per level are estimated low.
 double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
   const mfx_precision prec = list.prec;
   const int big = grouped_config(prec, pol.big), small = grouped_config(prec, pol.small), cus = list.cus;
@@ -343,9 +349,10 @@ double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
     return est;
   }
   if(list.levels == 1) return level_estimate(prec, big, sums[0][0], small, sums[0][1], cus);
-  if(list.lone) {
-    const bool slow = pol.small == 2 || list.slow_wait;
-    double est = (slow ? kSlowLevelWaitUs : kLoneLevelWaitUs) * (list.levels - 1);
+  const bool slow = pol.small == 2 || list.slow_wait;
+  const double wait = !list.lone ? kLevelWaitUs : slow ? kSlowLevelWaitUs : kLoneLevelWaitUs;
+  if(list.summed()) {
+    double est = wait * (list.levels - 1);
     for(const auto& s : sums) est += level_estimate(prec, big, s[0], small, s[1], cus);
     return est;
   }
@@ -357,7 +364,7 @@ double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
   const double busy = (double)(total[0].tiles + total[1].tiles) / cus;
   double last = 0.0, any = -1.0;
   const double work = sum_us(prec, big, total[0], busy, &last, &any) + sum_us(prec, small, total[1], busy, &last, &any);
-  double path = kLevelWaitUs * (list.levels - 1);
+  double path = wait * (list.levels - 1);
   // the first level's linked problems are as long as the longest tile at most
   path += last;
   for(int l = 1; l < list.levels; ++l) {
@@ -767,6 +774,7 @@ static mfx_status choose_plan(Handle* h, mfx_precision prec, const mfx_gemm_prob
   }
   list.emplace(prec, problems, count, deps, ndeps, cus_of(h));
   pl.policy = choose_grouped_policy(h, *list, deps, ndeps, &pl.estimate, &pl.tuned_dense);
+  pl.summed = list->summed();
   return MFX_SUCCESS;
 }
 
@@ -1181,13 +1189,15 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
   double dense = 0.0;
   d = dense_form(h, prec, problems, count, &dense);
   const double grouped = kGroupedFixedUs + pl.estimate;
-  // Ahead by more than the estimates' error. FP32, dense and the best grouped
-  // policy: estimated at 0.91 of it, eight chained products of 300 take 1.27 of
-  // its time. The fixed times of packed problems are estimated high, so that
-  // every packed list estimated below 1.0 (twenty, 2 to 16 problems) took 0.65
-  // to 0.94: split BF16, four chained products of 500 35 and 57 us, eight of 640
-  // (estimated at 0.86) 91 and 105, eight of 900 143 and 174.
-  if(!pl.tuned_dense && dense >= (prec == MFX_PREC_FP32 ? 0.9 : 0.92) * grouped) d.ops.clear();
+  // Clearly ahead only: the estimates differ from the times by 10 to 20 %. FP32:
+  // estimated at 0.91 of the grouped time, eight chained products of 300 take
+  // 1.27 of it. A packed list pays two or three launches a problem, which the
+  // model knows less well: at 0.82, six independent ones took 75 us dense and 55
+  // grouped (single BF16), though most lists up to 0.9 are faster dense. The sum
+  // of a lone chain's levels has no such outliers below 0.9 (split BF16, eight of
+  // 640 at 0.86: 91 and 105 us, of 900 at 0.72: 132 and 175), but above (single
+  // BF16, sixteen of 1200 at 0.90: 286 and 219).
+  if(!pl.tuned_dense && dense >= (prec == MFX_PREC_FP32 || pl.summed ? 0.9 : 0.8) * grouped) d.ops.clear();
   return d;
 }
 

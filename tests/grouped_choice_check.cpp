@@ -2,7 +2,8 @@
 // are packed, beside a chain that is read directly and holds nearly all of the
 // work, do not change the chain's policy; and a chain with several rounds of 64x64
 // tiles a level does not take them in one kernel, where nothing fills the last
-// round. Prints "OK" or the list that differs.
+// round; but FP32 chains are not priced so, as launches per level are estimated
+// low there. Prints "OK" or the list that differs.
 #include <cstdio>
 #include <vector>
 
@@ -48,6 +49,21 @@ int main() {
     if(plan_grouped(&h, prec, list.data(), 15, chain.data(), (int)chain.size(), pl) != MFX_SUCCESS) return 1;
     if(!pl.per_level && pl.small == 2) {
       std::printf("FAILED precision %d: policy %d for the chain of 640\n", (int)prec, pl.policy);
+      return 1;
+    }
+  }
+  // FP32, sixteen products of 400: 101 us in one kernel, 134 in a launch per level
+  {
+    std::vector<mfx_dep> chain;
+    for(int i = 8; i < 15; ++i)
+      for(int j : {2 * i - 16, 2 * i - 15}) chain.push_back({i, j});
+    const std::vector<mfx_gemm_problem> list(15, prob(400, 400, 400));
+    Handle h;
+    h.cu_count = 256;
+    GroupedPlan pl;
+    if(plan_grouped(&h, MFX_PREC_FP32, list.data(), 15, chain.data(), (int)chain.size(), pl) != MFX_SUCCESS) return 1;
+    if(pl.per_level) {
+      std::printf("FAILED policy %d for sixteen FP32 products of 400\n", pl.policy);
       return 1;
     }
   }

@@ -82,3 +82,23 @@ def test_a_tuned_policy_is_kept(handle, mfx, table):
     # three problems, the square root of their volume in the bucket of 2^16, two levels
     table({"g0:2:16:1": 20})
     assert any(x.startswith("grouped_") for x in recorded(handle, mats, scratch, out, "fp32"))
+
+
+def test_independent_packed_products_near_the_line(handle, mfx):
+    """Estimated at 0.82 of the grouped launch as dense launches, six independent products that are packed run grouped."""
+    print("independent packed products", flush=True)
+    shapes = [(518, 339, 1151), (163, 1448, 590), (667, 268, 714), (1742, 1815, 678), (501, 176, 2006), (392, 392, 392)]
+    ops = []
+    for i, (m, n, k) in enumerate(shapes):
+        A, B = torch.empty((m, k), device=DEV), torch.empty((k, n), device=DEV)
+        handle.fill_uniform(A, 41, 2 * i)
+        handle.fill_uniform(B, 41, 2 * i + 1)
+        ops.append((A, B, torch.full((m, n), float("nan"), device=DEV)))
+    handle.timing_begin()
+    handle.grouped([mfx.problem(*o) for o in ops], [], prec="bf16")
+    rec = handle.timing_end()
+    handle.grouped_status()
+    assert any(x.startswith("grouped_") for x in rec)
+    for A, B, C in ops:
+        want = A.double() @ B.double()
+        assert torch.linalg.norm(C.double() - want) < TOL["bf16"] * torch.linalg.norm(want)
