@@ -228,6 +228,7 @@ struct ListSummary {
   std::vector<int> level;
   bool lone = false;      // problems with producers or consumers hold more than half of the work
   bool slow_wait = false; // a problem with producers or consumers has its operands packed
+  double first_k = 0.0;   // longest K of the first level's problems with consumers
   std::vector<std::array<TileSums, kShapes>> all;  // per level: every problem on one shape
   std::vector<int> best;        // per level: the configuration estimated shortest for all of its problems
   std::vector<double> best_us;  // and that estimate
@@ -253,6 +254,7 @@ struct ListSummary {
       slow_wait = slow_wait || (linked[i] && prec != MFX_PREC_FP32 && q.k % 16 != 0);
       if(q.m <= 0 || q.n <= 0) continue;
       const double k = (double)std::max<int64_t>(q.k, 1);
+      if(linked[i] && level[i] == 0) first_k = std::max(first_k, k);
       const bool slow = packed_small(prec, q.k);
       for(int s = 0; s < kShapes; ++s) all[level[i]][s].add(tiles(i, s), k, slow);
     }
@@ -338,6 +340,10 @@ constexpr double kLevelLaunchUs = 16.0, kLevelWaitUs = 8.0, kLoneLevelWaitUs = 6
 // took 211; 87 on 128x128). FP32 chains keep the spread: summed, some were
 // chosen better (eight of 768 195 -> 122 us), others worse (sixteen of 400 101 ->
 // 134, thirty-two of 768 367 -> 475), as launches per level are estimated low.
+// BF16 tiles of 64x64 run two workgroups to a CU, which take turns: with more
+// tiles than CUs a tile of the chain takes up to twice its time (split BF16, four
+// chained products of 384 beside thirty small problems: estimated at 43 us
+// without that, 77 measured; 52 on 128x128 tiles).
 double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
   const mfx_precision prec = list.prec;
   const int big = grouped_config(prec, pol.big), small = grouped_config(prec, pol.small), cus = list.cus;
@@ -367,11 +373,13 @@ double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
   double path = wait * (list.levels - 1);
   // the first level's linked problems are as long as the longest tile at most
   path += last;
+  const double share = prec != MFX_PREC_FP32 && pol.big == 2 && pol.small == 2 ? std::min(2.0, std::max(1.0, busy)) : 1.0;
+  path += (share - 1.0) * (tile_cost(prec, 2).fixed + 1e-3 * ns_per_k(tile_cost(prec, 2), busy) * list.first_k);
   for(int l = 1; l < list.levels; ++l) {
     double longest = 0.0;
     sum_us(prec, big, sums[l][0], busy, &longest, &any);
     sum_us(prec, small, sums[l][1], busy, &longest, &any);
-    path += longest;
+    path += share * longest;
   }
   return std::max(work / cus + 0.25 * last, path);
 }

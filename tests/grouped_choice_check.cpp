@@ -3,7 +3,9 @@
 // work, do not change the chain's policy; and a chain with several rounds of 64x64
 // tiles a level does not take them in one kernel, where nothing fills the last
 // round; but FP32 chains are not priced so, as launches per level are estimated
-// low there. Prints "OK" or the list that differs.
+// low there. Nor does a packed precision's chain take two 64x64 workgroups per CU
+// in one kernel where the problems beside it keep both busy. Prints "OK" or the
+// list that differs.
 #include <cstdio>
 #include <vector>
 
@@ -64,6 +66,20 @@ int main() {
     if(plan_grouped(&h, MFX_PREC_FP32, list.data(), 15, chain.data(), (int)chain.size(), pl) != MFX_SUCCESS) return 1;
     if(pl.per_level) {
       std::printf("FAILED policy %d for sixteen FP32 products of 400\n", pl.policy);
+      return 1;
+    }
+  }
+  // thirty small problems beside eight chained products of 384: 113 us on two
+  // 64x64 workgroups per CU, 73 on 128x128 tiles (split BF16; 100 and 55 single)
+  for(mfx_precision prec : {MFX_PREC_SPLIT_BF16, MFX_PREC_BF16}) {
+    std::vector<mfx_gemm_problem> list(7, prob(384, 384, 384));
+    for(int i = 0; i < 30; ++i) list.push_back(prob(64 + 112 * i % 448, 64 + 176 * i % 448, 64 + 304 * i % 448));
+    Handle h;
+    h.cu_count = 256;
+    GroupedPlan pl;
+    if(plan_grouped(&h, prec, list.data(), 37, deps.data(), (int)deps.size(), pl) != MFX_SUCCESS) return 1;
+    if(!pl.per_level && pl.small == 2) {
+      std::printf("FAILED precision %d: policy %d for the chain of 384 beside thirty problems\n", (int)prec, pl.policy);
       return 1;
     }
   }
