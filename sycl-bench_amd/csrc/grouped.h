@@ -252,7 +252,7 @@ struct GroupedPlan {
   size_t total_bytes = 0;
   int policy = 0, big = 0, small = 0;  // tile policy and its configurations
   double estimate = -1.0;              // microseconds estimated for it; -1: forced or tuned
-  bool summed = false;                 // the estimate is the sum of a lone chain's levels
+  bool summed = false;                 // the estimate counts a lone chain's levels
   bool tuned_dense = false;            // tuned: dense launches instead (kDenseListPolicy)
   bool all_vec = true;                 // every problem allows 128-bit operand loads
   double flops = 0.0;

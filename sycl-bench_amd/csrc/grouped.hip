@@ -238,7 +238,7 @@ struct ListSummary {
     if(count > 0) levels = *std::max_element(level.begin(), level.end()) + 1;
   }
 
-  // one kernel is estimated by the sum of the levels
+  // the sum of the levels is part of one kernel's estimate
   bool summed() const { return lone && levels > 1 && prec != MFX_PREC_FP32; }
 
   void gather(const mfx_dep* deps, int ndeps) {
@@ -333,13 +333,16 @@ constexpr double kLevelLaunchUs = 16.0, kLevelWaitUs = 8.0, kLoneLevelWaitUs = 6
 
 // Estimated microseconds of a launch under a policy.  One launch per level:
 // the levels' sum.  One kernel: all work spread over the CUs, or the chain of
-// the levels' longest tiles where that is longer; but the levels' sum too for a
-// BF16 chain that holds most of the work, as nothing else fills a level's last
-// round of tiles (spread over the CUs, eight chained products of 768 beside
-// thirty small problems were estimated at 95 us on 64x64 tiles, single BF16, and
-// took 211; 87 on 128x128). FP32 chains keep the spread: summed, some were
-// chosen better (eight of 768 195 -> 122 us), others worse (sixteen of 400 101 ->
-// 134, thirty-two of 768 367 -> 475), as launches per level are estimated low.
+// the levels' longest tiles where that is longer. For a BF16 chain that holds
+// most of the work, the mean of this and the levels' sum: little else fills a
+// level's last round of tiles, but the next level's products whose producers are
+// done do (spread alone, eight chained products of 768 beside thirty small
+// problems were estimated at 95 us on 64x64 tiles, single BF16, and took 211; 87
+// on 128x128; the sum alone slows chains with many rounds a level, split BF16,
+// eight of 1616 beside twenty 376 -> 417). FP32 chains keep the spread: summed,
+// some were chosen better (eight of 768 195 -> 122 us), others worse (sixteen of
+// 400 101 -> 134, thirty-two of 768 367 -> 475), as launches per level are
+// estimated low.
 // BF16 tiles of 64x64 run two workgroups to a CU, which take turns: with more
 // tiles than CUs a tile of the chain takes up to twice its time (split BF16, four
 // chained products of 384 beside thirty small problems: estimated at 43 us
@@ -357,11 +360,6 @@ double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
   if(list.levels == 1) return level_estimate(prec, big, sums[0][0], small, sums[0][1], cus);
   const bool slow = pol.small == 2 || list.slow_wait;
   const double wait = !list.lone ? kLevelWaitUs : slow ? kSlowLevelWaitUs : kLoneLevelWaitUs;
-  if(list.summed()) {
-    double est = wait * (list.levels - 1);
-    for(const auto& s : sums) est += level_estimate(prec, big, s[0], small, s[1], cus);
-    return est;
-  }
   TileSums total[2];
   for(const auto& s : sums) {
     total[0].add(s[0]);
@@ -381,7 +379,11 @@ double policy_estimate(const GroupedPolicy& pol, ListSummary& list) {
     sum_us(prec, small, sums[l][1], busy, &longest, &any);
     path += share * longest;
   }
-  return std::max(work / cus + 0.25 * last, path);
+  const double spread = std::max(work / cus + 0.25 * last, path);
+  if(!list.summed()) return spread;
+  double summed = wait * (list.levels - 1);
+  for(const auto& l : sums) summed += level_estimate(prec, big, l[0], small, l[1], cus);
+  return 0.5 * (spread + summed);
 }
 
 // Policies that run the same launch for `prec`: FP32 has no direct form, and one
@@ -1201,10 +1203,9 @@ DenseList dense_list(Handle* h, mfx_precision prec, const mfx_gemm_problem* prob
   // estimated at 0.91 of the grouped time, eight chained products of 300 take
   // 1.27 of it. A packed list pays two or three launches a problem, which the
   // model knows less well: at 0.82, six independent ones took 75 us dense and 55
-  // grouped (single BF16), though most lists up to 0.9 are faster dense. The sum
-  // of a lone chain's levels has no such outliers below 0.9 (split BF16, eight of
-  // 640 at 0.86: 91 and 105 us, of 900 at 0.72: 132 and 175), but above (single
-  // BF16, sixteen of 1200 at 0.90: 286 and 219).
+  // grouped (single BF16), though most lists up to 0.9 are faster dense. Lone
+  // chains have no such outliers below 0.9 (split BF16, eight of 640: 91 and 105
+  // us, of 900: 132 and 175), but above (single BF16, sixteen of 1200: 286 and 219).
   if(!pl.tuned_dense && dense >= (prec == MFX_PREC_FP32 || pl.summed ? 0.9 : 0.8) * grouped) d.ops.clear();
   return d;
 }
