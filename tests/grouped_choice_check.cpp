@@ -4,8 +4,8 @@
 // tiles a level does not take them in one kernel, where nothing fills the last
 // round; but FP32 chains are not priced so, as launches per level are estimated
 // low there. Nor does a packed precision's chain take two 64x64 workgroups per CU
-// in one kernel where the problems beside it keep both busy. Prints "OK" or the
-// list that differs.
+// in one kernel where the problems beside it keep both busy; and a chain with many
+// rounds of tiles a level stays in one kernel. Prints "OK" or the list that differs.
 #include <cstdio>
 #include <vector>
 
@@ -80,6 +80,20 @@ int main() {
     if(plan_grouped(&h, prec, list.data(), 37, deps.data(), (int)deps.size(), pl) != MFX_SUCCESS) return 1;
     if(!pl.per_level && pl.small == 2) {
       std::printf("FAILED precision %d: policy %d for the chain of 384 beside thirty problems\n", (int)prec, pl.policy);
+      return 1;
+    }
+  }
+  // eight split-BF16 products of 1600 beside small problems: 350 us in one kernel,
+  // 382 in a launch per level
+  {
+    std::vector<mfx_gemm_problem> list(7, prob(1600, 1600, 1600));
+    for(int i = 0; i < 20; ++i) list.push_back(prob(64 + 112 * i % 448, 64 + 176 * i % 448, 64 + 304 * i % 448));
+    Handle h;
+    h.cu_count = 256;
+    GroupedPlan pl;
+    if(plan_grouped(&h, MFX_PREC_SPLIT_BF16, list.data(), 27, deps.data(), (int)deps.size(), pl) != MFX_SUCCESS) return 1;
+    if(pl.per_level) {
+      std::printf("FAILED policy %d for the chain of 1600 beside twenty problems\n", pl.policy);
       return 1;
     }
   }
