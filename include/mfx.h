@@ -371,9 +371,9 @@ mfx_status mfx_config_info(mfx_precision prec, int32_t config, int32_t* bm, int3
 mfx_status mfx_force_config(mfx_handle handle, mfx_precision prec, int32_t config);
 /* Split-K override for later gemm / syrk / syr2k calls: -1 automatic
  * (the default: k slices when the tile grid leaves the CUs short of work),
- * 1 never, >= 2 that many k slices (fewer when K or the 32 MiB partial-tile
- * bound does not allow them; FP32 splits single products on tiles up to
- * 128x128 only).
+ * 1 never, >= 2 that many k slices of every tile (fewer when K or the 32 MiB
+ * partial-tile bound does not allow them), in every precision, for one product
+ * or two, full grids and triangles.
  * Split results are summed in slice order, so they are reproducible, but not
  * bit-identical to the unsplit kernel's.  No counterpart in the reference. */
 mfx_status mfx_force_splits(mfx_handle handle, int32_t splits);

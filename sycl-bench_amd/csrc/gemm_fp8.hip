@@ -14,7 +14,7 @@
 // are zero-padded to the tile and to 128.  Exponents: E[row/128][k/128].
 //
 // Contraction tiles: 256x256 (four waves of 128x128, or eight of 128x64),
-// 128x128 (four waves of 64x64, or eight of 64x32) or 64x64 (waves of 32x32);
+// 128x128 (four waves of 64x64) or 64x64 (waves of 32x32);
 // each wave's rows and columns lie inside one 128-block, so its A and B
 // scales are one byte each per stage.  Stage = 128 k (single) or 64 k
 // (two-term), up to four of them in LDS, filled by direct global-to-LDS loads,

@@ -545,11 +545,11 @@ constexpr int64_t kMaxPartialBytes = (int64_t)32 << 20;
 // The configuration for `op` without k slices, in place of `config` (chosen with
 // them): `config` itself where it was forced or tuned.
 int whole_config(Handle* h, mfx_precision p, const DenseOp& op, int config);
-// Estimated microseconds of a dense launch on `config` (tile_cost's model)
-// and the split plan behind it; partial tiles take at most max_partial bytes.
 // Estimated microseconds of `count` workgroups of `len` k each (no split).
 double tile_span(mfx_precision p, int config, int64_t count, double len, int cus);
 bool bf16_two_per_cu(mfx_precision p, int config, int64_t tiles, int64_t k, int cus);
+// Estimated microseconds of a dense launch on `config` (tile_span's model)
+// and the split plan behind it; partial tiles take at most max_partial bytes.
 double plan_splits(mfx_precision p, int config, int64_t tiles, int64_t k, int cus, int64_t max_partial, SplitPlan* plan);
 mfx_status launch_dense_fp8(Handle* h, const DenseOp& op, bool two_term, int config, hipStream_t s);
 // Packed operands and split-K partial tiles (*partial of them, at the end).

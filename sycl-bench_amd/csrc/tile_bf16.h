@@ -33,10 +33,11 @@ constexpr int kb_per_stage() {
 }
 __host__ __device__ inline int kb_per_stage_of(int nhl) { return nhl == 2 ? 2 : 4; }
 
-// bf16_tile keeps each thread's chunk offsets within a tile's panel in 32
-// bits: at most (BM / 32) blocks of kbs * NHL * 64 chunks, BM <= 256.  So the
-// packed paths take K only while 8 * kbs * NHL * 64 < 2^31, i.e. K below
-// 2^25 (split BF16) or 2^26 (single BF16).
+// bf16_tile_pipe, the grouped launch's tile for packed operands, keeps each
+// thread's chunk offsets within a tile's panel in 32 bits (bf16_tile has 64):
+// at most (BM / 32) blocks of kbs * NHL * 64 chunks, BM <= 256.  So the packed
+// paths, dense and grouped alike, take K only while 8 * kbs * NHL * 64 < 2^31,
+// i.e. K below 2^25 (split BF16) or 2^26 (single BF16).
 inline bool bf16_k_supported(int64_t k, int nhl) {
   const int64_t stage = 16 * kb_per_stage_of(nhl);
   const int64_t kbs = (k + stage - 1) / stage * stage / 16;
@@ -314,9 +315,10 @@ __device__ __forceinline__ void zero_acc(floatx16 (&acc)[FM][FN]) {
 // so its address is kept in scalar registers.  The order of the MFMAs of one
 // accumulator is k block by k block, lo*hi, hi*lo, hi*hi within one.
 // Measured on MI355X, kernel alone, against one stage in flight and fragments
-// read when needed: N = 8192 split BF16 2.48 -> 2.12 ms (1331 -> 1555
-// TFLOP/s), single BF16 0.947 -> 0.796 ms; 1024 x 1024 x 4096 split BF16 on
-// 64x64 tiles 75.7 -> 31.6 us.
+// read when needed: N = 8192 with beta = 0 split BF16 2.44 -> 2.11 ms (1350 ->
+// 1565 TFLOP/s), single BF16 0.94 -> 0.81 ms (2.46 -> 2.15 and 1.01 -> 0.87 ms
+// where the epilogue also reads C); 1024 x 1024 x 4096 split BF16 on 64x64
+// tiles 75.7 -> 31.6 us.
 template <int BM, int BN, int WM, int WN, int NHL, int MOST = 4>
 __device__ __forceinline__ void bf16_tile(const BfTileArgs& t, int tm, int tn, int s0, int s1, const Epilogue& ep,
     int er, int ec, u32x4* lds) {

@@ -285,7 +285,7 @@ class Handle:
         _check(self.lib.mfx_force_config(self.h, prec_id(prec), config), "mfx_force_config")
 
     def force_splits(self, splits):
-        """FP32 split-K override: -1 automatic, 1 never, >= 2 that many k slices."""
+        """Split-K override, every precision: -1 automatic, 1 never, >= 2 that many k slices."""
         _check(self.lib.mfx_force_splits(self.h, splits), "mfx_force_splits")
 
     def force_grouped_policy(self, policy):
